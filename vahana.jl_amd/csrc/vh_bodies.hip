@@ -1642,6 +1642,140 @@ __global__ __launch_bounds__(256) void k_diffuse_stencil(StencilSpec sp, const u
     w[f] = v;
 }
 
+// The same step for a type of one-byte records (a lone Bool) that is the
+// raster and nothing else, as add_raster! makes it. A raster row is the cells
+// of one line along dimension 0 (consecutive bytes), worked on in groups of 8
+// cells, each from one 8-byte window per stencil offset. Only the first and
+// the last two groups of a row meet its ends. The others are computed by
+// waves of 64 groups of ROW_R rows: lane q works out the row of offset k + q (an
+// offset outside the raster becomes the cells themselves, which changes
+// nothing) and the wave takes it from there into a scalar address. The end
+// groups of all rows go to lanes of their own waves (the last blocks in y):
+// there a window is clamped into the row and shifted back, which leaves 0 for
+// cells outside, and a periodic row ors in the wrapped end. Bound: 20 MB of
+// cells read and written at 3162^2 are 4 us at the copy rate; instruction
+// issue comes first. 3162^2 cells, Moore neighbourhood, nearly all inactive:
+// k_diffuse_stencil 266 us (divisions and byte loads per cell); this with the
+// rows in scalar instructions 24 us, with the rows by lanes but the end groups
+// within the other waves 18 us, apart 16 us, two rows a wave 15 us (four: the
+// same).
+constexpr uint32_t ROW_U = 8;   // offsets at a time
+constexpr uint32_t ROW_R = 2;   // rows of a wave
+struct RowSpec {
+    int32_t dims[4];
+    uint32_t periodic, nst;                            // nst: a multiple of ROW_U (padded with zero offsets)
+    int32_t reach;                                     // largest |offset| along dimension 0
+    uint32_t off[VH_STENCIL_MAX];                      // four signed bytes in a word
+};
+// 8 bytes at any address: three words from the word they start in and a byte
+// shift. Reads up to 3 bytes past them.
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3), aligned(4)));
+__device__ __forceinline__ uint64_t ld8(const uint8_t* p) {
+    const uint32_t m = (uint32_t)(uintptr_t)p & 3u;
+    const u32x3 t = *(const u32x3*)(p - m);
+    return (uint64_t)__builtin_amdgcn_alignbyte(t.y, t.x, m) | (uint64_t)__builtin_amdgcn_alignbyte(t.z, t.y, m) << 32;
+}
+__device__ __forceinline__ uint64_t nonzero_bytes(uint64_t v) {   // each to 1
+    return ((((v & 0x7F7F7F7F7F7F7F7Full) + 0x7F7F7F7F7F7F7F7Full) | v) >> 7) & 0x0101010101010101ull;
+}
+// the row at offset word `off` from the one at coordinates c (its first cell)
+// and the offset along dimension 0; outside the raster the row itself and 0
+__device__ __forceinline__ void stencil_row(const RowSpec& sp, const int32_t* c, uint32_t row, uint32_t off,
+                                            int32_t& first, int32_t& dx) {
+    uint32_t lin = 0, stride = 1;
+    bool in = true;
+    for (uint32_t d = 1; d < 4; d++) {
+        const int32_t dim = sp.dims[d];
+        const int32_t o = c[d] - (int32_t)(int8_t)(off >> (8 * d));   // |offset| <= extent
+        const int32_t ow = o < 0 ? o + dim : o >= dim ? o - dim : o;
+        in = in && (sp.periodic || ow == o);
+        lin += (uint32_t)ow * stride;
+        stride *= (uint32_t)dim;
+    }
+    dx = in ? (int32_t)(int8_t)off : 0;
+    first = (int32_t)((in ? lin : row) * (uint32_t)sp.dims[0]);   // (< 2^31 cells)
+}
+__device__ __forceinline__ void row_coords(const RowSpec& sp, uint32_t row, int32_t* c) {
+    for (uint32_t d = 1; d < 4; d++) {   // (unused dimensions have extent 1)
+        const uint32_t dim = (uint32_t)sp.dims[d];
+        c[d] = (int32_t)(dim == 1u ? 0u : row % dim);
+        row = dim == 1u ? row : row / dim;
+    }
+}
+__global__ __launch_bounds__(256) void k_diffuse_rows(RowSpec sp, const uint8_t* __restrict__ rs,
+                                                      uint8_t* __restrict__ ws, uint32_t nrows, uint32_t yblocks) {
+    const int32_t nx = sp.dims[0], groups = (nx + 7) / 8;
+    if (blockIdx.y < yblocks) {   // groups 1 .. groups - 3
+        const int32_t lane = (int32_t)(threadIdx.x & 63u);
+        const uint32_t row = (blockIdx.y * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * ROW_R;
+        if (row >= nrows) return;   // uniform
+        const int32_t g = 1 + (int32_t)(blockIdx.x * 64u) + lane;
+        if (g - lane > groups - 3) return;                  // uniform
+        const int32_t x = 8 * (g <= groups - 3 ? g : 1);    // (every lane works out offsets)
+        uint32_t rw[ROW_R];
+        int32_t c[ROW_R][4];
+        uint64_t v[ROW_R];
+#pragma unroll
+        for (uint32_t j = 0; j < ROW_R; j++) {
+            rw[j] = row + j < nrows ? row + j : row;
+            row_coords(sp, rw[j], c[j]);
+            v[j] = ld8(rs + (uint64_t)rw[j] * (uint32_t)nx + x);
+        }
+        for (uint32_t k = 0; k < sp.nst; k += ROW_U) {
+            uint32_t off = sp.off[k];   // lane q: offset k + q, from scalar loads (the launch
+#pragma unroll                          // arguments are slow to reach by vector loads)
+            for (uint32_t q = 1; q < ROW_U; q++) off = lane == (int32_t)q ? sp.off[k + q] : off;
+            uint64_t u[ROW_R][ROW_U];
+#pragma unroll
+            for (uint32_t j = 0; j < ROW_R; j++) {
+                int32_t first, dx;
+                stencil_row(sp, c[j], rw[j], off, first, dx);
+                const int32_t from = first - dx;
+#pragma unroll
+                for (uint32_t q = 0; q < ROW_U; q++)
+                    u[j][q] = ld8(rs + (int64_t)__builtin_amdgcn_readlane(from, (int)q) + x);
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < ROW_R; j++)
+#pragma unroll
+                for (uint32_t q = 0; q < ROW_U; q++) v[j] |= u[j][q];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < ROW_R; j++) {
+            const uint64_t w = nonzero_bytes(v[j]);
+            if (g <= groups - 3 && row + j < nrows) __builtin_memcpy(ws + (uint64_t)(row + j) * (uint32_t)nx + x, &w, 8);
+        }
+        return;
+    }
+    int32_t c[4];
+    // the end groups: 0, groups - 2 and groups - 1 of every row
+    const uint32_t t = ((blockIdx.y - yblocks) * gridDim.x + blockIdx.x) * 256u + threadIdx.x;
+    const uint32_t row = t / 3u, which = t % 3u;
+    if (row >= nrows) return;
+    const int32_t x = which == 0 ? 0 : 8 * (groups - 3 + (int32_t)which);   // (groups >= 2; twice the same for 2)
+    row_coords(sp, row, c);
+    const uint8_t* r0 = rs + (uint64_t)row * (uint32_t)nx;
+    const int32_t xc = x + 8 > nx ? nx - 8 : x;   // clamped; the shift drops the cells before x
+    uint64_t v = ld8(r0 + xc) >> (8 * (x - xc));
+    for (uint32_t k = 0; k < sp.nst; k++) {
+        int32_t first, dx;
+        stencil_row(sp, c, row, sp.off[k], first, dx);
+        const uint8_t* r = rs + first;
+        const int32_t a = x - dx, past = a + 8 - nx;   // cells a .. a + 7; a >= -7, past <= 14
+        // the cells in the row, then (periodic) the wrapped ones
+        uint64_t u = ld8(r + (a < 0 ? 0 : past > 0 ? nx - 8 : a));
+        u = a < 0 ? u << (-8 * a) : past >= 8 ? 0ull : past > 0 ? u >> (8 * past) : u;
+        if (sp.periodic && (a < 0 || past > 0)) {
+            const uint64_t w = ld8(r + (a < 0 ? nx - 8 : past > 8 ? past - 8 : 0));
+            u |= a < 0 ? w >> (8 * (8 + a)) : past < 8 ? w << (8 * (8 - past)) : w;
+        }
+        v |= u;
+    }
+    v = nonzero_bytes(v);
+    uint8_t* w = ws + (uint64_t)row * (uint32_t)nx + x;
+    for (int32_t q = 0; q < 8 && x + q < nx; q++) w[q] = (uint8_t)(v >> (8 * q));
+}
+
 }  // namespace
 
 // ====================================================================== launchers
@@ -2157,6 +2291,36 @@ int launch_diffuse_stencil(Sim& s, int t, int et, uint32_t field) {
     uint64_t ncells = 1;
     for (uint32_t d = 0; d < sp.ndims; d++) ncells *= (uint64_t)sp.dims[d];
     if (!A.nslots) return VH_OK;
+    // rows of 8-cell groups: one-byte records, every slot a cell, rows of at
+    // least 16 cells (every 8-byte load stays inside its row), offsets of at
+    // most 7 cells along dimension 0 (one wrap, one partial group) and of at
+    // most the extent along the others (one wrap), and a grid within its
+    // limits; the rest takes the kernel that works cell by cell
+    const uint64_t nx = (uint64_t)sp.dims[0], nrows = ncells / nx;
+    bool rows = A.bytes == 1 && field == 0 && sp.first_nr == 1 && ncells == A.nslots && ncells <= 0x7FFFFFFFull &&
+                nx >= 16 && nrows <= 128000;
+    RowSpec rsp;
+    rsp.periodic = sp.periodic;
+    rsp.reach = 0;
+    for (uint32_t d = 0; d < 4; d++) rsp.dims[d] = d < sp.ndims ? (int32_t)sp.dims[d] : 1;
+    memset(rsp.off, 0, sizeof rsp.off);
+    for (uint32_t k = 0; k < sp.nst && rows; k++) {
+        const int dx = std::abs((int)sp.off[k][0]);
+        rows = dx <= 7;
+        for (uint32_t d = 1; d < 4; d++) rows = rows && std::abs((int)sp.off[k][d]) <= rsp.dims[d];
+        memcpy(&rsp.off[k], sp.off[k], 4);
+        rsp.reach = std::max(rsp.reach, dx);
+    }
+    rsp.nst = (sp.nst + ROW_U - 1) / ROW_U * ROW_U;
+    if (rows) {
+        // the blocks of 64 groups by 4 rows, then those of the end groups
+        const unsigned gx = grid_for((nx + 7) / 8, 64), gy = grid_for(nrows, 4 * ROW_R);
+        const unsigned ey = grid_for(3 * nrows, 256 * gx);
+        hipLaunchKernelGGL(k_diffuse_rows, dim3(gx, gy + ey), dim3(256), 0, s.stream, rsp,
+                           (const uint8_t*)A.rstate(), (uint8_t*)A.wstate(), (uint32_t)nrows, gy);
+        HIPCHECK(hipGetLastError());
+        return VH_OK;
+    }
     hipLaunchKernelGGL(k_diffuse_stencil, dim3(grid_for(A.nslots, 256)), dim3(256), 0, s.stream, sp,
                        (const uint8_t*)A.rstate(), (uint8_t*)A.wstate(), A.nslots, ncells, A.bytes, field);
     HIPCHECK(hipGetLastError());
