@@ -47,3 +47,68 @@ def test_diffuse_rows(vh, ora, gpu_ready, dims, dist, metric, periodic):
         got.append(out)
     for k, (a, b) in enumerate(zip(*got)):
         assert np.array_equal(a, b), k
+
+
+def _ragged_edges(n, seed):
+    """In-degrees 0, 1, ..., 9, 0, 1, ... (every remainder of the bodies'
+    groups of four), uniform sources, edges in no order."""
+    rng = np.random.default_rng(seed)
+    to = np.repeat(np.arange(1, n + 1), np.arange(n) % 10)
+    to = rng.permutation(to).astype(np.uint64)
+    tid = np.uint64(1) << np.uint64(56)
+    return tid | rng.integers(1, n + 1, len(to)).astype(np.uint64), tid | to
+
+
+@pytest.mark.parametrize("n", [1, 63, 1025])
+@pytest.mark.parametrize("hints", [(), ("Immortal",)], ids=["mortal", "immortal"])
+def test_sum_neighbors_ragged(vh, ora, gpu_ready, hints, n):
+    """Int64 sums that wrap, over rows of 0 to 9 in-edges; with mortal agents
+    a third dies first (their edges go)."""
+    fr, to = _ragged_edges(n, n)
+    got = []
+    for V in (vh, ora):
+        A, E = V.struct("A", [("foo", "<i8")]), V.struct("E")
+        model = (V.ModelTypes() | V.register_agenttype_(A, *hints) | V.register_edgetype_(E, "Stateless", target=A)
+                 | V.create_model("sum"))
+        sim = V.create_simulation(model)
+        st = np.zeros(n, dtype=A.dtype)
+        st["foo"] = np.arange(n) * 0x1234567812345 + (1 << 62)
+        sim._add_agents_array(A, st)
+        if len(to):
+            sim._add_edges_array(E, fr, to)
+        V.finish_init_(sim)
+        if not hints:
+            V.apply_(sim, V.transitions.die_if("odd"), A, [A], A)
+        for _ in range(2):
+            V.apply_(sim, V.transitions.sum_neighbors(E), A, [A, E], A)
+        raw, died = _states(sim, A)
+        got.append((raw[~died], died))
+    assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][0], got[1][0])
+
+
+@pytest.mark.parametrize("n", [2, 64, 1025])
+@pytest.mark.parametrize("fields", [[("foo", "<i8")], []], ids=["state", "stateless"])
+def test_added_edges_ragged(vh, ora, gpu_ready, fields, n):
+    """neighbor_foo_edges adds 0 to 18 edges per agent: targets, sources in
+    insertion order and states as the checker has them."""
+    fr, to = _ragged_edges(n, n + 7)
+    got = []
+    for V in (vh, ora):
+        A, E, F = V.struct("A", [("foo", "<i8")]), V.struct("E"), V.struct("F", fields)
+        model = (V.ModelTypes() | V.register_agenttype_(A, "Immortal") | V.register_edgetype_(E, "Stateless", target=A)
+                 | V.register_edgetype_(F, *([] if fields else ["Stateless"]), target=A) | V.create_model("add"))
+        sim = V.create_simulation(model)
+        st = np.zeros(n, dtype=A.dtype)
+        st["foo"] = np.arange(n)
+        sim._add_agents_array(A, st)
+        sim._add_edges_array(E, fr, to)
+        V.finish_init_(sim)
+        out = []
+        for _ in range(2):
+            V.apply_(sim, V.transitions.neighbor_foo_edges(E, F, -1), A, [A, E], F)
+            t, f, s = sim._read_edges(F)
+            out += [t.copy(), f.copy(), np.ascontiguousarray(s).view(np.uint8) if fields else np.zeros(0)]
+        got.append(out)
+    assert len(got[0][0]) == 2 * len(to)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)

@@ -36,8 +36,13 @@ struct Body<VH_TR_SUM_NEIGHBORS> {
                 vh_flag(c, VH_DERR_HINT);
                 return true;
             }
-            for (uint32_t k = b; k < e; k++) {
-                const uint8_t* ns = d_state(c, vh_src_id(E, k));
+            const Neighbors nb(c, et);
+            const uint8_t* n[4];
+            uint32_t k = b;
+            for (; k + 4 <= e && nb.four(k, n); k += 4)
+                sum += ld_i64(n[0]) + ld_i64(n[1]) + ld_i64(n[2]) + ld_i64(n[3]);
+            for (; k < e; k++) {
+                const uint8_t* ns = nb.state(k);
                 if (!ns) return true;
                 sum += ld_i64(ns);
             }
@@ -107,10 +112,17 @@ struct Body<VH_TR_NEIGHBOR_FOO_EDGES> {
             const DEdge& E = c->e[et];
             uint8_t es[8];
             st_i64(es, foo);
-            for (uint32_t k = b; k < e; k++) {
-                uint64_t nid = vh_src_id(E, k);
-                em.edge(nid, id, es);
-                em.edge(id, nid, es);
+            const Sources src(E);
+            for (uint32_t k = b; k < e; k += 4) {
+                uint64_t nid[4];
+                src.four(k, e, nid);
+                uint64_t f[8], t[8];
+#pragma unroll
+                for (uint32_t q = 0; q < 4; q++) {
+                    f[2 * q] = t[2 * q + 1] = nid[q];
+                    t[2 * q] = f[2 * q + 1] = id;
+                }
+                em.edges(f, t, 2 * min(e - k, 4u), es);
             }
         }
         return true;
