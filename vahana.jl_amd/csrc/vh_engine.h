@@ -141,7 +141,12 @@ struct Sim {
     DCtx h_ctx;                    // last uploaded context
     DevBuf d_ctx;
     bool ctx_valid = false;
+    // contexts on their way to d_ctx: pinned (behind h_stats), CTX_SLOTS of
+    // them, the first ctx_used taken since the stream was last waited for
+    DCtx* h_ctx_ring = nullptr;
+    uint32_t ctx_used = 0;
     DevBuf d_err;                  // uint32 error word
+    bool err_written = true;       // a kernel that can set d_err was enqueued since it was last read as 0
     DevBuf d_stats;                // small readback area
     uint64_t* h_stats = nullptr;   // pinned mirror of d_stats
     Scratch scratch;
@@ -224,6 +229,7 @@ void fill_weights(float* w, uint64_t n, uint64_t wseed, hipStream_t st);
 // host graph helper (vh_graph.cpp)
 extern "C" int vh_bfs_order(uint64_t n, uint64_t m, const uint32_t* a, const uint32_t* b,
                             uint64_t* new_nr);
+constexpr uint32_t CTX_SLOTS = 8;
 // engine services the bodies use
 int readback(Sim& s, int n);                           // d_stats -> h_stats, synchronous
 int ensure_slots(Sim& s, int t, uint64_t slots);

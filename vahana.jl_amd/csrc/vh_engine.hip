@@ -152,6 +152,7 @@ extern "C" int vh_debug_set_device_error(vh_sim_t h, uint32_t flags) {
     HIPCHECK(hipMemcpy(&e, s.d_err.p, 4, hipMemcpyDeviceToHost));
     e |= flags;
     HIPCHECK(hipMemcpy(s.d_err.p, &e, 4, hipMemcpyHostToDevice));
+    s.err_written = true;
     return VH_OK;
 }
 
@@ -191,13 +192,15 @@ extern "C" int vh_sim_create(vh_model_t mh, vh_sim_t* out) {
         s.e[et].src64 = s.m->na != 1;
         s.e[et].src_type = 1;
     }
-    e = hipHostMalloc((void**)&s.h_stats, 64 * sizeof(uint64_t), hipHostMallocDefault);
+    // the mirror of d_stats, then the contexts' slots
+    e = hipHostMalloc((void**)&s.h_stats, 64 * sizeof(uint64_t) + CTX_SLOTS * sizeof(DCtx), hipHostMallocDefault);
     if (e != hipSuccess) {
         (void)hipEventDestroy(s.last);
         (void)hipStreamDestroy(s.stream);
         delete h;
         return hip_fail(e, "hipHostMalloc");
     }
+    s.h_ctx_ring = (DCtx*)(s.h_stats + 64);
     int r = s.d_stats.ensure(64 * sizeof(uint64_t), s.stream);
     if (!r) r = s.d_err.ensure(sizeof(uint32_t), s.stream);
     if (!r) r = s.d_ctx.ensure(sizeof(DCtx), s.stream);
@@ -630,11 +633,30 @@ static void compute_layout(Sim& s, const EdgeStore& E, RowLayout& L, uint64_t& r
     }
 }
 
-int vh::readback(Sim& s, int n) {
-    HIPCHECK(hipMemcpyAsync(s.h_stats, s.d_stats.p, n * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                            s.stream));
-    HIPCHECK(hipStreamSynchronize(s.stream));
+// n words between device memory and pinned host memory, either way. A kernel
+// in place of a copy command: one wave's loads and stores, where a copy of a
+// few bytes or of a context (6 KB) costs its own command and, from or to
+// pageable memory, a wait of its own.
+static __global__ __launch_bounds__(256) void k_words(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
+                                                      uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+}
+static int copy_words(void* dst, const void* src, size_t bytes, hipStream_t st) {
+    hipLaunchKernelGGL(k_words, dim3(1), dim3(bytes <= 256 ? 64 : 256), 0, st, (uint32_t*)dst, (const uint32_t*)src,
+                       (uint32_t)(bytes / 4));
+    HIPCHECK(hipGetLastError());
     return VH_OK;
+}
+// waits for the simulation's stream: every context on its way has arrived
+static int wait_stream(Sim& s) {
+    HIPCHECK(hipStreamSynchronize(s.stream));
+    s.ctx_used = 0;
+    return VH_OK;
+}
+
+int vh::readback(Sim& s, int n) {
+    RC(copy_words(s.h_stats, s.d_stats.p, n * sizeof(uint64_t), s.stream));
+    return wait_stream(s);
 }
 
 // Build the CSR of E from (optionally) its current entries followed by `nlog`
@@ -668,6 +690,7 @@ static int build_csr(Sim& s, EdgeStore& E, bool keep_base, const uint64_t* d_to,
     if (!keys || !vals || !kalt || !valt || (!ignorefrom && !from) || (bytes && !sts) || !flag)
         return set_error(VH_ERR_OOM, "scratch allocation failed");
     uint32_t* err = s.d_err.as<uint32_t>();
+    s.err_written = true;
     if (nbase)
         hipLaunchKernelGGL(k_base_expand, dim3(grid_for(E.rows, 256)), dim3(256), 0, st,
                            E.off.as<uint32_t>(), E.src.p, (uint32_t)E.src64, E.src_type,
@@ -1387,20 +1410,35 @@ static void fill_ctx(Sim& s, const vh_apply_desc* d, DCtx& c) {
 }
 
 static int upload_ctx(Sim& s, const DCtx& c) {
+    s.err_written = true;   // (the kernels that take a context can flag)
     if (s.ctx_valid && memcmp(&c, &s.h_ctx, sizeof c) == 0) return VH_OK;
-    s.h_ctx = c;
-    HIPCHECK(hipMemcpyAsync(s.d_ctx.p, &s.h_ctx, sizeof(DCtx), hipMemcpyHostToDevice, s.stream));
-    // the source is pageable host memory: make sure the copy has consumed it
-    // before h_ctx can change again
-    HIPCHECK(hipStreamSynchronize(s.stream));
+    // through a slot of pinned memory that no copy still reads: a wait only
+    // where CTX_SLOTS contexts were sent since the last one
+    if (s.ctx_used == CTX_SLOTS) RC(wait_stream(s));
+    // (a captured copy would read the slot as it is at each replay)
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIPCHECK(hipStreamIsCapturing(s.stream, &cap));
+    if (cap != hipStreamCaptureStatusNone)
+        return set_error(VH_ERR_DEVICE, "a transition that needs its context uploaded can not be captured");
+    DCtx* slot = s.h_ctx_ring + s.ctx_used;
+    s.ctx_valid = false;
+    *slot = s.h_ctx = c;
+    RC(copy_words(s.d_ctx.p, slot, sizeof(DCtx), s.stream));
+    s.ctx_used++;
     s.ctx_valid = true;
     return VH_OK;
 }
 
+// waits for the stream and reports the device error word; the word is read
+// only when a kernel that can set it ran since it was last read (the SIR,
+// opinion and contact kernels can not)
 static int check_errors(Sim& s) {
-    HIPCHECK(hipStreamSynchronize(s.stream));
-    uint32_t e = 0;
-    HIPCHECK(hipMemcpy(&e, s.d_err.p, 4, hipMemcpyDeviceToHost));
+    uint32_t* const word = (uint32_t*)(s.h_stats + 63);
+    const bool read = s.err_written;
+    if (read) RC(copy_words(word, s.d_err.p, 4, s.stream));
+    RC(wait_stream(s));
+    const uint32_t e = read ? *word : 0u;
+    s.err_written = false;
     if (!e) return VH_OK;
     fill_u32(s.d_err.as<uint32_t>(), 0, 1, s.stream);
     HIPCHECK(hipStreamSynchronize(s.stream));
