@@ -112,3 +112,61 @@ def test_added_edges_ragged(vh, ora, gpu_ready, fields, n):
     assert len(got[0][0]) == 2 * len(to)
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+# one record, partial blocks, one block per tail group and more, a second tail
+# level, and more block results than the tail takes (a level of its own first)
+@pytest.mark.parametrize("n", [1, 2047, 2049, 9 * 2048 + 5, 2048 * 2048 + 1, 32768 * 2048 + 2049])
+def test_mapreduce_levels(vh, ora, gpu_ready, n):
+    """Field and computed maps: every level's order is the checker's tree."""
+    small = n < 1 << 22
+    rng = np.random.default_rng(n)
+    fields = [("x", "<f8"), ("g", "u1")] if small else [("g", "u1")]
+    st = None
+    got = []
+    for V in (vh, ora):
+        A = V.struct("A", fields)
+        sim = V.create_simulation(V.ModelTypes() | V.register_agenttype_(A, "Immortal") | V.create_model("levels"))
+        if st is None:
+            st = np.zeros(n, dtype=A.dtype)
+            st["g"] = rng.integers(0, 5, n)
+            if small:
+                st["x"] = rng.normal(0, 1, n)
+        sim._add_agents_array(A, st)
+        V.finish_init_(sim)
+        sim.order = 1
+        f = V.expr.field
+        out = [V.mapreduce(sim, "g", "+", A), V.mapreduce(sim, V.Field("g", 3), "+", A), V.mapreduce(sim, "g", "max", A),
+               V.mapreduce(sim, f("g") * 2.5 - 1, "+", A)]
+        if small:
+            out += [V.mapreduce(sim, "x", op, A) for op in ("+", "max", "min")]
+            out += [V.mapreduce(sim, f("x") * f("g"), "+", A)]
+        got.append(out)
+    assert [repr(v) for v in got[0]] == [repr(v) for v in got[1]]
+
+
+@pytest.mark.parametrize("depth", [1, 3, 4, 5])
+def test_expr_depth(vh, ora, gpu_ready, depth):
+    """Programs of each stack depth around the one that fits the registers
+    (4), the last operands on top: x op (x op (... select ...))."""
+    n = 5000
+    rng = np.random.default_rng(depth)
+    got = []
+    for V in (vh, ora):
+        A = V.struct("A", [("x", "<f8"), ("k", "<i4"), ("b", "?")])
+        sim = V.create_simulation(V.ModelTypes() | V.register_agenttype_(A) | V.create_model("depth"))
+        st = np.zeros(n, dtype=A.dtype)
+        r = np.random.default_rng(depth)
+        st["x"], st["k"], st["b"] = r.normal(0, 1, n), r.integers(-9, 9, n), r.random(n) < 0.5
+        sim._add_agents_array(A, st)
+        V.finish_init_(sim)
+        sim.order = 1
+        f = V.expr.field
+        out = []
+        for leaf in (f("k"), f("x"), f("b")):
+            e = V.expr.where(f("b"), leaf, f("k")) if depth >= 3 else leaf
+            for _ in range(depth - 3 if depth >= 3 else depth - 1):
+                e = f("k") - e
+            out += [V.mapreduce(sim, e, op, A) for op in ("+", "max")] + [V.mapreduce(sim, e > 0, "+", A)]
+        got.append(out)
+    assert [repr(v) for v in got[0]] == [repr(v) for v in got[1]]
