@@ -170,3 +170,25 @@ def test_expr_depth(vh, ora, gpu_ready, depth):
             out += [V.mapreduce(sim, e, op, A) for op in ("+", "max")] + [V.mapreduce(sim, e > 0, "+", A)]
         got.append(out)
     assert [repr(v) for v in got[0]] == [repr(v) for v in got[1]]
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("case", ["light", "heavy", "sparse"])
+def test_opinion_one_pass_blocks(vh, ora, gpu_ready, case, f32):
+    """Blocks of 256 agents around one and two tiles of slots: without heavy
+    agents (rows of exactly 64 in-edges among them), with one (65), with long
+    stretches of isolated agents; the last block partial."""
+    n = 256 * 3 + 7
+    deg = {"light": lambda i: np.where(i < 256, 12, np.where(i < 512, 13 - i % 3, 64 * (i % 5 == 0))),
+           "heavy": lambda i: np.where(i == 300, 65, np.where(i == n - 1, 200, i % 9)),
+           "sparse": lambda i: np.where(i % 251 == 0, 3, 0)}[case](np.arange(n))
+    rng = np.random.default_rng(n)
+    to = rng.permutation(np.repeat(np.arange(1, n + 1), deg)).astype(np.uint32)
+    fr = rng.integers(1, n + 1, len(to)).astype(np.uint32)
+    w = (rng.random(len(to)) * 0.9 + 0.05).astype(np.float32)
+    g = vh.models.build_opinion(vh, n, seed=2, f32=f32, edges=(fr, to, w))
+    c = vh.models.build_opinion(ora, n, seed=2, f32=f32, edges=(fr, to, w))
+    for k in range(3):
+        vh.models.step_opinion(vh, g)
+        vh.models.step_opinion(ora, c)
+        assert np.array_equal(_states(g.sim, g.T)[0], _states(c.sim, c.T)[0]), k

@@ -485,8 +485,43 @@ __device__ __forceinline__ uint32_t op_light_scan(uint32_t ld, uint32_t* s_wsum,
 // block are processed in tiles of OP_TILE slots: all threads load sources and
 // weights coalesced and gather OP_U neighbour states each, staging state and
 // weight by slot in LDS; then every thread adds its own agent's slots.
-constexpr int OP_TILE = 2048;
-constexpr int OP_U = 8;   // gathers in flight per thread
+//
+// The rows of a block without heavy agents are one range of the CSR: slot q
+// is in-edge b0 + q, and an agent's slots start at its own offset. Only a
+// block with a heavy agent (its rows are skipped) has to number its slots by
+// a scan and look up each slot's agent in LDS. us per step with the lookup in
+// every block, without it, and tiles of 3072 slots (the mean block of 10 to 12
+// in-edges an agent in one tile) in place of 2048: 1501 Float32 agents 8.9,
+// 5.5, 4.5 (a chain of latencies); 2 10^5 Float64 agents 23.3, 19.4, 19.3; 24
+// simulations of 5.8 10^6 agents in all 462, 408, 405, where the neighbours'
+// lines from beyond the L2 bound it (about 9 TB/s).
+constexpr int OP_TILE = 3072;
+constexpr int OP_U = OP_TILE / 256;   // gathers in flight per thread
+
+template <class T>
+struct OpLDS {
+    T x[OP_TILE];
+    float w[OP_TILE];
+    uint8_t own[OP_TILE];   // blocks with heavy agents: agent of each slot,
+    uint32_t b[256], p[256], wsum[4];   // its first in-edge, its first slot
+};
+
+// the slots [lo, hi) of an agent, staged from t0 on, added in order
+template <class T>
+__device__ __forceinline__ void op_sum_slots(const OpLDS<T>& sm, uint32_t lo, uint32_t hi, uint32_t t0, T xi, T eps,
+                                             T& num, T& den) {
+    uint32_t p = lo;
+    for (; p + 4 <= hi; p += 4) {   // (four slots' reads ahead of their sums)
+        const uint32_t q = p - t0;
+        const T x0 = sm.x[q], x1 = sm.x[q + 1], x2 = sm.x[q + 2], x3 = sm.x[q + 3];
+        const float w0 = sm.w[q], w1 = sm.w[q + 1], w2 = sm.w[q + 2], w3 = sm.w[q + 3];
+        op_accum(x0, w0, xi, eps, num, den);
+        op_accum(x1, w1, xi, eps, num, den);
+        op_accum(x2, w2, xi, eps, num, den);
+        op_accum(x3, w3, xi, eps, num, den);
+    }
+    for (; p < hi; p++) op_accum(sm.x[p - t0], sm.w[p - t0], xi, eps, num, den);
+}
 
 template <class T>
 __device__ __forceinline__ void opinion_block(const uint32_t* __restrict__ off,
@@ -494,66 +529,86 @@ __device__ __forceinline__ void opinion_block(const uint32_t* __restrict__ off,
                                               const T* __restrict__ x, const float* __restrict__ w,
                                               T* __restrict__ xo, uint64_t n, uint64_t nrows,
                                               uint64_t rowbase, T eps, uint32_t blk) {
-    __shared__ T s_x[OP_TILE];
-    __shared__ float s_w[OP_TILE];
-    __shared__ uint8_t s_own[OP_TILE];
-    __shared__ uint32_t s_b[256], s_p[256], s_wsum[4];
+    __shared__ OpLDS<T> sm;
     const int tid = threadIdx.x;
-    const uint64_t i = (uint64_t)blk * 256 + tid;
+    const uint64_t i0 = (uint64_t)blk * 256, i = i0 + tid;
+    const uint64_t r0 = i0 < nrows ? i0 : nrows, r1 = i0 + 256 < nrows ? i0 + 256 : nrows;
+    const uint32_t b0 = nrows ? off[rowbase + r0] : 0u, e0 = nrows ? off[rowbase + r1] : 0u;   // the block's in-edges
     uint32_t b = 0, d = 0;
     T xi = (T)0;
     if (i < n) {
-        xi = (*(x + i));
+        xi = x[i];
         if (i < nrows) {
-            b = (*(off + rowbase + i));
-            d = (*(off + rowbase + i + 1)) - b;
+            b = off[rowbase + i];
+            d = off[rowbase + i + 1] - b;
         }
     }
     const bool light = i < n && d <= 64u;
-    const uint32_t ld = light ? d : 0u;
-    uint32_t total;
-    const uint32_t P = op_light_scan(ld, s_wsum, total);
-    s_b[tid] = b;
-    s_p[tid] = P;
     T num = (T)0, den = (T)0;
-    for (uint32_t t0 = 0; t0 < total; t0 += OP_TILE) {
-        const uint32_t lo = P > t0 ? P : t0;
-        const uint32_t hi = (P + ld) < (t0 + OP_TILE) ? (P + ld) : (t0 + OP_TILE);
-        for (uint32_t p = lo; p < hi; p++) s_own[p - t0] = (uint8_t)tid;
-        __syncthreads();
-        const uint32_t cnt = (total - t0) < (uint32_t)OP_TILE ? (total - t0) : (uint32_t)OP_TILE;
-        // batches of OP_U slots per thread: all index loads, then all gathers
-        for (uint32_t q0 = 0; q0 < cnt; q0 += 256u * OP_U) {
+    if (!__syncthreads_or(d > 64u)) {
+        const uint32_t P = b - b0, total = e0 - b0;   // (P of an agent without a row: not used)
+        for (uint32_t t0 = 0; t0 < total; t0 += OP_TILE) {
+            uint32_t sj[OP_U];
+            float wk[OP_U];
+            T xj[OP_U];
+#pragma unroll
+            for (int u = 0; u < OP_U; u++) {
+                const uint32_t q = t0 + (uint32_t)u * 256u + tid;
+                const uint32_t k = b0 + (q < total ? q : 0u);   // (past the end: a valid dummy)
+                sj[u] = src[k];
+                wk[u] = w[k];
+            }
+#pragma unroll
+            for (int u = 0; u < OP_U; u++) xj[u] = x[sj[u] - 1];
+#pragma unroll
+            for (int u = 0; u < OP_U; u++) {
+                sm.x[u * 256 + tid] = xj[u];
+                sm.w[u * 256 + tid] = wk[u];
+            }
+            __syncthreads();
+            const uint32_t lo = P > t0 ? P : t0, hi = P + d < t0 + OP_TILE ? P + d : t0 + OP_TILE;
+            if (d) op_sum_slots(sm, lo, hi, t0, xi, eps, num, den);
+            if (t0 + OP_TILE < total) __syncthreads();
+        }
+    } else {
+        const uint32_t ld = light ? d : 0u;
+        uint32_t total;
+        const uint32_t P = op_light_scan(ld, sm.wsum, total);
+        sm.b[tid] = b;
+        sm.p[tid] = P;
+        for (uint32_t t0 = 0; t0 < total; t0 += OP_TILE) {
+            const uint32_t lo = P > t0 ? P : t0;
+            const uint32_t hi = (P + ld) < (t0 + OP_TILE) ? (P + ld) : (t0 + OP_TILE);
+            for (uint32_t p = lo; p < hi; p++) sm.own[p - t0] = (uint8_t)tid;
+            __syncthreads();
+            const uint32_t cnt = (total - t0) < (uint32_t)OP_TILE ? (total - t0) : (uint32_t)OP_TILE;
             uint32_t kk[OP_U], sj[OP_U];
             float wk[OP_U];
             T xj[OP_U];
 #pragma unroll
             for (int u = 0; u < OP_U; u++) {
-                const uint32_t q = q0 + (uint32_t)u * 256u + tid;
-                const uint32_t a = q < cnt ? s_own[q] : 0u;
-                kk[u] = q < cnt ? s_b[a] + (t0 + q - s_p[a]) : 0xFFFFFFFFu;
+                const uint32_t q = (uint32_t)u * 256u + tid;
+                const uint32_t a = q < cnt ? sm.own[q] : 0u;
+                kk[u] = q < cnt ? sm.b[a] + (t0 + q - sm.p[a]) : 0xFFFFFFFFu;
             }
 #pragma unroll
             for (int u = 0; u < OP_U; u++) {
-                sj[u] = kk[u] != 0xFFFFFFFFu ? (*(src + kk[u])) : 1u;
-                wk[u] = kk[u] != 0xFFFFFFFFu ? (*(w + kk[u])) : 0.0f;
+                sj[u] = kk[u] != 0xFFFFFFFFu ? src[kk[u]] : 1u;
+                wk[u] = kk[u] != 0xFFFFFFFFu ? w[kk[u]] : 0.0f;
             }
 #pragma unroll
             for (int u = 0; u < OP_U; u++) xj[u] = kk[u] != 0xFFFFFFFFu ? x[sj[u] - 1] : (T)0;
 #pragma unroll
             for (int u = 0; u < OP_U; u++) {
-                const uint32_t q = q0 + (uint32_t)u * 256u + tid;
-                if (q < cnt) {
-                    s_x[q] = xj[u];
-                    s_w[q] = wk[u];
-                }
+                sm.x[u * 256 + tid] = xj[u];
+                sm.w[u * 256 + tid] = wk[u];
             }
+            __syncthreads();
+            if (lo < hi) op_sum_slots(sm, lo, hi, t0, xi, eps, num, den);
+            __syncthreads();
         }
-        __syncthreads();
-        for (uint32_t p = lo; p < hi; p++) op_accum(s_x[p - t0], s_w[p - t0], xi, eps, num, den);
-        __syncthreads();
     }
-    if (light) *(xo + i) = den > (T)0 ? num / den : xi;
+    if (light) xo[i] = den > (T)0 ? num / den : xi;
 }
 
 template <class T>
@@ -603,16 +658,23 @@ __global__ __launch_bounds__(256) void k_opinion(const uint32_t* __restrict__ of
 // Many simulations' one-pass opinion steps in one launch: block b belongs to
 // the member with the largest blk0 <= b (its heavy-wave blocks first, then
 // its light blocks), every member with its own CSR, states and eps.
+// Blocks go to the 8 XCDs in turn, so XCD q takes the logical blocks
+// [q per, (q + 1) per): its L2 then holds the states of one or two members at
+// a time instead of a share of every member's (24 members of 10^4 to 10^6
+// Float64 agents: 494 -> 462 us a step, with the kernel as it was then).
 template <class T>
-__global__ __launch_bounds__(256) void k_opinion_multi(const OpMember* __restrict__ mem, uint32_t nm) {
+__global__ __launch_bounds__(256) void k_opinion_multi(const OpMember* __restrict__ mem, uint32_t nm,
+                                                       uint32_t nblocks) {
+    const uint32_t per = gridDim.x / 8u, blk = (blockIdx.x % 8u) * per + blockIdx.x / 8u;
+    if (blk >= nblocks) return;
     uint32_t lo = 0, hi = nm;
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) / 2;
-        if (mem[mid].blk0 <= blockIdx.x) lo = mid;
+        if (mem[mid].blk0 <= blk) lo = mid;
         else hi = mid;
     }
     const OpMember& m = mem[lo];
-    const uint32_t local = blockIdx.x - m.blk0;
+    const uint32_t local = blk - m.blk0;
     if (local >= m.nh) {
         opinion_block<T>(m.off, m.src, (const T*)m.x, m.w, (T*)m.xo, m.n, m.nrows, m.rowbase, (T)m.eps,
                          local - m.nh);
@@ -2277,20 +2339,21 @@ int opinion_defer_launch(OpinionDefer& c, hipStream_t st, DevBuf& dev, void** ho
             om.blk0 = (uint32_t)blocks;
             blocks += nb;
         }
-        if (blocks > 0x7FFFFFFFull) return set_error(VH_ERR_CAPACITY, "batched opinion launch too large");
+        if (blocks > 0x7FFFFFF0ull) return set_error(VH_ERR_CAPACITY, "batched opinion launch too large");
         const size_t bytes = v.size() * sizeof(OpMember);
         if (*host_off + bytes > *host_cap) return set_error(VH_ERR_CAPACITY, "batch staging");
         memcpy((uint8_t*)*host + *host_off, v.data(), bytes);
         HIPCHECK(hipMemcpyAsync((uint8_t*)dev.p + *host_off, (uint8_t*)*host + *host_off, bytes,
                                 hipMemcpyHostToDevice, st));
+        const uint32_t grid = (uint32_t)((blocks + 7) / 8 * 8);
         const OpMember* d = (const OpMember*)((uint8_t*)dev.p + *host_off);
         *host_off += (bytes + 255) & ~(size_t)255;
         if (k == 0)
-            hipLaunchKernelGGL(k_opinion_multi<double>, dim3((uint32_t)blocks), dim3(256), 0, st, d,
-                               (uint32_t)v.size());
+            hipLaunchKernelGGL(k_opinion_multi<double>, dim3(grid), dim3(256), 0, st, d, (uint32_t)v.size(),
+                               (uint32_t)blocks);
         else
-            hipLaunchKernelGGL(k_opinion_multi<float>, dim3((uint32_t)blocks), dim3(256), 0, st, d,
-                               (uint32_t)v.size());
+            hipLaunchKernelGGL(k_opinion_multi<float>, dim3(grid), dim3(256), 0, st, d, (uint32_t)v.size(),
+                               (uint32_t)blocks);
         HIPCHECK(hipGetLastError());
         v.clear();
     }
