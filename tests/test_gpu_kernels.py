@@ -192,3 +192,27 @@ def test_opinion_one_pass_blocks(vh, ora, gpu_ready, case, f32):
         vh.models.step_opinion(vh, g)
         vh.models.step_opinion(ora, c)
         assert np.array_equal(_states(g.sim, g.T)[0], _states(c.sim, c.T)[0]), k
+
+
+# contacts (a group of four and remainders, the 32 of a mask, past it),
+# redraws, deaths, agents: one word, a partial block, and sizes at which the
+# filter's groups hold 2 slots (its bits for single slots end at 1 310 720)
+# and blocks of 1024 begin (262 144)
+CONTACTS = [(1, 16, 0.05, 1), (3, 0, 0.1, 64), (4, 1, 0.5, 63), (5, 16, 0.3, 257), (31, 3, 0.1, 1000),
+            (32, 16, 0.02, 777), (33, 16, 0.02, 777), (7, 16, 0.02, 262_144), (3, 16, 0.04, 1_310_721)]
+
+
+@pytest.mark.parametrize("C,R,pd,n", CONTACTS)
+def test_contact_masks(vh, ora, gpu_ready, C, R, pd, n):
+    """States, died flags and contacts of three steps (two at the large
+    sizes), newborn slots among them."""
+    M = vh.models
+    g, c = (M.build_contact(V, n, seed=9, n_init=max(1, n // 5)) for V in (vh, ora))
+    for k in range(3 if n < 100_000 else 2):
+        for V, m in ((vh, g), (ora, c)):
+            M.step_contact(V, m, seed=9, beta=0.3, p_death=pd, n_contacts=C, max_redraw=R)
+        (a, da), (b, db) = _states(g.sim, g.T), _states(c.sim, c.T)
+        assert np.array_equal(da, db), k
+        assert np.array_equal(a[~da], b[~db]), k
+        for x, y in zip(g.sim._read_edges(g.E)[:2], c.sim._read_edges(c.E)[:2]):
+            assert np.array_equal(x, y), k

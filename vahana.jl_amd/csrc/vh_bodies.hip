@@ -1405,190 +1405,337 @@ __global__ void k_heavy_rows(const uint32_t* __restrict__ off, uint64_t rows, ui
 // state: health byte 0, susceptibility float at bytes 4-7.
 // The step runs on per-slot flag bitmaps (64 slots per word): `sp` marks
 // slots that are dead in the read state or die in this step, `dead` the
-// former, `inf` slots infected in the read state. A partner draw reads one
-// bit of `sp` and, for the ~4% of partners it marks, one of `dead`. At 10^7
-// slots each map is 1.25 MB, so the two hot ones stay in one XCD's 4 MB L2
-// while the draws and neighbour checks gather from them (the state vector
-// itself is 80 MB and is streamed past the cache).
+// former, `inf` slots infected in the read state. At 10^7 slots each is 1.25
+// MB, in reach of every XCD's L2, but the 2 10^8 partner draws of a step are
+// more than the L2s' random reads deliver (0.78 ms of them): so a draw first
+// asks a filter in LDS, one bit per group of 2^fshift slots, the smallest
+// groups that fit (8 slots at 10^7: 28% of the draws go on to `sp` with 4% of
+// the slots marked).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ bool cbit(const uint64_t* __restrict__ b, uint64_t i) {
     return (b[i >> 6] >> (i & 63)) & 1ull;
 }
 
-// one thread per slot, whole waves per word (grid = nwords * 64 threads)
+// one thread per slot, whole blocks of 4 words (the last block's words past
+// nwords are not stored)
 __global__ __launch_bounds__(256) void k_contact_flags(const uint64_t* __restrict__ rs,
                                                        const uint8_t* __restrict__ died, uint64_t n,
                                                        uint32_t t, vh_contact_params p, uint64_t step,
                                                        ContactBits B) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    uint64_t w = i >> 6;
-    if (w >= B.nwords) return;   // uniform per wave
-    bool in = i < n;
-    bool dead = !in || died[i] != 0;
-    bool inf = in && (__builtin_nontemporal_load(rs + i) & 0xFFu) == VH_I;
-    bool dn = !dead && vh_u01(vh_hash(p.seed, vh_make_id(t, i + 1), step, VH_KEY_DEATH)) < p.p_death;
-    uint64_t md = __ballot(dead), mi = __ballot(inf), mn = __ballot(dn);
-    if ((threadIdx.x & 63u) == 0) {
-        B.sp[w] = md | mn;
+    __shared__ uint32_t s_f[4];
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t w = i >> 6;
+    const uint32_t lane = threadIdx.x & 63u;
+    const bool in = i < n;
+    const bool dead = !in || died[i] != 0;
+    const uint32_t h = in ? (uint32_t)(__builtin_nontemporal_load(rs + i) & 0xFFu) : 0u;
+    const bool inf = in && h == VH_I;
+    const bool dn = !dead && vh_u01(vh_hash(p.seed, vh_make_id(t, i + 1), step, VH_KEY_DEATH)) < p.p_death;
+    const uint64_t md = __ballot(dead), mi = __ballot(inf), mn = __ballot(dn), m = md | mn;
+    const uint64_t ms = __ballot(h == VH_S) & ~m;
+    if (lane == 0 && w < B.nwords) {
+        B.sp[w] = m;
         B.dead[w] = md;
         B.inf[w] = mi;
-        B.dcnt[w] = (uint32_t)__popcll(mn);
+        B.sus[w] = ms;
+        B.cnt[w] = (uint32_t)__popcll(mn);
+    }
+    if (B.filt) {   // 256 >> fshift bits per block
+        const uint32_t g = B.fshift, nb = 64u >> g;
+        const uint64_t f = __ballot(lane < nb && ((m >> ((lane << g) & 63u)) & ((1ull << (1u << g)) - 1ull)));
+        uint8_t* out = B.filt + (uint64_t)blockIdx.x * (32u >> g);
+        if (g <= 2) {
+            if (lane == 0) {
+                uint8_t* o = out + (threadIdx.x >> 6) * (8u >> g);
+                if (g == 0) *(uint64_t*)o = f;
+                else if (g == 1) *(uint32_t*)o = (uint32_t)f;
+                else *(uint16_t*)o = (uint16_t)f;
+            }
+        } else {
+            if (lane == 0) s_f[threadIdx.x >> 6] = (uint32_t)f;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                const uint32_t v = s_f[0] | s_f[1] << nb | s_f[2] << 2 * nb | s_f[3] << 3 * nb;
+                if (g == 3) *(uint32_t*)out = v;
+                else if (g == 4) *(uint16_t*)out = (uint16_t)v;
+                else *out = (uint8_t)v;
+            }
+        }
     }
 }
 
-// Health update, death flag, partner draws. The kept partners of every
-// slot (accepted draws whose partner does not die in this step, in draw
-// order) go to a fixed-stride log, row i at log[i * n_contacts], written
-// through LDS as one contiguous block range. Dynamic LDS: 256 * n_contacts
-// words when `staged`.
-__global__ __launch_bounds__(256) void k_contact_main(
-    const uint32_t* __restrict__ off, const uint32_t* __restrict__ src, const uint64_t* __restrict__ rs,
-    uint64_t* __restrict__ ws, uint8_t* __restrict__ died_now, uint64_t n, uint64_t nrows,
-    uint64_t rowbase, uint32_t t, vh_contact_params p, uint64_t step, ContactBits B,
-    uint32_t* __restrict__ kept, uint32_t* __restrict__ log, uint32_t staged) {
-    extern __shared__ u32x4 lds_v[];   // 16-byte aligned
-    uint32_t* lds = (uint32_t*)lds_v;
-    const uint32_t C = p.n_contacts;
+// the partner of draw r of contact cc (0-based slot; n < 2^32)
+__device__ __forceinline__ uint32_t contact_draw(uint64_t pre, uint32_t n, const vh_contact_params& p, uint32_t cc,
+                                                 uint32_t r) {
+    const uint64_t hh = vh_hash_fin(pre, VH_KEY_PARTNER + (uint64_t)cc * p.max_redraw + r);
+    return __umulhi((uint32_t)(hh >> 32), n);
+}
+// contact cc of slot i: draws until a partner that lives in the read state
+// and is not i (at most max_redraw); false when there is none or it dies in
+// this step
+__device__ __forceinline__ bool contact_partner(uint64_t pre, uint32_t n, const vh_contact_params& p, uint64_t i,
+                                                uint32_t cc, const ContactBits& B, uint32_t& j) {
+    for (uint32_t r = 0; r < p.max_redraw; r++) {
+        j = contact_draw(pre, n, p, cc, r);
+        if (j == i) continue;
+        if (!cbit(B.sp, j)) return true;
+        if (!cbit(B.dead, j)) return false;   // dies in this step: not kept
+    }
+    return false;
+}
+// Infections: a susceptible slot gets infected when some in-edge (a contact of
+// the last step) has an infected source and a draw below beta * susceptibility.
+// "Some" has no order: the draw (ALU) first, the source's flag only for the
+// few draws below. A block lists the susceptible slots of INF_W words and its
+// threads take them off the list, so that all lanes draw: at the endemic state
+// 15% of the slots are susceptible, and with each slot on its own lane every
+// wave went through all draws for those (390 us of the 10^7-slot step; listed,
+// with the draws before the lookups, 68 us). The word of `sus` is replaced by
+// the slots that get infected.
+constexpr uint32_t INF_W = 32;
+__global__ __launch_bounds__(256) void k_contact_infect(const uint32_t* __restrict__ off,
+                                                        const uint32_t* __restrict__ src,
+                                                        const uint64_t* __restrict__ rs, uint64_t nrows,
+                                                        uint64_t rowbase, uint32_t t, vh_contact_params p,
+                                                        uint64_t step, ContactBits B) {
+    __shared__ uint32_t s_n, s_bits[2 * INF_W];
+    __shared__ uint16_t s_list[64 * INF_W];
     const uint32_t tid = threadIdx.x;
-    const uint64_t i0 = (uint64_t)blockIdx.x * 256;
-    const uint64_t i = i0 + tid;
-
-    bool live = i < n && !cbit(B.dead, i);
-    bool survive = false;
-    uint32_t nk = 0;
-    if (live) {
-        const uint64_t id = vh_make_id(t, i + 1);
-        const uint64_t pre = vh_hash_pre(p.seed, id, step);
-        const uint64_t s = __builtin_nontemporal_load(rs + i);
-        uint32_t h = (uint32_t)(s & 0xFFu);
-        if (h == VH_S) {
-            if (off && i < nrows) {
-                float susc = __uint_as_float((uint32_t)(s >> 32));
-                double pinf = p.beta * (double)susc;
-                const uint64_t pt = vh_u01_below(pinf);
-                uint32_t b = off[rowbase + i], e = off[rowbase + i + 1];
-                // "some in-edge k has an infected source and u_k < pinf" is
-                // order-free: test the draw first (ALU) and look up the
-                // source's flag only for the few draws below pinf
-                if (vh_any_infecting(pre, pt, b, e, [&](uint32_t k) { return cbit(B.inf, src[k] - 1); }))
-                    h = VH_I;
-            }
-        } else if (h == VH_I) {
-            if (vh_u01(vh_hash_fin(pre, VH_KEY_RECOVER)) < p.gamma) h = VH_R;
-        }
-        if (cbit(B.sp, i))   // live and marked: dies in this step
-            died_now[i] = 1;
-        else {
-            survive = true;
-            __builtin_nontemporal_store((s & ~(uint64_t)0xFFu) | h, ws + i);
-        }
+    const uint64_t w0 = (uint64_t)blockIdx.x * INF_W;
+    if (tid == 0) s_n = 0;
+    if (tid < 2 * INF_W) s_bits[tid] = 0;
+    __syncthreads();
+    for (uint32_t q = tid; q < 64 * INF_W; q += 256) {   // a wave: the slots of a word
+        const uint64_t w = w0 + (q >> 6);
+        const uint64_t m = w < B.nwords ? B.sus[w] : 0ull;
+        if (!m) continue;   // uniform per wave
+        uint32_t base = 0;
+        if ((q & 63u) == 0) base = atomicAdd(&s_n, (uint32_t)__popcll(m));
+        base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        const uint32_t l = q & 63u;
+        if ((m >> l) & 1ull) s_list[base + (uint32_t)__popcll(m & ((1ull << l) - 1ull))] = (uint16_t)q;
     }
-    if (survive) {
+    __syncthreads();
+    for (uint32_t k = tid; k < s_n; k += 256) {
+        const uint32_t q = s_list[k];
+        const uint64_t i = w0 * 64 + q;
+        if (i >= nrows) continue;
+        const uint32_t b = off[rowbase + i], e = off[rowbase + i + 1];
+        if (b == e) continue;
+        const double pinf = p.beta * (double)__uint_as_float((uint32_t)(rs[i] >> 32));
         const uint64_t pre = vh_hash_pre(p.seed, vh_make_id(t, i + 1), step);
-        uint32_t* row = staged ? lds + (uint64_t)tid * C : log + i * C;
-        uint64_t key = VH_KEY_PARTNER;
-        for (uint32_t cc = 0; cc < C; cc++, key += p.max_redraw) {
-            for (uint32_t r = 0; r < p.max_redraw; r++) {
-                uint64_t hh = vh_hash_fin(pre, key + r);
-                uint64_t j = 1 + (((hh >> 32) * n) >> 32);
-                if (j == i + 1) continue;
-                if (cbit(B.sp, j - 1)) {
-                    if (cbit(B.dead, j - 1)) continue;   // dead in the read state: redraw
-                    break;                               // dies in this step: not kept
+        if (vh_any_infecting(pre, vh_u01_below(pinf), b, e, [&](uint32_t x) { return cbit(B.inf, src[x] - 1); }))
+            atomicOr(&s_bits[q >> 5], 1u << (q & 31u));
+    }
+    __syncthreads();
+    if (tid < INF_W && w0 + tid < B.nwords)
+        B.sus[w0 + tid] = (uint64_t)s_bits[2 * tid] | (uint64_t)s_bits[2 * tid + 1] << 32;
+}
+// health update of live slot i; true when it survives the step
+__device__ __forceinline__ bool contact_health(const uint64_t* __restrict__ rs, uint64_t* __restrict__ ws,
+                                               const vh_contact_params& p, const ContactBits& B, uint64_t i,
+                                               uint64_t pre) {
+    const uint64_t s = __builtin_nontemporal_load(rs + i);
+    uint32_t h = (uint32_t)(s & 0xFFu);
+    if (cbit(B.sp, i)) return false;   // live and marked: dies in this step
+    if (h == VH_S) {
+        if (cbit(B.sus, i)) h = VH_I;
+    } else if (h == VH_I) {
+        if (vh_u01(vh_hash_fin(pre, VH_KEY_RECOVER)) < p.gamma) h = VH_R;
+    }
+    __builtin_nontemporal_store((s & ~(uint64_t)0xFFu) | h, ws + i);
+    return true;
+}
+
+// Health update, death flag, and which of up to 32 contacts of every slot are
+// kept: `masks` gets a bit per kept contact and a bit per kept contact that
+// was not its first draw, from which k_contact_edges draws the partners again
+// (8 bytes a slot in place of 4 per contact written and read back). Blocks
+// stay with the filter in LDS and take tiles of BS slots in turn. Four first
+// draws at a time: their hashes, filter bits, and the reads of `sp` that are
+// left are in flight together; what is not accepted there (4% of the draws)
+// is settled after the loop, so that a wave runs the redraws of its lanes
+// together. Bound: instruction issue, 50 vector instructions a draw with seven
+// quarter-rate products among them (0.3 ms for 2 10^8 draws). 10^7 slots, 20
+// contacts, 2% deaths: with infections in the same loop, each draw in the L2
+// and the partners to a log 1055 us, so 440 us (filter groups of 16 slots and
+// two blocks per CU 500; 2, 5, 8 or 10 draws at a time 465, 437, 476, 436).
+template <int BS, bool FILTER>
+__global__ __launch_bounds__(BS) void k_contact_main(const uint64_t* __restrict__ rs, uint64_t* __restrict__ ws,
+                                                     uint8_t* __restrict__ died_now, uint32_t n, uint32_t t,
+                                                     vh_contact_params p, uint64_t step, ContactBits B,
+                                                     uint32_t fwords, uint2* __restrict__ masks) {
+    extern __shared__ u32x4 lds_v[];   // the filter: fwords words, a multiple of 4
+    const uint32_t* F = (const uint32_t*)lds_v;
+    const uint32_t tid = threadIdx.x, C = p.n_contacts;
+    for (uint32_t q = tid; q < fwords / 4; q += BS) lds_v[q] = ((const u32x4*)B.filt)[q];
+    __syncthreads();
+    for (uint64_t i0 = (uint64_t)blockIdx.x * BS; i0 < n; i0 += (uint64_t)gridDim.x * BS) {
+        const uint64_t i = i0 + tid;
+        uint32_t km = 0, rm = 0;
+        if (i < n && !cbit(B.dead, i)) {
+            const uint64_t pre = vh_hash_pre(p.seed, vh_make_id(t, i + 1), step);
+            if (contact_health(rs, ws, p, B, i, pre) && p.max_redraw) {
+                uint32_t todo = 0;
+                for (uint32_t c0 = 0; c0 < C; c0 += 4) {
+                    uint32_t j[4];
+                    bool ask[4];
+                    uint32_t word[4];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) j[u] = contact_draw(pre, n, p, c0 + u, 0);
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) {
+                        const uint32_t g = j[u] >> B.fshift;
+                        ask[u] = !FILTER || ((F[g >> 5] >> (g & 31u)) & 1u);
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) {
+                        word[u] = 0;
+                        if (ask[u]) word[u] = ((const uint32_t*)B.sp)[j[u] >> 5];
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) {
+                        const bool take = j[u] != (uint32_t)i && !((word[u] >> (j[u] & 31u)) & 1u);
+                        km |= take ? 1u << (c0 + u) : 0u;
+                    }
                 }
-                row[nk++] = (uint32_t)j;
-                break;
+                const uint32_t all = C == 32 ? 0xFFFFFFFFu : (1u << C) - 1u;   // (the last group may pass C)
+                km &= all;
+                todo = all & ~km;
+                while (todo) {
+                    const uint32_t cc = (uint32_t)__builtin_ctz(todo);
+                    todo &= todo - 1u;
+                    uint32_t jj;
+                    if (contact_partner(pre, n, p, i, cc, B, jj)) {
+                        km |= 1u << cc;
+                        rm |= 1u << cc;
+                    }
+                }
             }
         }
-    }
-    if (i < n) kept[i] = nk;
-    if (staged) {
-        __syncthreads();
-        uint64_t rows_here = n - i0 < 256 ? n - i0 : 256;
-        uint64_t len = rows_here * C;
-        uint32_t* dst = log + i0 * C;   // 16-byte aligned: i0 is a multiple of 256
-        uint64_t len4 = len >> 2;
-        for (uint64_t q = tid; q < len4; q += 256)
-            __builtin_nontemporal_store(*(const u32x4*)(lds + 4 * q), (u32x4*)(dst + 4 * q));
-        for (uint64_t q = 4 * len4 + tid; q < len; q += 256) dst[q] = lds[q];
+        if (i < n) {
+            masks[i] = make_uint2(km, rm);
+            died_now[i] = cbit(B.sp, i) && !cbit(B.dead, i);
+        }
+        const uint32_t sum = wave_incl_scan((uint32_t)__popc(km));
+        if ((tid & 63u) == 63u && i >> 6 < B.nwords) B.cnt[B.nwords + (i >> 6)] = sum;
     }
 }
 
-// newborns of this step's deaths, in slot order of the dying callers: the
-// top of the reuse stack first, then fresh slots (src/AgentMethods.jl:37-89)
-__global__ void k_contact_births(uint64_t n, uint32_t t, vh_contact_params p, uint64_t step,
-                                 ContactBits B, const uint32_t* __restrict__ dpos,
-                                 const uint32_t* __restrict__ reuse, uint64_t nreuse, uint64_t nextid,
-                                 uint64_t* __restrict__ ws, uint8_t* __restrict__ died) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// The rebuilt contact CSR (row i = caller slot i, kept partners in draw
+// order) from the masks: cpos is the scan of B.cnt (its entry nwords: the
+// deaths, then contacts before each word of slots). A wave's rows are one
+// range of the CSR: the partners are drawn into LDS at their place and
+// written out as one range per block. Dynamic LDS: 256 * n_contacts words.
+// Bound: the 800 MB of a 2 10^8 contact CSR (0.16 ms) and the hashes
+// (0.22 ms); from the log it was 337 us, so 238 us.
+__global__ __launch_bounds__(256) void k_contact_edges(uint32_t n, uint32_t t, vh_contact_params p, uint64_t step,
+                                                       ContactBits B, const uint2* __restrict__ masks,
+                                                       const uint32_t* __restrict__ cpos, uint32_t* __restrict__ off,
+                                                       uint32_t* __restrict__ src) {
+    extern __shared__ u32x4 lds_v[];
+    uint32_t* lds = (uint32_t*)lds_v;
+    const uint32_t tid = threadIdx.x, C = p.n_contacts;
+    const uint64_t i0 = (uint64_t)blockIdx.x * 256, i = i0 + tid, w0 = i0 >> 6;
+    const uint64_t w1 = w0 + 4 < B.nwords ? w0 + 4 : B.nwords;
+    const uint32_t deaths = cpos[B.nwords];
+    const uint32_t base = cpos[B.nwords + w0] - deaths, end = cpos[B.nwords + w1] - deaths;
+    uint2 m = make_uint2(0u, 0u);
+    if (i < n) m = masks[i];
+    const uint32_t cnt = (uint32_t)__popc(m.x), incl = wave_incl_scan(cnt);
+    if (i < n) {
+        const uint32_t o = cpos[B.nwords + (i >> 6)] - deaths + incl - cnt;
+        off[i] = o;
+        if (i == n - 1) off[n] = o + cnt;
+        uint32_t* row = lds + (o - base);
+        const uint64_t pre = vh_hash_pre(p.seed, vh_make_id(t, i + 1), step);
+        const uint32_t first = m.x & ~m.y;
+        for (uint32_t cc = 0; cc < C; cc++)
+            if ((first >> cc) & 1u)
+                row[__popc(m.x & ((1u << cc) - 1u))] = contact_draw(pre, n, p, cc, 0) + 1u;
+        for (uint32_t re = m.y; re; re &= re - 1u) {
+            const uint32_t cc = (uint32_t)__builtin_ctz(re);
+            uint32_t j = 0;
+            (void)contact_partner(pre, n, p, i, cc, B, j);
+            row[__popc(m.x & ((1u << cc) - 1u))] = j + 1u;
+        }
+    }
+    __syncthreads();
+    for (uint32_t q = tid; q < end - base; q += 256) __builtin_nontemporal_store(lds[q], src + base + q);
+}
+
+// More than 32 contacts per slot: the kept partners of a slot go to a
+// fixed-stride log (row i at log[i * n_contacts]), their counts to `kept`.
+__global__ __launch_bounds__(256) void k_contact_main_log(const uint64_t* __restrict__ rs, uint64_t* __restrict__ ws,
+                                                          uint8_t* __restrict__ died_now, uint32_t n, uint32_t t,
+                                                          vh_contact_params p, uint64_t step, ContactBits B,
+                                                          uint32_t* __restrict__ kept, uint32_t* __restrict__ log) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    uint64_t word = B.sp[i >> 6] & ~B.dead[i >> 6];   // dying in this step
-    uint32_t lane = (uint32_t)(i & 63);
-    if (!((word >> lane) & 1ull)) return;
-    uint64_t g = dpos[i >> 6] + (uint64_t)__popcll(word & ((1ull << lane) - 1ull));
-    uint64_t slot = g < nreuse ? reuse[nreuse - 1 - g] : nextid + (g - nreuse);
-    float ns = 0.5f + 0.5f * vh_u01f(vh_hash(p.seed, vh_make_id(t, i + 1), step, VH_KEY_BIRTH));
-    ws[slot - 1] = (uint64_t)VH_S | ((uint64_t)__float_as_uint(ns) << 32);
-    died[slot - 1] = 0;
+    uint32_t nk = 0;
+    if (!cbit(B.dead, i)) {
+        const uint64_t pre = vh_hash_pre(p.seed, vh_make_id(t, i + 1), step);
+        if (contact_health(rs, ws, p, B, i, pre)) {
+            uint32_t* row = log + i * p.n_contacts;
+            for (uint32_t cc = 0; cc < p.n_contacts; cc++) {
+                uint32_t j;
+                if (contact_partner(pre, n, p, i, cc, B, j)) row[nk++] = j + 1u;
+            }
+        }
+    }
+    kept[i] = nk;
+    died_now[i] = cbit(B.sp, i) && !cbit(B.dead, i);
+}
+// the CSR from the log
+__global__ __launch_bounds__(256) void k_contact_edges_log(uint64_t n, uint32_t C, const uint32_t* __restrict__ kept,
+                                                           const uint32_t* __restrict__ log,
+                                                           const uint32_t* __restrict__ off,
+                                                           uint32_t* __restrict__ src) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t k = kept[i], o = off[i];
+    for (uint32_t r = 0; r < k; r++) src[o + r] = log[i * C + r];
+}
+
+// Newborns and deaths go by words, one thread each: 2% of the slots die, so
+// a thread per slot spent its time on waves that held one or none (35 and 19
+// us at 10^7 slots, by words 12 and 5 us).
+// Newborns of this step's deaths, in slot order of the dying callers: the top
+// of the reuse stack first, then fresh slots (src/AgentMethods.jl:37-89).
+__global__ void k_contact_births(uint32_t t, vh_contact_params p, uint64_t step, ContactBits B,
+                                 const uint32_t* __restrict__ dpos, const uint32_t* __restrict__ reuse,
+                                 uint64_t nreuse, uint64_t nextid, uint64_t* __restrict__ ws,
+                                 uint8_t* __restrict__ died) {
+    const uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= B.nwords) return;
+    uint64_t g = dpos[w];
+    for (uint64_t m = B.sp[w] & ~B.dead[w]; m; m &= m - 1ull, g++) {   // dying in this step
+        const uint64_t i = w * 64 + (uint32_t)__builtin_ctzll(m);
+        const uint64_t slot = g < nreuse ? reuse[nreuse - 1 - g] : nextid + (g - nreuse);
+        const float ns = 0.5f + 0.5f * vh_u01f(vh_hash(p.seed, vh_make_id(t, i + 1), step, VH_KEY_BIRTH));
+        ws[slot - 1] = (uint64_t)VH_S | ((uint64_t)__float_as_uint(ns) << 32);
+        died[slot - 1] = 0;
+    }
 }
 
 // this step's deaths onto the reuse stack in slot order (src/AgentMethods.jl:314-345)
-__global__ void k_contact_deaths(uint64_t n, ContactBits B, const uint32_t* __restrict__ dpos,
-                                 uint32_t* __restrict__ reuse, uint64_t base, uint8_t* __restrict__ died) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint64_t word = B.sp[i >> 6] & ~B.dead[i >> 6];   // dying in this step
-    uint32_t lane = (uint32_t)(i & 63);
-    if (!((word >> lane) & 1ull)) return;
-    uint64_t g = dpos[i >> 6] + (uint64_t)__popcll(word & ((1ull << lane) - 1ull));
-    reuse[base + g] = (uint32_t)(i + 1);
-    died[i] = 1;
+__global__ void k_contact_deaths(ContactBits B, const uint32_t* __restrict__ dpos, uint32_t* __restrict__ reuse,
+                                 uint64_t base, uint8_t* __restrict__ died) {
+    const uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= B.nwords) return;
+    uint64_t g = dpos[w];
+    for (uint64_t m = B.sp[w] & ~B.dead[w]; m; m &= m - 1ull, g++) {   // dying in this step
+        const uint64_t i = w * 64 + (uint32_t)__builtin_ctzll(m);
+        reuse[base + g] = (uint32_t)(i + 1);
+        died[i] = 1;
+    }
 }
 
 // rows past the last caller (fresh newborn slots) are empty
 __global__ void k_contact_extend(uint32_t* __restrict__ off, uint64_t from_row, uint64_t rows) {
     uint64_t r = from_row + 1 + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r <= rows) off[r] = off[from_row];
-}
-
-// The rebuilt contact CSR (row i = caller slot i, kept partners in draw
-// order): the block's log rows are read as one contiguous range, compacted
-// in LDS and written as the block's contiguous CSR range. Dynamic LDS:
-// 2 * 256 * n_contacts words when `staged`.
-__global__ __launch_bounds__(256) void k_contact_edges(uint64_t n, uint32_t C,
-                                                       const uint32_t* __restrict__ kept,
-                                                       const uint32_t* __restrict__ log,
-                                                       const uint32_t* __restrict__ off,
-                                                       uint32_t* __restrict__ src, uint32_t staged) {
-    extern __shared__ u32x4 lds_v[];   // 16-byte aligned
-    uint32_t* lds = (uint32_t*)lds_v;
-    const uint32_t tid = threadIdx.x;
-    const uint64_t i0 = (uint64_t)blockIdx.x * 256;
-    const uint64_t i = i0 + tid;
-    if (!staged) {   // uniform
-        if (i >= n) return;
-        uint32_t k = kept[i], o = off[i];
-        for (uint32_t r = 0; r < k; r++) src[o + r] = log[i * C + r];
-        return;
-    }
-    uint32_t* lin = lds;
-    uint32_t* lout = lds + 256 * C;
-    const uint64_t rows_here = n - i0 < 256 ? n - i0 : 256;
-    const uint64_t len = rows_here * C;
-    const uint32_t* lsrc = log + i0 * C;   // 16-byte aligned: i0 is a multiple of 256
-    const uint64_t len4 = len >> 2;
-    for (uint64_t q = tid; q < len4; q += 256)
-        *(u32x4*)(lin + 4 * q) = __builtin_nontemporal_load((const u32x4*)(lsrc + 4 * q));
-    for (uint64_t q = 4 * len4 + tid; q < len; q += 256) lin[q] = lsrc[q];
-    const uint32_t base = off[i0], end = off[i0 + rows_here];
-    __syncthreads();
-    if (i < n) {
-        uint32_t k = kept[i], o = off[i] - base;
-        for (uint32_t r = 0; r < k; r++) lout[o + r] = lin[tid * C + r];
-    }
-    __syncthreads();
-    for (uint32_t q = tid; q < end - base; q += 256) __builtin_nontemporal_store(lout[q], src + base + q);
 }
 
 // ----------------------------------------------------------------- raster stencils
@@ -2440,39 +2587,72 @@ int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t st
     *ndeaths = 0;
     if (n >= 0xFFFFFFFFull) return set_error(VH_ERR_CAPACITY, "contact: too many slots");
     if ((uint64_t)n * C >= 0xFFFFFFFFull) return set_error(VH_ERR_CAPACITY, "contact: too many contacts");
-    // LDS staging of 256 rows of C contacts (main: one buffer, CSR copy: two)
-    const uint32_t staged = C >= 1 && C <= 32;
-    const uint64_t nw = (n + 63) / 64;
+    const uint64_t nw = (n + 63) / 64, nblk = (n + 255) / 256;
+    // up to 32 contacts: a mask per slot and the partners drawn again; more:
+    // a log. The filter takes the smallest groups whose bits fit a CU's LDS;
+    // groups of more than 32 slots would nearly all be marked
+    const bool masked = C <= 32;
     ContactBits B;
     B.nwords = nw;
+    B.fshift = 0;
+    B.filt = nullptr;
+    while ((nblk * 32) >> B.fshift > 163840) B.fshift++;
+    const uint32_t fwords = masked && n && B.fshift <= 5 ? (uint32_t)((((nblk * 32) >> B.fshift) + 15) / 16 * 4) : 0u;
     B.sp = (uint64_t*)s.scratch.take(nw * 8 + 8);
     B.dead = (uint64_t*)s.scratch.take(nw * 8 + 8);
     B.inf = (uint64_t*)s.scratch.take(nw * 8 + 8);
-    B.dcnt = (uint32_t*)s.scratch.take(nw * 4 + 8);
-    uint32_t* dpos = (uint32_t*)s.scratch.take((nw + 1) * 4 + 8);
-    uint32_t* kept = (uint32_t*)s.scratch.take(n * 4 + 8);
-    uint32_t* log = (uint32_t*)s.scratch.take(n * C * 4 + 8);
-    if (!B.sp || !B.dead || !B.inf || !B.dcnt || !dpos || !kept || !log) return set_error(VH_ERR_OOM, "scratch");
+    B.sus = (uint64_t*)s.scratch.take(nw * 8 + 8);
+    B.cnt = (uint32_t*)s.scratch.take(2 * nw * 4 + 8);
+    if (fwords) B.filt = (uint8_t*)s.scratch.take((uint64_t)fwords * 4 + 64);
+    uint32_t* dpos = (uint32_t*)s.scratch.take((2 * nw + 1) * 4 + 8);
+    uint2* masks = masked ? (uint2*)s.scratch.take(n * 8 + 8) : nullptr;
+    uint32_t* kept = masked ? nullptr : (uint32_t*)s.scratch.take(n * 4 + 8);
+    uint32_t* log = masked ? nullptr : (uint32_t*)s.scratch.take(n * C * 4 + 8);
+    if (!B.sp || !B.dead || !B.inf || !B.sus || !B.cnt || (fwords && !B.filt) || !dpos || (masked ? !masks : !kept || !log))
+        return set_error(VH_ERR_OOM, "scratch");
     uint64_t nd = 0, ne = 0;
     if (n) {
-        hipLaunchKernelGGL(k_contact_flags, dim3(grid_for(nw * 64, 256)), dim3(256), 0, st,
-                           (const uint64_t*)A.rstate(), A.died.as<uint8_t>(), n, (uint32_t)t, p, step, B);
-        if (scan_excl_u32(B.dcnt, dpos, nw, s.scratch, st)) return set_error(VH_ERR_DEVICE, "scan");
-        hipLaunchKernelGGL(k_contact_main, dim3(grid_for(n, 256)), dim3(256), staged ? 256 * C * 4 : 0, st,
-                           E.rows ? E.off.as<uint32_t>() : nullptr, E.src.as<uint32_t>(),
-                           (const uint64_t*)A.rstate(), (uint64_t*)A.wstate(), A.died_now.as<uint8_t>(), n,
-                           E.rows ? E.nrows[t] : 0ull, E.rowbase[t], (uint32_t)t, p, step, B, kept, log,
-                           staged);
-        HIPCHECK(hipGetLastError());
-        RC(E.off.ensure((n + 1) * 4 + 8, st));
-        if (scan_excl_u32(kept, E.off.as<uint32_t>(), n, s.scratch, st))
-            return set_error(VH_ERR_DEVICE, "scan");
+        hipLaunchKernelGGL(k_contact_flags, dim3((unsigned)nblk), dim3(256), 0, st, (const uint64_t*)A.rstate(),
+                           A.died.as<uint8_t>(), n, (uint32_t)t, p, step, B);
+        hipLaunchKernelGGL(k_contact_infect, dim3(grid_for(nw, INF_W)), dim3(256), 0, st, E.off.as<uint32_t>(),
+                           E.src.as<uint32_t>(), (const uint64_t*)A.rstate(), E.rows ? E.nrows[t] : 0ull, E.rowbase[t],
+                           (uint32_t)t, p, step, B);
+        const uint32_t* total;   // the contacts kept (less the deaths when masked)
+        if (masked) {
+            // blocks of 1024 when that leaves every CU one, as many per CU as
+            // their filters fit
+            const uint32_t cus = device_cus(), fb = fwords * 4;
+            const bool big = n >= 1024ull * cus || !fwords;
+            const uint32_t bs = big ? 1024u : 256u, fit = std::max(1u, std::min(2048u / bs, fb ? 163840u / fb : 32u));
+            const dim3 g((unsigned)std::min<uint64_t>((n + bs - 1) / bs, (uint64_t)cus * fit));
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, g, dim3(bs), fb, st, (const uint64_t*)A.rstate(), (uint64_t*)A.wstate(),
+                                   A.died_now.as<uint8_t>(), (uint32_t)n, (uint32_t)t, p, step, B, fwords, masks);
+            };
+            if (!fwords) launch(k_contact_main<1024, false>);   // (too many slots for a filter)
+            else if (big) launch(k_contact_main<1024, true>);
+            else launch(k_contact_main<256, true>);
+            HIPCHECK(hipGetLastError());
+            // deaths and contacts numbered in one scan (its differences hold
+            // modulo 2^32)
+            if (scan_excl_u32(B.cnt, dpos, 2 * nw, s.scratch, st)) return set_error(VH_ERR_DEVICE, "scan");
+            total = dpos + 2 * nw;
+        } else {
+            if (scan_excl_u32(B.cnt, dpos, nw, s.scratch, st)) return set_error(VH_ERR_DEVICE, "scan");
+            hipLaunchKernelGGL(k_contact_main_log, dim3((unsigned)nblk), dim3(256), 0, st, (const uint64_t*)A.rstate(),
+                               (uint64_t*)A.wstate(), A.died_now.as<uint8_t>(), (uint32_t)n, (uint32_t)t, p, step, B, kept,
+                               log);
+            HIPCHECK(hipGetLastError());
+            RC(E.off.ensure((n + 1) * 4 + 8, st));
+            if (scan_excl_u32(kept, E.off.as<uint32_t>(), n, s.scratch, st)) return set_error(VH_ERR_DEVICE, "scan");
+            total = E.off.as<uint32_t>() + n;
+        }
         HIPCHECK(hipMemcpyAsync((uint32_t*)s.d_stats.p, dpos + nw, 4, hipMemcpyDeviceToDevice, st));
-        HIPCHECK(hipMemcpyAsync((uint32_t*)s.d_stats.p + 1, E.off.as<uint32_t>() + n, 4,
-                                hipMemcpyDeviceToDevice, st));
+        HIPCHECK(hipMemcpyAsync((uint32_t*)s.d_stats.p + 1, total, 4, hipMemcpyDeviceToDevice, st));
         RC(readback(s, 1));
         nd = ((const uint32_t*)s.h_stats)[0];
         ne = ((const uint32_t*)s.h_stats)[1];
+        if (masked) ne = (uint32_t)(ne - nd);
     }
     if (nd) {
         uint64_t consumed = std::min<uint64_t>(nd, A.nreuse);
@@ -2482,28 +2662,30 @@ int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t st
             if (A.nextid - 1 + fresh > n)
                 fill_u8(A.died_now.as<uint8_t>() + n, 0, A.nextid - 1 + fresh - n, st);
         }
-        hipLaunchKernelGGL(k_contact_births, dim3(grid_for(n, 256)), dim3(256), 0, st, n, (uint32_t)t, p,
-                           step, B, dpos, A.reuse.as<uint32_t>(), A.nreuse, A.nextid, (uint64_t*)A.wstate(),
-                           A.died.as<uint8_t>());
+        hipLaunchKernelGGL(k_contact_births, dim3(grid_for(nw, 128)), dim3(128), 0, st, (uint32_t)t, p, step, B, dpos,
+                           A.reuse.as<uint32_t>(), A.nreuse, A.nextid, (uint64_t*)A.wstate(), A.died.as<uint8_t>());
         A.nreuse -= consumed;
         A.nextid += fresh;
         RC(A.reuse.ensure((A.nreuse + nd) * 4 + 8, st, A.nreuse * 4));
-        hipLaunchKernelGGL(k_contact_deaths, dim3(grid_for(n, 256)), dim3(256), 0, st, n, B, dpos,
+        hipLaunchKernelGGL(k_contact_deaths, dim3(grid_for(nw, 128)), dim3(128), 0, st, B, dpos,
                            A.reuse.as<uint32_t>(), A.nreuse, A.died.as<uint8_t>());
         A.nreuse += nd;
         HIPCHECK(hipGetLastError());
     }
     // rows = caller slots; rows of dead callers and of newborns are empty
     uint64_t rows = std::max(n, A.nextid - 1);
-    RC(E.off.ensure((rows + 1) * 4 + 8, st, (n + 1) * 4));
+    RC(E.off.ensure((rows + 1) * 4 + 8, st, masked ? 0 : (n + 1) * 4));
+    RC(E.src.ensure(ne * 4 + 8, st));
     if (!n) fill_u32(E.off.as<uint32_t>(), 0, 1, st);
+    else if (masked)
+        hipLaunchKernelGGL(k_contact_edges, dim3((unsigned)nblk), dim3(256), 256 * C * 4, st, (uint32_t)n, (uint32_t)t,
+                           p, step, B, masks, dpos, E.off.as<uint32_t>(), E.src.as<uint32_t>());
+    else if (ne)
+        hipLaunchKernelGGL(k_contact_edges_log, dim3((unsigned)nblk), dim3(256), 0, st, n, C, kept, log,
+                           E.off.as<uint32_t>(), E.src.as<uint32_t>());
     if (rows > n)
         hipLaunchKernelGGL(k_contact_extend, dim3(grid_for(rows - n, 256)), dim3(256), 0, st,
                            E.off.as<uint32_t>(), n, rows);
-    RC(E.src.ensure(ne * 4 + 8, st));
-    if (ne)
-        hipLaunchKernelGGL(k_contact_edges, dim3(grid_for(n, 256)), dim3(256), staged ? 2 * 256 * C * 4 : 0,
-                           st, n, C, kept, log, E.off.as<uint32_t>(), E.src.as<uint32_t>(), staged);
     HIPCHECK(hipGetLastError());
     for (int u = 0; u <= VH_MAXA; u++) {
         E.rowbase[u] = 0;

@@ -192,13 +192,17 @@ int opinion_defer_launch(OpinionDefer& c, hipStream_t st, DevBuf& dev, void** ho
 // diffuse over an unchanged device stencil: neighbours from the stencil
 // arithmetic instead of the CSR (same neighbour set; the body is an OR)
 int launch_diffuse_stencil(Sim& s, int t, int et, uint32_t field);
-// contact model: per-step flag bitmaps, one bit per slot (64 per word)
+// contact model: per-step flag bitmaps, one bit per slot (64 per word), and
+// the per-word counts whose scan numbers deaths and contacts
 struct ContactBits {
     uint64_t* sp;     // dead in the read state or dying in this step (padding set)
     uint64_t* dead;   // dead in the read state (padding set)
     uint64_t* inf;    // infected in the read state
-    uint32_t* dcnt;   // deaths per word
+    uint64_t* sus;    // susceptible, living through this step; then those of them that get infected
+    uint32_t* cnt;    // deaths per word, then (from nwords on) contacts kept per word
     uint64_t nwords;
+    uint8_t* filt;    // one bit per group of 2^fshift slots: sp has a bit in it (null: no filter)
+    uint32_t fshift;
 };
 // one apply! of the contact model incl. its births, deaths and contact CSR
 int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t step, uint64_t* ndeaths);

@@ -1527,7 +1527,9 @@ static int apply_one(Sim& s, const vh_apply_desc* d) {
             HIPCHECK(hipMemcpyAsync(A.wstate(), A.rstate(), A.nslots * A.bytes,
                                     hipMemcpyDeviceToDevice, st));
         }
-        if (A.mortal && A.nslots) fill_u8(A.died_now.as<uint8_t>(), 0, A.nslots, st);
+        // (the contact body writes the flag of every slot of its call type)
+        if (A.mortal && A.nslots && !(kind == K_CONTACT && in_mask(callmask, t)))
+            fill_u8(A.died_now.as<uint8_t>(), 0, A.nslots, st);
     }
     for (int et = 0; et < m.ne; et++) s.e[et].writeable = in_mask(d->write_edges, et);
 
