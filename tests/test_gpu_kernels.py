@@ -216,3 +216,25 @@ def test_contact_masks(vh, ora, gpu_ready, C, R, pd, n):
         assert np.array_equal(a[~da], b[~db]), k
         for x, y in zip(g.sim._read_edges(g.E)[:2], c.sim._read_edges(c.E)[:2]):
             assert np.array_equal(x, y), k
+
+
+@pytest.mark.parametrize("expose", [0, 1])
+@pytest.mark.parametrize("block", [64, 256, 1024])
+def test_ensemble_four_agents_per_thread(vh, ora, gpu_ready, opts, block, expose):
+    """Members around a thread's four agents, a bitmap word and a tile (256 to
+    4096 agents), against their solo runs on the checker."""
+    opts(sir_expose=expose, sir_expose_min=0)
+    E = vh.ensemble.Ensemble()
+    E.set_config(block, False)
+    E.set_tiles([4, 4, 4])
+    sizes = [1, 3, 33, 255, 1023, 1025, 4097, 12345]
+    ids = [E.add_sir(n, 6.0, 0.2, 50 + k, 60 + k, n_init=max(1, n // 60)) for k, n in enumerate(sizes)]
+    E.step(9)
+    E.step(3, use_graph=False)
+    for k, (mid, n) in enumerate(zip(ids, sizes)):
+        m = vh.models.build_sir(ora, n, seed=50 + k, n_init=max(1, n // 60), init="frac",
+                                edges=vh.inputs.graph_gnp(n, 6.0, 60 + k))
+        for _ in range(12):
+            vh.models.step_sir(ora, m, p_inf=0.2, seed=50 + k, recovery=7)
+        got, want = E.read(mid)[0], m.sim._read_agents(m.T)[0]
+        assert np.array_equal(np.ascontiguousarray(got).view(np.uint8), np.ascontiguousarray(want).view(np.uint8)), n

@@ -37,6 +37,34 @@ __device__ __forceinline__ bool vh_any_infecting(uint64_t pre, uint64_t pt, uint
     }
     return false;
 }
+// The exposure of a wave's infected agents (every lane of the wave calls; inf:
+// the lane's agent i is to be marked from): the bit of each of their
+// out-neighbours is set in `bits`. Four agents at a time, 16 lanes each: the
+// few infected of a wave have their out-edges in flight together, where a lane
+// of its own walks them one load and one atomic after the other.
+__device__ __forceinline__ void vh_expose_wave(bool inf, uint64_t i, const uint32_t* __restrict__ out_off,
+                                               const uint32_t* __restrict__ out_dst, uint32_t* __restrict__ bits) {
+    uint64_t m = __ballot(inf);
+    if (!m) return;
+    const uint32_t lane = threadIdx.x & 63u, g = lane >> 4, l = lane & 15u;
+    uint32_t b = 0, e = 0;
+    if (inf) {
+        b = out_off[i];
+        e = out_off[i + 1];
+    }
+    while (m) {
+        uint64_t t = m;   // its lowest bit: the agent of lane group g
+        for (uint32_t q = 0; q < g; q++) t &= t ? t - 1ull : 0ull;
+        const int who = t ? (int)__builtin_ctzll(t) : 0;
+        const uint32_t bb = (uint32_t)__shfl((int)b, who, 64), ee = (uint32_t)__shfl((int)e, who, 64);
+        if (t)
+            for (uint32_t k = bb + l; k < ee; k += 16) {
+                const uint32_t v = out_dst[k];
+                atomicOr(bits + (v >> 5), 1u << (v & 31u));
+            }
+        for (uint32_t q = 0; q < 4; q++) m &= m ? m - 1ull : 0ull;
+    }
+}
 // stream keys of the model bodies (the `c` word of vh_hash)
 #define VH_KEY_RECOVER (1ull << 40)
 #define VH_KEY_DEATH   (2ull << 40)

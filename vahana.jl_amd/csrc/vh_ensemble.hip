@@ -106,6 +106,7 @@ __global__ void k_member_offsets(const uint32_t* __restrict__ keys, uint64_t ne,
     out_off[v] = (uint32_t)lo;
 }
 
+constexpr uint32_t ENS_TILE = 4096;   // agents of a logical block at most (1024 threads, four each)
 constexpr int ENS_CLASSES = 3;   // member size classes of the tile choice
 
 struct MemberDesc {
@@ -189,10 +190,12 @@ __device__ __forceinline__ uint32_t ens_block(uint32_t nblocks, uint32_t remap) 
     return b;   // >= nblocks: no block
 }
 
+typedef uint32_t ens_u32x4 __attribute__((ext_vector_type(4)));
 // grid-stride over the logical blocks (of their member's `tile` agents):
 // members whose pass is off, and blocks without an agent to mark (by the
 // block's counts of the previous launch: infected, and infected in it), cost
-// a read or two per logical block, not a block launch
+// a read or two per logical block, not a block launch (7 us a step of 48
+// members; 17 us with a lane per agent that walked its out-edges)
 __global__ __launch_bounds__(256) void k_ens_expose(const MemberDesc* __restrict__ md,
                                                     const uint32_t* __restrict__ bmember,
                                                     const uint32_t* __restrict__ bstart, uint32_t nblocks,
@@ -209,30 +212,37 @@ __global__ __launch_bounds__(256) void k_ens_expose(const MemberDesc* __restrict
         const MemberDesc& m = md[mi];
         uint32_t* bits = m.bits + parity * m.nw;
         const uint64_t a0 = bstart[lb];
-        for (uint32_t o = threadIdx.x; o < m.tile; o += 256) {
+        // four consecutive agents per lane (tiles are multiples of 64)
+        for (uint32_t o = 4 * threadIdx.x; o < m.tile; o += 4 * 256) {
             const uint64_t i = a0 + o;
-            if (i >= m.n) continue;
-            const uint32_t st = m.rs[i];
-            // infected, and (unless full) infected in the previous launch
-            if ((st & 0xFFu) != VH_I || (!full && (st >> 16) != 0u)) continue;
-            for (uint32_t k = m.out_off[i]; k < m.out_off[i + 1]; k++) {
-                const uint32_t v = m.out_dst[k];
-                atomicOr(bits + (v >> 5), 1u << (v & 31u));
-            }
+            const uint32_t in = i >= m.n ? 0u : m.n - i < 4 ? (uint32_t)(m.n - i) : 4u;
+            ens_u32x4 v = {0u, 0u, 0u, 0u};
+            if (in == 4) v = *(const ens_u32x4*)(m.rs + i);
+            else
+                for (uint32_t q = 0; q < in; q++) v[q] = m.rs[i + q];
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++)
+                // infected, and (unless full) infected in the previous launch
+                vh_expose_wave(q < in && (v[q] & 0xFFu) == VH_I && (full || (v[q] >> 16) == 0u), i + q, m.out_off,
+                               m.out_dst, bits);
         }
     }
 }
 
 // one launch for every member: logical block b belongs to member
 // bmember[b] and covers agents [bstart[b], bstart[b] + tile) of it, thread t
-// the agents bstart[b] + t + k * blockDim, k < tile / blockDim (dec null: no
-// exposure; else per-block infected counts of the written state go to
+// the agents bstart[b] + t + k * blockDim, k < tile / blockDim, or with four
+// agents per thread bstart[b] + 4 t and the three after it, the agents that
+// draw listed (48 members, 7.6 10^6 agents, 200 steps of an epidemic: one agent
+// per thread 52 us a step and 39 us with nothing to draw, blocks' chains of
+// loads; four per thread 32 and 15 us, listed 26 us) (dec null: no exposure; else per-block infected counts of the written state go to
 // blkcnt[(parity ^ 1) * nblocks + b])
 __global__ void k_sir_ensemble(const MemberDesc* __restrict__ md, const uint32_t* __restrict__ bmember,
                                const uint32_t* __restrict__ bstart, uint32_t nblocks, uint32_t remap,
                                const uint32_t* __restrict__ dec, uint32_t parity, uint64_t lidx,
                                uint32_t* __restrict__ blkcnt) {
-    __shared__ uint32_t s_inf[16], s_new[16];
+    __shared__ uint32_t s_inf[16], s_new[16], s_n, s_bits[ENS_TILE / 32];
+    __shared__ uint16_t s_list[ENS_TILE];
     const uint32_t b = ens_block(nblocks, remap);
     if (b >= nblocks) return;   // whole block
     const uint32_t mi = bmember[b];
@@ -243,28 +253,84 @@ __global__ void k_sir_ensemble(const MemberDesc* __restrict__ md, const uint32_t
     const bool ex = (dm & 1u) != 0u;
     const uint32_t apt = m.tile / blockDim.x;
     uint32_t c_inf = 0, c_new = 0;   // this wave's infected (and newly infected) agents
-    for (uint32_t k = 0; k < apt; k++) {
-        const uint64_t i = a0 + threadIdx.x + (uint64_t)k * blockDim.x;
-        const bool in = i < m.n;
-        uint32_t s = in ? m.rs[i] : 0u;
+    // susceptible agent i gets infected in this step
+    auto infects = [&](uint64_t i) -> bool {
+        const uint64_t pre = vh_hash_pre(m.seed, vh_make_id(m.type, i + 1), m.step);
+        // the draw first, the source's state only below p (as in k_sir)
+        return vh_any_infecting(pre, vh_u01_below(m.p), m.off[i], m.off[i + 1],
+                                [&](uint32_t q) { return (m.rs[m.src[q] - 1] & 0xFFu) == VH_I; });
+    };
+    // the new state of an agent in state s
+    auto next = [&](uint32_t s, bool infected) -> uint32_t {
         const uint32_t h = s & 0xFFu;
-        const bool skip = in && h == VH_S && ex && !((m.bits[parity * m.nw + (i >> 5)] >> (i & 31u)) & 1u);
-        if (in && h == VH_S && !skip) {
-            const uint64_t pre = vh_hash_pre(m.seed, vh_make_id(m.type, i + 1), m.step);
-            const uint64_t pt = vh_u01_below(m.p);
-            const uint32_t bb = m.off[i], e = m.off[i + 1];
-            // the draw first, the source's state only below p (as in k_sir)
-            if (vh_any_infecting(pre, pt, bb, e,
-                                 [&](uint32_t q) { return (m.rs[m.src[q] - 1] & 0xFFu) == VH_I; }))
-                s = (s & 0xFF00u) | VH_I;
-        } else if (in && h == VH_I) {
-            const uint32_t days = ((s >> 16) + 1u) & 0xFFFFu;
-            s = (s & 0xFF00u) | (days << 16) | (days >= m.rec ? VH_R : VH_I);
+        if (h == VH_S && infected) return (s & 0xFF00u) | VH_I;
+        if (h != VH_I) return s;
+        const uint32_t days = ((s >> 16) + 1u) & 0xFFFFu;
+        return (s & 0xFF00u) | (days << 16) | (days >= m.rec ? VH_R : VH_I);
+    };
+    auto count = [&](bool in, uint32_t s) {
+        c_inf += (uint32_t)__popcll(__ballot(in && (s & 0xFFu) == VH_I));
+        c_new += (uint32_t)__popcll(__ballot(in && (s & 0xFFu) == VH_I && (s >> 16) == 0u));
+    };
+    if (apt == 4) {
+        // four consecutive agents per thread: one 16-byte load and store, the
+        // four bits of one bitmap word. The agents that draw are listed and
+        // the block's threads take them off the list, so that all lanes draw
+        if (threadIdx.x == 0) s_n = 0;
+        for (uint32_t q = threadIdx.x; q < m.tile / 32; q += blockDim.x) s_bits[q] = 0;
+        __syncthreads();
+        const uint32_t o = 4 * threadIdx.x, lane = threadIdx.x & 63u;
+        const uint64_t i = a0 + o;
+        const uint32_t in = i >= m.n ? 0u : m.n - i < 4 ? (uint32_t)(m.n - i) : 4u;
+        ens_u32x4 v = {0u, 0u, 0u, 0u};
+        if (in == 4) v = *(const ens_u32x4*)(m.rs + i);
+        else
+            for (uint32_t q = 0; q < in; q++) v[q] = m.rs[i + q];
+        const uint32_t bits = !ex ? 0xFu : in ? m.bits[parity * m.nw + (i >> 5)] >> (i & 31u) : 0u;
+        uint64_t need[4];
+        uint32_t total = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++) {
+            need[q] = __ballot(q < in && (v[q] & 0xFFu) == VH_S && ((bits >> q) & 1u));
+            total += (uint32_t)__popcll(need[q]);
         }
-        if (in) m.ws[i] = s;
-        if (dec) {
-            c_inf += (uint32_t)__popcll(__ballot(in && (s & 0xFFu) == VH_I));
-            c_new += (uint32_t)__popcll(__ballot(in && (s & 0xFFu) == VH_I && (s >> 16) == 0u));
+        if (total) {   // uniform per wave
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(&s_n, total);
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++) {
+                if ((need[q] >> lane) & 1ull)
+                    s_list[base + (uint32_t)__popcll(need[q] & ((1ull << lane) - 1ull))] = (uint16_t)(o + q);
+                base += (uint32_t)__popcll(need[q]);
+            }
+        }
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < s_n; k += blockDim.x) {
+            const uint32_t l = s_list[k];
+            if (infects(a0 + l)) atomicOr(&s_bits[l >> 5], 1u << (l & 31u));
+        }
+        __syncthreads();
+        const uint32_t hit = s_bits[o >> 5] >> (o & 31u);
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++) v[q] = next(v[q], (hit >> q) & 1u);
+        if (in == 4) *(ens_u32x4*)(m.ws + i) = v;
+        else
+            for (uint32_t q = 0; q < in; q++) m.ws[i + q] = v[q];
+        if (dec)
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++) count(q < in, v[q]);
+    } else {
+        for (uint32_t k = 0; k < apt; k++) {
+            const uint64_t i = a0 + threadIdx.x + (uint64_t)k * blockDim.x;
+            const bool in = i < m.n;
+            uint32_t s = in ? m.rs[i] : 0u;
+            const bool skip = in && ex && !((m.bits[parity * m.nw + (i >> 5)] >> (i & 31u)) & 1u);
+            if (in) {
+                s = next(s, (s & 0xFFu) == VH_S && !skip && infects(i));
+                m.ws[i] = s;
+            }
+            if (dec) count(in, s);
         }
     }
     if (dec) {
@@ -380,8 +446,13 @@ struct vh_ensemble {
     size_t h_table_cap = 0;
     void* h_descs = nullptr;
     size_t h_descs_cap = 0;
-    uint32_t block = 256, remap = 1;
-    uint32_t apt[ENS_CLASSES] = {1, 1, 1};   // agents per thread of each size class
+    // plain block order: contiguous runs of blocks per XCD leave some XCDs with
+    // the members whose epidemics are over (48 members, 7.6 10^6 agents: 47 us
+    // a step against 32). Four agents per thread from 10^4 agents (a block of
+    // a smaller member would leave the launch with few blocks; 256 threads in
+    // place of 128 or 512: 25.9, 26.5, 28.0 us)
+    uint32_t block = 256, remap = 0;
+    uint32_t apt[ENS_CLASSES] = {1, 4, 4};   // agents per thread of each size class
     DevBuf d_desc, d_bmember, d_bstart;
     DevBuf d_mblk, d_blkcnt, d_dec;   // exposure: member block ranges, per-block counts, decisions
     Scratch oscr;                     // scratch of the members' out-edge builds (step stream)
