@@ -238,3 +238,26 @@ def test_ensemble_four_agents_per_thread(vh, ora, gpu_ready, opts, block, expose
             vh.models.step_sir(ora, m, p_inf=0.2, seed=50 + k, recovery=7)
         got, want = E.read(mid)[0], m.sim._read_agents(m.T)[0]
         assert np.array_equal(np.ascontiguousarray(got).view(np.uint8), np.ascontiguousarray(want).view(np.uint8)), n
+
+
+# around a tile of 2048 pairs, several, and the switch to tiles of 8192
+# (4 194 304) with and without a partial last tile
+@pytest.mark.parametrize("ne,n", [(1, 1), (63, 300), (2047, 5), (2048, 70_000), (2049, 256), (70_001, 66_000),
+                                  (4_194_303, 100_000), (4_194_304, 257), (4_202_500, 17_000_000)])
+def test_edges_sorted_stably(vh, gpu_ready, ne, n):
+    """The CSR of edges added in random order: targets ascending, each
+    target's edges (source, state) in the order they were added."""
+    rng = np.random.default_rng(ne)
+    A, E = vh.struct("A", [("x", "u1")]), vh.struct("E", [("k", "<u4")])
+    sim = vh.create_simulation(vh.ModelTypes() | vh.register_agenttype_(A, "Immortal")
+                               | vh.register_edgetype_(E, target=A) | vh.create_model("sort"))
+    sim._add_agents_array(A, np.zeros(n, dtype=A.dtype))
+    tid = np.uint64(1) << np.uint64(56)
+    fr, to = (tid | rng.integers(1, n + 1, ne).astype(np.uint64) for _ in range(2))
+    st = np.zeros(ne, dtype=E.dtype)
+    st["k"] = np.arange(ne)
+    sim._add_edges_array(E, fr, to, st)
+    vh.finish_init_(sim)
+    order = np.argsort(to, kind="stable")
+    t, f, s = sim._read_edges(E)
+    assert np.array_equal(t, to[order]) and np.array_equal(f, fr[order]) and np.array_equal(s["k"], order)

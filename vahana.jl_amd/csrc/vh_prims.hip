@@ -201,108 +201,132 @@ int scan_excl_u64(const uint32_t* in, uint64_t* out, uint64_t n, Scratch& s, hip
 }
 
 // ------------------------------------------------------------------ radix sort
-// 8-bit digits, 256 threads x 16 items per tile.  Tile element e of wave w is
-// tile_base + w*1024 + i*64 + lane (i = 0..15), so each wave walks its
-// contiguous quarter in index order; ranks inside an item row come from a
-// ballot match over the 8 digit bits, which keeps the sort stable.
-constexpr int RB = 256;
-constexpr int RI = 16;
-constexpr int RTILE = RB * RI;
+// 8-bit digits, tiles of 512 threads x RI items.  Tile element e of wave w is
+// tile_base + w * 64 RI + i * 64 + lane (i < RI), so each wave walks its
+// contiguous eighth in index order; ranks inside an item row come from a
+// ballot match over the 8 digit bits and the wave's count of the digit so
+// far, which keeps the sort stable.
+//
+// The scatter puts the tile in digit order in LDS first and writes it from
+// there, so that the elements of a digit leave as one run: written straight
+// from the ranks, a wave's 64 elements went to as many lines, and the lines of
+// all tiles at work (2 x 256 each) were evicted half written (a pass over 10^8
+// pairs: 1416 us, so 558; over 10^6: 31, so 21). Tiles of 8192 make runs of 32,
+// a line; below RADIX_LARGE pairs tiles of 2048 leave no CU idle.
+constexpr int RB = 512;
 constexpr int RW = RB / 64;
+constexpr uint64_t RADIX_LARGE = 4u << 20;
 
+template <int RI>
 __global__ __launch_bounds__(RB) void k_radix_hist(const uint32_t* __restrict__ keys, uint64_t n,
                                                    uint32_t shift, uint32_t ntiles,
                                                    uint32_t* __restrict__ hist) {
     __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0;
+    if (threadIdx.x < 256) h[threadIdx.x] = 0;
     __syncthreads();
-    uint64_t base = (uint64_t)blockIdx.x * RTILE;
+    const uint64_t base = (uint64_t)blockIdx.x * (RB * RI);
 #pragma unroll 4
     for (int i = 0; i < RI; i++) {
-        uint64_t e = base + (uint64_t)i * RB + threadIdx.x;
+        const uint64_t e = base + (uint64_t)i * RB + threadIdx.x;
         if (e < n) atomicAdd(&h[(keys[e] >> shift) & 255u], 1u);
     }
     __syncthreads();
-    hist[(uint64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    if (threadIdx.x < 256) hist[(uint64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
+template <int RI>
 __global__ __launch_bounds__(RB) void k_radix_scatter(const uint32_t* __restrict__ kin,
                                                       const uint32_t* __restrict__ vin,
                                                       uint32_t* __restrict__ kout,
                                                       uint32_t* __restrict__ vout, uint64_t n,
                                                       uint32_t shift, uint32_t ntiles,
                                                       const uint32_t* __restrict__ goff) {
-    __shared__ uint32_t whist[RW][256];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int d = threadIdx.x; d < RW * 256; d += RB) (&whist[0][0])[d] = 0;
+    constexpr uint32_t TILE = RB * RI;
+    __shared__ uint32_t whist[RW][256];   // the waves' digit counts, then their first places in the tile
+    __shared__ uint32_t gbase[256], wsum[4];
+    __shared__ uint32_t sk[TILE], sv[TILE];
+    const uint32_t tid = threadIdx.x;
+    const int lane = tid & 63, w = tid >> 6;
+    for (uint32_t d = tid; d < RW * 256; d += RB) (&whist[0][0])[d] = 0;
     __syncthreads();
-    const uint64_t wbase = (uint64_t)blockIdx.x * RTILE + (uint64_t)w * (64 * RI);
-    uint32_t k[RI], v[RI];
-#pragma unroll
-    for (int i = 0; i < RI; i++) {
-        uint64_t e = wbase + (uint64_t)i * 64 + lane;
-        if (e < n) {
-            k[i] = kin[e];
-            v[i] = vin ? vin[e] : (uint32_t)e;
-            atomicAdd(&whist[w][(k[i] >> shift) & 255u], 1u);
-        }
-    }
-    __syncthreads();
-    {
-        // digit d: running offset over the waves of this tile
-        const int d = threadIdx.x;
-        uint32_t b = goff[(uint64_t)d * ntiles + blockIdx.x];
-#pragma unroll
-        for (int q = 0; q < RW; q++) {
-            uint32_t c = whist[q][d];
-            whist[q][d] = b;
-            b += c;
-        }
-    }
-    __syncthreads();
+    const uint64_t tbase = (uint64_t)blockIdx.x * TILE, wbase = tbase + (uint64_t)w * (64 * RI);
+    const uint32_t cnt = n - tbase < TILE ? (uint32_t)(n - tbase) : TILE;
     const uint64_t lt = (1ull << lane) - 1ull;
+    uint32_t k[RI], v[RI], rank[RI];
 #pragma unroll
     for (int i = 0; i < RI; i++) {
-        uint64_t e = wbase + (uint64_t)i * 64 + lane;
-        const bool valid = e < n;
-        uint32_t d = valid ? ((k[i] >> shift) & 255u) : 256u;
+        const uint64_t e = wbase + (uint64_t)i * 64 + lane;
+        k[i] = e < n ? kin[e] : 0u;
+        v[i] = vin ? (e < n ? vin[e] : 0u) : (uint32_t)e;
+    }
+#pragma unroll
+    for (int i = 0; i < RI; i++) {
+        const bool valid = wbase + (uint64_t)i * 64 + lane < n;
+        const uint32_t d = (k[i] >> shift) & 255u;
         uint64_t peers = __ballot(valid);
 #pragma unroll
-        for (int b = 0; b < 9; b++) {
-            uint64_t bal = __ballot((d >> b) & 1u);
+        for (int b = 0; b < 8; b++) {
+            const uint64_t bal = __ballot((d >> b) & 1u);
             peers &= ((d >> b) & 1u) ? bal : ~bal;
         }
-        uint32_t rank = 0, base = 0;
-        if (valid) {
-            rank = (uint32_t)__popcll(peers & lt);
-            base = whist[w][d];
-        }
+        const uint32_t r = (uint32_t)__popcll(peers & lt);
+        rank[i] = valid ? whist[w][d] + r : 0u;
         __builtin_amdgcn_wave_barrier();
-        if (valid) {
-            kout[base + rank] = k[i];
-            vout[base + rank] = v[i];
-            if (rank == 0) whist[w][d] = base + (uint32_t)__popcll(peers);
-        }
+        if (valid && r == 0) whist[w][d] += (uint32_t)__popcll(peers);
         __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    // digit d: its place in the tile and the waves' places behind it
+    uint32_t c = 0, incl = 0;
+    if (tid < 256) {
+#pragma unroll
+        for (int q = 0; q < RW; q++) {
+            const uint32_t t = whist[q][tid];
+            whist[q][tid] = c;
+            c += t;
+        }
+        incl = wave_incl_scan(c);
+        if (lane == 63) wsum[w] = incl;
+    }
+    __syncthreads();
+    if (tid < 256) {
+        uint32_t start = incl - c;
+        for (int q = 0; q < w; q++) start += wsum[q];
+#pragma unroll
+        for (int q = 0; q < RW; q++) whist[q][tid] += start;
+        gbase[tid] = goff[(uint64_t)tid * ntiles + blockIdx.x] - start;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < RI; i++) {
+        if (wbase + (uint64_t)i * 64 + lane < n) {
+            const uint32_t p = whist[w][(k[i] >> shift) & 255u] + rank[i];
+            sk[p] = k[i];
+            sv[p] = v[i];
+        }
+    }
+    __syncthreads();
+    for (uint32_t p = tid; p < cnt; p += RB) {
+        const uint32_t key = sk[p], o = gbase[(key >> shift) & 255u] + p;
+        kout[o] = key;
+        vout[o] = sv[p];
     }
 }
 
-int radix_sort_pairs(uint32_t** keys, uint32_t** vals, uint32_t* kalt, uint32_t* valt, uint64_t n,
-                     uint32_t bits, bool iota_vals, Scratch& s, hipStream_t st) {
-    if (n == 0) return 0;
-    uint32_t ntiles = (uint32_t)((n + RTILE - 1) / RTILE);
+template <int RI>
+static int radix_sort_impl(uint32_t** keys, uint32_t** vals, uint32_t* kalt, uint32_t* valt, uint64_t n,
+                           uint32_t bits, bool iota_vals, Scratch& s, hipStream_t st) {
+    const uint32_t ntiles = (uint32_t)((n + RB * RI - 1) / (RB * RI));
     uint32_t* hist = (uint32_t*)s.take((uint64_t)256 * ntiles * sizeof(uint32_t));
     uint32_t* goff = (uint32_t*)s.take(((uint64_t)256 * ntiles + 1) * sizeof(uint32_t));
     if (!hist || !goff) return -3;
     uint32_t *kin = *keys, *vin = *vals, *kout = kalt, *vout = valt;
-    if (bits == 0) bits = 1;
     bool first = true;
     for (uint32_t shift = 0; shift < bits; shift += 8) {
-        hipLaunchKernelGGL(k_radix_hist, dim3(ntiles), dim3(RB), 0, st, kin, n, shift, ntiles,
-                           hist);
+        hipLaunchKernelGGL(k_radix_hist<RI>, dim3(ntiles), dim3(RB), 0, st, kin, n, shift, ntiles, hist);
         int r = scan_excl_u32(hist, goff, (uint64_t)256 * ntiles, s, st);
         if (r) return r;
-        hipLaunchKernelGGL(k_radix_scatter, dim3(ntiles), dim3(RB), 0, st, kin,
+        hipLaunchKernelGGL(k_radix_scatter<RI>, dim3(ntiles), dim3(RB), 0, st, kin,
                            (first && iota_vals) ? (const uint32_t*)nullptr : vin, kout, vout, n,
                            shift, ntiles, goff);
         first = false;
@@ -312,6 +336,13 @@ int radix_sort_pairs(uint32_t** keys, uint32_t** vals, uint32_t* kalt, uint32_t*
     *keys = kin;
     *vals = vin;
     return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+int radix_sort_pairs(uint32_t** keys, uint32_t** vals, uint32_t* kalt, uint32_t* valt, uint64_t n,
+                     uint32_t bits, bool iota_vals, Scratch& s, hipStream_t st) {
+    if (n == 0) return 0;
+    if (bits == 0) bits = 1;
+    return n < RADIX_LARGE ? radix_sort_impl<4>(keys, vals, kalt, valt, n, bits, iota_vals, s, st)
+                           : radix_sort_impl<16>(keys, vals, kalt, valt, n, bits, iota_vals, s, st);
 }
 
 // ------------------------------------------------------------------ helpers
