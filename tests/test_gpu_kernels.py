@@ -261,3 +261,25 @@ def test_edges_sorted_stably(vh, gpu_ready, ne, n):
     order = np.argsort(to, kind="stable")
     t, f, s = sim._read_edges(E)
     assert np.array_equal(t, to[order]) and np.array_equal(f, fr[order]) and np.array_equal(s["k"], order)
+
+
+@pytest.mark.parametrize("late", [False, True])
+def test_ensemble_out_edges_together(vh, ora, gpu_ready, opts, late):
+    """Out-edges of several members from one sort: members without edges, of
+    one agent, around 256 rows, and one whose 9 10^6 edges end a batch; the
+    exposure pass on from the start, or only after the members were added."""
+    opts(sir_expose=0 if late else 1, sir_expose_min=0)
+    E = vh.ensemble.Ensemble()
+    sizes = [(1, 0.0), (256, 4.0), (300, 0.0), (255, 9.0), (257, 1.0), (900_000, 10.0), (513, 3.0), (70_000, 12.0)]
+    ids = [E.add_sir(n, d, 0.2, 70 + k, 80 + k, n_init=max(1, n // 60)) for k, (n, d) in enumerate(sizes)]
+    if late:
+        E.step(2)
+        opts(sir_expose=1)
+    E.step(6)
+    for k, (mid, (n, d)) in enumerate(zip(ids, sizes)):
+        m = vh.models.build_sir(ora, n, seed=70 + k, n_init=max(1, n // 60), init="frac",
+                                edges=vh.inputs.graph_gnp(n, d, 80 + k))
+        for _ in range(8 if late else 6):
+            vh.models.step_sir(ora, m, p_inf=0.2, seed=70 + k, recovery=7)
+        got, want = E.read(mid)[0], m.sim._read_agents(m.T)[0]
+        assert np.array_equal(np.ascontiguousarray(got).view(np.uint8), np.ascontiguousarray(want).view(np.uint8)), n

@@ -339,30 +339,6 @@ __global__ __launch_bounds__(256) void k_sir_expose(const uint32_t* __restrict__
     }
 }
 
-// row of every in-edge (transpose input) and its source index as key
-__global__ void k_edge_rows(const uint32_t* __restrict__ off, const uint32_t* __restrict__ src, uint64_t rows,
-                            uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= rows) return;
-    for (uint32_t k = off[r]; k < off[r + 1]; k++) {
-        keys[k] = src[k] - 1u;
-        vals[k] = (uint32_t)r;
-    }
-}
-// off[v] = first index whose key >= v, v in [0, n]
-__global__ void k_sorted_offsets(const uint32_t* __restrict__ keys, uint64_t ne, uint64_t n,
-                                 uint32_t* __restrict__ off) {
-    uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v > n) return;
-    uint64_t lo = 0, hi = ne;
-    while (lo < hi) {
-        uint64_t mid = (lo + hi) >> 1;
-        if ((uint64_t)keys[mid] < v) lo = mid + 1;
-        else hi = mid;
-    }
-    off[v] = (uint32_t)lo;
-}
-
 __global__ __launch_bounds__(256) void k_sir(const uint32_t* __restrict__ off,
                                              const uint32_t* __restrict__ src,
                                              const uint32_t* __restrict__ rs,
@@ -2046,28 +2022,16 @@ static int check_model_layout(Sim& s, int t, int et, uint32_t abytes, uint32_t e
 
 
 // Out-edges of E's rows (one agent type, rows from 0, 1-based sources up to
-// nsrc): the transpose, by a stable radix sort of the in-edges by source;
-// stamps array of nsrc entries, cleared once
+// nsrc): the transpose of its in-edges; the exposure bitmap and the counters
 static int build_out_csr(Sim& s, EdgeStore& E, uint64_t nsrc) {
     if (E.out_version == E.version && E.expo.p && E.expo.cap >= ((nsrc + 31) / 32) * 4 + 16) return VH_OK;
     hipStream_t st = s.stream;
-    const uint64_t ne = E.nedges, rows = E.rows;
-    uint32_t* keys = (uint32_t*)s.scratch.take(ne * 4 + 4);
-    uint32_t* vals = (uint32_t*)s.scratch.take(ne * 4 + 4);
-    uint32_t* ka = (uint32_t*)s.scratch.take(ne * 4 + 4);
-    uint32_t* va = (uint32_t*)s.scratch.take(ne * 4 + 4);
-    if (!keys || !vals || !ka || !va) return set_error(VH_ERR_OOM, "scratch");
-    hipLaunchKernelGGL(k_edge_rows, dim3(grid_for(rows, 256)), dim3(256), 0, st, E.off.as<uint32_t>(),
-                       E.src.as<uint32_t>(), rows, keys, vals);
-    uint32_t bits = 1;
-    while (bits < 32 && (nsrc >> bits) != 0) bits++;
-    if (radix_sort_pairs(&keys, &vals, ka, va, ne, bits, false, s.scratch, st))
-        return set_error(VH_ERR_DEVICE, "radix sort failed");
     RC(E.out_off.ensure((nsrc + 1) * 4 + 8, st));
-    RC(E.out_dst.ensure(ne * 4 + 8, st));
-    hipLaunchKernelGGL(k_sorted_offsets, dim3(grid_for(nsrc + 1, 256)), dim3(256), 0, st, keys, ne, nsrc,
-                       E.out_off.as<uint32_t>());
-    HIPCHECK(hipMemcpyAsync(E.out_dst.p, vals, ne * 4, hipMemcpyDeviceToDevice, st));
+    RC(E.out_dst.ensure(E.nedges * 4 + 8, st));
+    OutSeg seg = {E.off.as<uint32_t>(), E.src.as<uint32_t>(), E.out_off.as<uint32_t>(), E.out_dst.as<uint32_t>(),
+                  nullptr, 0, E.rows, nsrc, E.nedges};
+    out_edges_plan(&seg, 1);
+    RC(build_out_edges(&seg, nullptr, 1, s.scratch, st));
     RC(E.expo.ensure(((nsrc + 31) / 32) * 4 + 16, st));
     RC(E.expo_cnt.ensure(SIR_CTL_WORDS * 4 + 8, st));
     fill_u32(E.expo_cnt.as<uint32_t>(), 0u, SIR_CTL_WORDS, st);   // no complete counts yet

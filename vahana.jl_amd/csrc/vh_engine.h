@@ -207,9 +207,21 @@ struct ContactBits {
 // one apply! of the contact model incl. its births, deaths and contact CSR
 int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t step, uint64_t* ndeaths);
 // device G(n, p) CSR in target order (vh_ensemble.hip): off[n + 1], sources as
-// 1-based numbers; one host synchronisation
-int gnp_device(uint64_t n, double mean_deg, uint64_t seed, DevBuf& off, DevBuf& src, DevBuf& cdf,
-               Scratch& sc, hipStream_t st, uint64_t* nedges);
+// 1-based numbers; one host synchronisation (in gnp_degrees)
+int gnp_degrees(uint64_t n, double mean_deg, uint64_t seed, uint32_t* off, DevBuf& cdf, Scratch& sc,
+                hipStream_t st, uint64_t* nedges);
+int gnp_fill(uint64_t n, uint64_t seed, const uint32_t* off, uint32_t* src, hipStream_t st);
+// one in-edge CSR of an out-edge build (vh_ensemble.hip)
+struct OutSeg {
+    const uint32_t *off, *src;     // off[rows + 1], sources as 1-based numbers <= nsrc
+    uint32_t *out_off, *out_dst;   // nsrc + 1 offsets, ne target rows
+    uint32_t* bits;                // words cleared with it
+    uint64_t nwords, rows, nsrc, ne;
+    uint64_t edge0;                // (from here set by out_edges_plan) its place among the sorted edges
+    uint32_t key0, blk0, nblk;     // its first key, first block and number of blocks
+};
+uint32_t out_edges_plan(OutSeg* h, size_t nseg);
+int build_out_edges(const OutSeg* h, const OutSeg* d, size_t nseg, Scratch& sc, hipStream_t st);
 // CSR of a raster stencil (vh_bodies.hip): off[rows + 1] with the cell rows
 // at rowbase, sources as AgentIDs (src64) or numbers, uniform states
 int stencil_csr(Sim& s, EdgeStore& E, uint64_t rowbase, uint64_t rows);

@@ -82,28 +82,68 @@ __global__ void k_sir_init(uint32_t* st, uint64_t n, uint64_t seed, double frac,
     st[i] = vh_u01(vh_hash(seed, id, 0, VH_KEY_INIT)) < frac ? (uint32_t)VH_I : (uint32_t)VH_S;
 }
 
-// in-edge rows as transpose input: key = source index, value = row
-__global__ void k_member_edge_rows(const uint32_t* __restrict__ off, const uint32_t* __restrict__ src,
-                                   uint64_t n, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    for (uint32_t k = off[r]; k < off[r + 1]; k++) {
-        keys[k] = src[k] - 1u;
-        vals[k] = (uint32_t)r;
+// ---- out-edges of several in-edge CSRs at once
+// The transposes of all segments come from one radix sort: key = the segment's
+// first key + source, value = the row. A sort per segment is launches and tiny
+// scans (48 graphs of 10^3..10^6 agents: 22 launches and 3 allocations each,
+// 13 ms in the first step call and 5.3 ms of kernels; one sort per 2^23 edges:
+// 4.5 ms and 2.7 ms).
+__device__ __forceinline__ OutSeg out_seg(const OutSeg& one, const OutSeg* __restrict__ d, uint32_t nseg) {
+    if (!d) return one;
+    uint32_t lo = 0, hi = nseg - 1;   // the last segment with blk0 <= this block
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1) >> 1;
+        if (d[mid].blk0 <= blockIdx.x) lo = mid;
+        else hi = mid - 1;
+    }
+    return d[lo];
+}
+// 256 rows of a segment per block, a thread per edge: its row is searched in
+// the rows' offsets in LDS, and reads and writes are coalesced (a thread per
+// row that walks its edges wrote 64 lines at once: 10^6 rows of 10 edges 211
+// us, so 46)
+__global__ __launch_bounds__(256) void k_out_keys(OutSeg one, const OutSeg* __restrict__ d, uint32_t nseg,
+                                                  uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+    __shared__ uint32_t s_off[257];
+    const OutSeg g = out_seg(one, d, nseg);
+    const uint32_t tid = threadIdx.x;
+    const uint64_t r0 = (uint64_t)(blockIdx.x - g.blk0) * 256;
+    if (r0 >= g.rows) return;   // whole block
+    const uint32_t nr = g.rows - r0 < 256 ? (uint32_t)(g.rows - r0) : 256u;
+    if (tid < nr) s_off[tid] = g.off[r0 + tid];
+    if (tid == 0) s_off[nr] = g.off[r0 + nr];
+    __syncthreads();
+    const uint32_t e1 = s_off[nr];
+    for (uint64_t k = (uint64_t)s_off[0] + tid; k < e1; k += 256) {
+        uint32_t r = 0;   // the last row that starts at or before edge k
+#pragma unroll
+        for (uint32_t q = 128; q; q >>= 1)
+            if (r + q < nr && s_off[r + q] <= k) r += q;
+        keys[g.edge0 + k] = g.key0 + g.src[k] - 1u;
+        vals[g.edge0 + k] = (uint32_t)r0 + r;
     }
 }
-// out_off[v] = first index whose key >= v (keys sorted), v in [0, n]
-__global__ void k_member_offsets(const uint32_t* __restrict__ keys, uint64_t ne, uint64_t n,
-                                 uint32_t* __restrict__ out_off) {
-    uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v > n) return;
-    uint64_t lo = 0, hi = ne;
+// out_off[v] = first sorted edge whose key >= v, v in [0, nsrc]; a share of
+// the sorted rows copied to out_dst; the segment's bitmap words cleared
+__global__ __launch_bounds__(256) void k_out_place(OutSeg one, const OutSeg* __restrict__ d, uint32_t nseg,
+                                                   const uint32_t* __restrict__ keys,
+                                                   const uint32_t* __restrict__ vals) {
+    const OutSeg g = out_seg(one, d, nseg);
+    const uint64_t j = blockIdx.x - g.blk0, v = j * 256 + threadIdx.x;
+    keys += g.edge0;
+    vals += g.edge0;
+    if (v < g.nwords) g.bits[v] = 0u;
+    const uint64_t share = (g.ne + g.nblk - 1) / g.nblk;
+    const uint64_t c1 = (j + 1) * share < g.ne ? (j + 1) * share : g.ne;
+    for (uint64_t c = j * share + threadIdx.x; c < c1; c += 256) g.out_dst[c] = vals[c];
+    if (v > g.nsrc) return;
+    uint64_t lo = 0, hi = g.ne;
     while (lo < hi) {
-        uint64_t mid = (lo + hi) >> 1;
-        if ((uint64_t)keys[mid] < v) lo = mid + 1;
+        const uint64_t mid = (lo + hi) >> 1;
+        if ((uint64_t)keys[mid] < g.key0 + v) lo = mid + 1;
         else hi = mid;
     }
-    out_off[v] = (uint32_t)lo;
+    g.out_off[v] = (uint32_t)lo;
 }
 
 constexpr uint32_t ENS_TILE = 4096;   // agents of a logical block at most (1024 threads, four each)
@@ -373,28 +413,68 @@ namespace vh {
 // Directed G(n, p), p = mean_deg / (n - 1), as a CSR in target order: the
 // in-degree of target t is Binomial(n - 1, p) by inverse CDF, its sources are
 // distinct uniform draws != t in draw order (vh_graph_gnp is the host twin).
-// `cdf` and `sc` are working buffers; one host synchronisation (edge count).
-int gnp_device(uint64_t n, double mean_deg, uint64_t seed, DevBuf& off, DevBuf& src, DevBuf& cdf_buf,
-               Scratch& sc, hipStream_t st, uint64_t* nedges) {
+// gnp_degrees gives off[n + 1] (device) and, after a host synchronisation, the
+// number of edges, gnp_fill the sources; `cdf` and `sc` are working buffers.
+int gnp_degrees(uint64_t n, double mean_deg, uint64_t seed, uint32_t* off, DevBuf& cdf_buf, Scratch& sc,
+                hipStream_t st, uint64_t* nedges) {
     if (n == 0 || n >= 0xFFFFFFFFull) return set_error(VH_ERR_ARG, "G(n, p): bad n");
     double pe = n > 1 ? mean_deg / (double)(n - 1) : 0.0;
     std::vector<double> cdf = binom_cdf(n, pe);
     RC(cdf_buf.ensure(cdf.size() * 8, st));
-    RC(off.ensure((n + 1) * 4, st));
     uint32_t* deg = (uint32_t*)sc.take(n * 4 + 8);
     if (!deg) return set_error(VH_ERR_OOM, "scratch");
     HIPCHECK(hipMemcpyAsync(cdf_buf.p, cdf.data(), cdf.size() * 8, hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_gnp_degree, dim3(grid_for(n, 256)), dim3(256), 0, st, cdf_buf.as<double>(),
                        (uint32_t)cdf.size(), seed, n, deg);
-    if (scan_excl_u32(deg, off.as<uint32_t>(), n, sc, st)) return set_error(VH_ERR_DEVICE, "scan");
+    if (scan_excl_u32(deg, off, n, sc, st)) return set_error(VH_ERR_DEVICE, "scan");
     uint32_t ne = 0;
-    HIPCHECK(hipMemcpyAsync(&ne, off.as<uint32_t>() + n, 4, hipMemcpyDeviceToHost, st));
+    HIPCHECK(hipMemcpyAsync(&ne, off + n, 4, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipStreamSynchronize(st));   // also keeps `cdf` alive until the copy is done
-    RC(src.ensure((uint64_t)ne * 4 + 8, st));
-    hipLaunchKernelGGL(k_gnp_fill, dim3(grid_for(n, 256)), dim3(256), 0, st, n, seed, off.as<uint32_t>(),
-                       src.as<uint32_t>());
-    HIPCHECK(hipGetLastError());
     *nedges = ne;
+    return VH_OK;
+}
+int gnp_fill(uint64_t n, uint64_t seed, const uint32_t* off, uint32_t* src, hipStream_t st) {
+    hipLaunchKernelGGL(k_gnp_fill, dim3(grid_for(n, 256)), dim3(256), 0, st, n, seed, off, src);
+    HIPCHECK(hipGetLastError());
+    return VH_OK;
+}
+
+// Out-edges of `nseg` segments that share one sort (key0, edge0, blk0 and nblk
+// as out_edges_plan leaves them; `d`: their copy on the device, unused for one)
+uint32_t out_edges_plan(OutSeg* h, size_t nseg) {
+    uint64_t key = 0, edge = 0;
+    uint32_t blk = 0;
+    for (size_t i = 0; i < nseg; i++) {
+        h[i].key0 = (uint32_t)key;
+        h[i].edge0 = edge;
+        h[i].blk0 = blk;
+        h[i].nblk = (uint32_t)(std::max(std::max(h[i].rows, h[i].nsrc + 1), h[i].nwords) / 256 + 1);
+        key += h[i].nsrc;
+        edge += h[i].ne;
+        blk += h[i].nblk;
+    }
+    return blk;
+}
+int build_out_edges(const OutSeg* h, const OutSeg* d, size_t nseg, Scratch& sc, hipStream_t st) {
+    const OutSeg& z = h[nseg - 1];
+    const uint64_t ne = z.edge0 + z.ne, nkeys = z.key0 + z.nsrc;
+    const uint32_t blocks = z.blk0 + z.nblk;
+    uint32_t* keys = (uint32_t*)sc.take(ne * 4 + 4);
+    uint32_t* vals = (uint32_t*)sc.take(ne * 4 + 4);
+    uint32_t* ka = (uint32_t*)sc.take(ne * 4 + 4);
+    uint32_t* va = (uint32_t*)sc.take(ne * 4 + 4);
+    if (!keys || !vals || !ka || !va) return set_error(VH_ERR_OOM, "scratch");
+    if (nseg == 1) d = nullptr;
+    if (ne) {
+        hipLaunchKernelGGL(k_out_keys, dim3(blocks), dim3(256), 0, st, h[0], d, (uint32_t)nseg, keys, vals);
+        uint32_t bits = 1;
+        while (bits < 32 && (nkeys >> bits) != 0) bits++;
+        if (radix_sort_pairs(&keys, &vals, ka, va, ne, bits, false, sc, st))
+            return set_error(VH_ERR_DEVICE, "radix sort failed");
+    }
+    hipLaunchKernelGGL(k_out_place, dim3(blocks), dim3(256), 0, st, h[0], d, (uint32_t)nseg,
+                       (const uint32_t*)keys, (const uint32_t*)vals);
+    HIPCHECK(hipGetLastError());
     return VH_OK;
 }
 // w[k] = (2 (h >> 41) + 1) 2^-24, h = vh_hash(wseed, k, 0, VH_KEY_WEIGHT): the
@@ -420,15 +500,28 @@ struct Member {
     uint64_t seed;
     double p;
     uint32_t rec;
-    DevBuf off, src, st[2];
-    DevBuf out_off, out_dst, bits;   // out-edges and the two exposure bitmaps
+    // one allocation for all of a member's device memory (a buffer each was
+    // seven allocations and frees, 17 and 58 us each): states, in-edge CSR and,
+    // unless the exposure pass is off, out-edges and the two exposure bitmaps
+    DevBuf buf;
+    DevBuf out_buf;                  // out-edges and bitmaps when `buf` was taken without them
+    uint32_t *off = nullptr, *src = nullptr, *st[2] = {nullptr, nullptr};
+    uint32_t *out_off = nullptr, *out_dst = nullptr, *bits = nullptr;
+    uint64_t bytes = 0;              // of states and in-edges
     uint64_t nw = 0;                 // words per bitmap
     bool out_ready = false;          // built (on the first step with the exposure pass)
     int cur = 0;
     std::shared_ptr<StepDone> done;   // the last launch that wrote this member
+    size_t out_bytes() const { return pad(n * 4 + 4) + pad(nedges * 4) + pad(2 * nw * 4); }
+    void out_place(uint8_t* p) {
+        out_off = (uint32_t*)p;
+        out_dst = (uint32_t*)(p + pad(n * 4 + 4));
+        bits = (uint32_t*)(p + pad(n * 4 + 4) + pad(nedges * 4));
+    }
+    static size_t pad(size_t b) { return (b + 8 + 255) & ~(size_t)255; }
     void release() {
-        off.release(); src.release(); st[0].release(); st[1].release();
-        out_off.release(); out_dst.release(); bits.release();
+        buf.release();
+        out_buf.release();
     }
 };
 
@@ -456,6 +549,9 @@ struct vh_ensemble {
     DevBuf d_desc, d_bmember, d_bstart;
     DevBuf d_mblk, d_blkcnt, d_dec;   // exposure: member block ranges, per-block counts, decisions
     Scratch oscr;                     // scratch of the members' out-edge builds (step stream)
+    DevBuf d_segs;                    // the segments of the builds of one step call
+    void* h_segs = nullptr;           // and their pinned staging
+    size_t h_segs_cap = 0;
     uint64_t launches = 0;            // step launches so far (bitmap parity)
     bool expose_last = false;         // the exposure pass ran in the last step call
     std::vector<MemberDesc> h_desc;
@@ -540,19 +636,19 @@ static int upload_desc(vh_ensemble* e) {
     for (auto& kv : e->members) {
         Member* m = kv.second;
         MemberDesc d;
-        d.off = m->off.as<uint32_t>();
-        d.src = m->src.as<uint32_t>();
-        d.rs = m->st[m->cur].as<uint32_t>();
-        d.ws = m->st[m->cur ^ 1].as<uint32_t>();
+        d.off = m->off;
+        d.src = m->src;
+        d.rs = m->st[m->cur];
+        d.ws = m->st[m->cur ^ 1];
         d.n = m->n;
         d.step = m->step;
         d.seed = m->seed;
         d.p = m->p;
         d.rec = m->rec;
         d.type = 1;
-        d.out_off = m->out_off.as<uint32_t>();
-        d.out_dst = m->out_dst.as<uint32_t>();
-        d.bits = m->bits.as<uint32_t>();
+        d.out_off = m->out_off;
+        d.out_dst = m->out_dst;
+        d.bits = m->bits;
         d.nw = m->nw;
         d.tile = member_tile(e, m->n);
         d.pad = 0;
@@ -587,11 +683,12 @@ extern "C" int vh_ensemble_destroy(vh_ensemble_t e) {
         delete m;
     }
     e->d_desc.release(); e->d_bmember.release(); e->d_bstart.release(); e->d_cdf.release();
-    e->d_mblk.release(); e->d_blkcnt.release(); e->d_dec.release();
+    e->d_mblk.release(); e->d_blkcnt.release(); e->d_dec.release(); e->d_segs.release();
     e->scratch.release();
     e->oscr.release();
     if (e->h_table) (void)hipHostFree(e->h_table);
     if (e->h_descs) (void)hipHostFree(e->h_descs);
+    if (e->h_segs) (void)hipHostFree(e->h_segs);
     if (e->own_streams) {
         (void)hipStreamDestroy(e->aux);
         (void)hipStreamDestroy(e->stream);
@@ -600,33 +697,49 @@ extern "C" int vh_ensemble_destroy(vh_ensemble_t e) {
     return VH_OK;
 }
 
-// the member's out-edges (the transpose of its in-edge CSR, by a stable radix
-// sort on the source) and its two exposure bitmaps, cleared
-static int member_out_edges(Member* m, uint64_t ne, Scratch& sc, hipStream_t st) {
-    const uint64_t n = m->n;
-    uint32_t* keys = (uint32_t*)sc.take(ne * 4 + 4);
-    uint32_t* vals = (uint32_t*)sc.take(ne * 4 + 4);
-    uint32_t* ka = (uint32_t*)sc.take(ne * 4 + 4);
-    uint32_t* va = (uint32_t*)sc.take(ne * 4 + 4);
-    if (!keys || !vals || !ka || !va) return set_error(VH_ERR_OOM, "scratch");
-    RC(m->out_off.ensure((n + 1) * 4 + 8, st));
-    RC(m->out_dst.ensure(ne * 4 + 8, st));
-    m->nw = (n + 31) / 32;
-    RC(m->bits.ensure(2 * m->nw * 4 + 8, st));
-    fill_u32(m->bits.as<uint32_t>(), 0u, 2 * m->nw, st);
-    if (ne) {
-        hipLaunchKernelGGL(k_member_edge_rows, dim3(grid_for(n, 256)), dim3(256), 0, st, m->off.as<uint32_t>(),
-                           m->src.as<uint32_t>(), n, keys, vals);
-        uint32_t bits = 1;
-        while (bits < 32 && (n >> bits) != 0) bits++;
-        if (radix_sort_pairs(&keys, &vals, ka, va, ne, bits, false, sc, st))
-            return set_error(VH_ERR_DEVICE, "radix sort failed");
-        HIPCHECK(hipMemcpyAsync(m->out_dst.p, vals, ne * 4, hipMemcpyDeviceToDevice, st));
+// The out-edges (the transposes of the in-edge CSRs) of the members that have
+// none yet, and their exposure bitmaps, cleared: on the step stream, idle here.
+// Members share a sort up to OUT_BATCH edges, which fills the chip; 2^25 takes
+// as long (48 members: 2.7 ms of kernels) and four times the 150 MB of scratch.
+constexpr uint64_t OUT_BATCH = 1ull << 23;
+static int build_members_out(vh_ensemble* e) {
+    std::vector<OutSeg> segs;
+    std::vector<Member*> ms;
+    std::vector<size_t> first;   // first segment of each batch
+    uint64_t ne = 0, nkeys = 0, most = 0;
+    for (auto& kv : e->members) {
+        Member* m = kv.second;
+        if (m->out_ready) continue;
+        if (!m->out_off) {
+            RC(m->out_buf.ensure(m->out_bytes(), e->stream));
+            m->out_place(m->out_buf.as<uint8_t>());
+        }
+        if (segs.empty() || ne + m->nedges > OUT_BATCH || nkeys + m->n > 0x7FFFFFFFull) {
+            first.push_back(segs.size());
+            ne = nkeys = 0;
+        }
+        ne += m->nedges;
+        nkeys += m->n;
+        most = std::max(most, ne);
+        segs.push_back({m->off, m->src, m->out_off, m->out_dst, m->bits, 2 * m->nw, m->n, m->n, m->nedges});
+        ms.push_back(m);
     }
-    hipLaunchKernelGGL(k_member_offsets, dim3(grid_for(n + 1, 256)), dim3(256), 0, st, keys, ne, n,
-                       m->out_off.as<uint32_t>());
-    HIPCHECK(hipGetLastError());
-    m->out_ready = true;
+    if (segs.empty()) return VH_OK;
+    first.push_back(segs.size());
+    for (size_t b = 0; b + 1 < first.size(); b++) out_edges_plan(&segs[first[b]], first[b + 1] - first[b]);
+    const size_t bytes = segs.size() * sizeof(OutSeg);
+    RC(pinned(&e->h_segs, &e->h_segs_cap, bytes));
+    memcpy(e->h_segs, segs.data(), bytes);
+    RC(e->d_segs.ensure(bytes, e->stream));
+    HIPCHECK(hipMemcpyAsync(e->d_segs.p, e->h_segs, bytes, hipMemcpyHostToDevice, e->stream));
+    for (size_t b = 0; b + 1 < first.size(); b++) {
+        e->oscr.reset(e->stream);   // (waits for the previous build when it spilled)
+        // four buffers of the pairs, the tiles' digit counts and their scans
+        if (e->oscr.reserve(most * 18 + (4u << 20), e->stream)) return set_error(VH_ERR_OOM, "scratch");
+        RC(build_out_edges(&segs[first[b]], e->d_segs.as<OutSeg>() + first[b], first[b + 1] - first[b], e->oscr,
+                           e->stream));
+    }
+    for (Member* m : ms) m->out_ready = true;
     return VH_OK;
 }
 
@@ -642,15 +755,30 @@ extern "C" int vh_ensemble_add_sir(vh_ensemble_t e, const vh_sir_member* sm, uin
     m->rec = sm->recovery;
     m->step = 1;
     hipStream_t st = e->aux;   // builds run beside the step launches
-    int rc = m->st[0].ensure(sm->n * 4, st);
-    if (!rc) rc = m->st[1].ensure(sm->n * 4, st);
     uint64_t ne = 0;
     e->scratch.reset(st);
-    if (!rc) rc = gnp_device(sm->n, sm->mean_deg, sm->graph_seed, m->off, m->src, e->d_cdf, e->scratch, st, &ne);
-    if (rc) { m->release(); delete m; return rc; }
+    uint32_t* off = (uint32_t*)e->scratch.take(sm->n * 4 + 8);   // until the number of edges is known
+    int rc = off ? gnp_degrees(sm->n, sm->mean_deg, sm->graph_seed, off, e->d_cdf, e->scratch, st, &ne)
+                 : set_error(VH_ERR_OOM, "scratch");
     m->nedges = ne;
+    m->nw = (m->n + 31) / 32;
+    const size_t sb = Member::pad(sm->n * 4), ob = Member::pad(sm->n * 4 + 4);
+    m->bytes = 2 * sb + ob + Member::pad(ne * 4);
+    const bool out = g_opts.sir_expose != 0;
+    if (!rc) rc = m->buf.ensure(m->bytes + (out ? m->out_bytes() : 0), st);
+    if (!rc) {
+        uint8_t* p = m->buf.as<uint8_t>();
+        m->st[0] = (uint32_t*)p;
+        m->st[1] = (uint32_t*)(p + sb);
+        m->off = (uint32_t*)(p + 2 * sb);
+        m->src = (uint32_t*)(p + 2 * sb + ob);
+        if (out) m->out_place(p + m->bytes);
+        rc = gnp_fill(sm->n, sm->graph_seed, off, m->src, st);
+    }
+    if (rc) { m->release(); delete m; return rc; }
+    HIPCHECK(hipMemcpyAsync(m->off, off, (sm->n + 1) * 4, hipMemcpyDeviceToDevice, st));
     double frac = (double)sm->n_init / (double)sm->n;
-    hipLaunchKernelGGL(k_sir_init, dim3(grid_for(sm->n, 256)), dim3(256), 0, st, m->st[0].as<uint32_t>(),
+    hipLaunchKernelGGL(k_sir_init, dim3(grid_for(sm->n, 256)), dim3(256), 0, st, m->st[0],
                        sm->n, sm->seed, frac, 1u);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(st));
@@ -721,12 +849,7 @@ extern "C" int vh_ensemble_step(vh_ensemble_t e, uint32_t steps, int use_graph) 
     for (auto& kv : e->members) total += kv.second->n;
     const bool expose = g_opts.sir_expose != 0 && (int64_t)total >= g_opts.sir_expose_min;
     if (expose) {
-        for (auto& kv : e->members) {
-            Member* m = kv.second;
-            if (m->out_ready) continue;
-            e->oscr.reset(e->stream);   // (waits for the previous build when it spilled)
-            RC(member_out_edges(m, m->nedges, e->oscr, e->stream));
-        }
+        RC(build_members_out(e));
         // the bitmaps were not kept while the pass was off: every member's
         // next exposure launch is a full one
         if (!e->expose_last) fill_u32(e->d_dec.as<uint32_t>(), 0u, nm, e->stream);
@@ -845,7 +968,7 @@ extern "C" int vh_ensemble_read(vh_ensemble_t e, uint32_t id, void* states, uint
     // only the launches that wrote this member must be complete: a member
     // past its horizon is read while later steps of the others run
     if (m->done) HIPCHECK(hipEventSynchronize(m->done->ev));
-    HIPCHECK(hipMemcpyAsync(states, m->st[m->cur].p, m->n * 4, hipMemcpyDeviceToHost, e->aux));
+    HIPCHECK(hipMemcpyAsync(states, m->st[m->cur], m->n * 4, hipMemcpyDeviceToHost, e->aux));
     HIPCHECK(hipStreamSynchronize(e->aux));
     return VH_OK;
 }
@@ -857,7 +980,7 @@ extern "C" int vh_ensemble_info(vh_ensemble_t e, uint64_t* members, uint64_t* ag
         Member* m = kv.second;
         a += m->n;
         ed += m->nedges;
-        by += m->off.cap + m->src.cap + m->st[0].cap + m->st[1].cap;
+        by += m->bytes;
     }
     *members = e->members.size();
     *agents = a;
@@ -890,7 +1013,7 @@ extern "C" int vh_ensemble_autotune(vh_ensemble_t e, uint32_t trial_steps, uint3
     for (auto& kv : e->members) {
         Member* m = kv.second;
         RC(snap[k].ensure(m->n * 4 + 4, e->stream));
-        HIPCHECK(hipMemcpyAsync(snap[k].p, m->st[m->cur].p, m->n * 4, hipMemcpyDeviceToDevice, e->stream));
+        HIPCHECK(hipMemcpyAsync(snap[k].p, m->st[m->cur], m->n * 4, hipMemcpyDeviceToDevice, e->stream));
         saved.push_back({m->cur, m->step});
         present[size_class(m->n)] = true;
         k++;
@@ -945,7 +1068,7 @@ extern "C" int vh_ensemble_autotune(vh_ensemble_t e, uint32_t trial_steps, uint3
         Member* m = kv.second;
         m->cur = saved[k].first;
         m->step = saved[k].second;
-        HIPCHECK(hipMemcpyAsync(m->st[m->cur].p, snap[k].p, m->n * 4, hipMemcpyDeviceToDevice, e->stream));
+        HIPCHECK(hipMemcpyAsync(m->st[m->cur], snap[k].p, m->n * 4, hipMemcpyDeviceToDevice, e->stream));
         k++;
     }
     HIPCHECK(hipStreamSynchronize(e->stream));
