@@ -283,3 +283,22 @@ def test_ensemble_out_edges_together(vh, ora, gpu_ready, opts, late):
             vh.models.step_sir(ora, m, p_inf=0.2, seed=70 + k, recovery=7)
         got, want = E.read(mid)[0], m.sim._read_agents(m.T)[0]
         assert np.array_equal(np.ascontiguousarray(got).view(np.uint8), np.ascontiguousarray(want).view(np.uint8)), n
+
+
+# one target; around 256 targets; a block of several passes (256 x 40 > 4096
+# edges); most agents a source, so that every list draws again; degrees of
+# thousands
+@pytest.mark.parametrize("n,deg", [(1, 0.0), (2, 1.0), (255, 16.0), (256, 17.5), (257, 100.0), (1000, 40.0), (40, 30.0),
+                                   (2500, 2000.0), (100_001, 8.0)])
+def test_gnp_sources(vh, gpu_ready, n, deg):
+    """The device's G(n, p) against the host twin."""
+    A, E = vh.struct("A", [("x", "u1")]), vh.struct("E", [])
+    sim = vh.create_simulation(vh.ModelTypes() | vh.register_agenttype_(A, "Immortal")
+                               | vh.register_edgetype_(E, "Stateless", target=A) | vh.create_model("gnp"))
+    sim._add_agents_array(A, np.zeros(n, dtype=A.dtype))
+    sim._add_edges_gnp(E, deg, 11)
+    vh.finish_init_(sim)
+    t, f, _ = sim._read_edges(E)
+    fr, to = vh.inputs.graph_gnp(n, deg, 11)
+    tid = np.uint64(1) << np.uint64(56)
+    assert np.array_equal(t, tid | to.astype(np.uint64)) and np.array_equal(f, tid | fr.astype(np.uint64))

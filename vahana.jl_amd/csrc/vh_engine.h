@@ -210,7 +210,7 @@ int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t st
 // 1-based numbers; one host synchronisation (in gnp_degrees)
 int gnp_degrees(uint64_t n, double mean_deg, uint64_t seed, uint32_t* off, DevBuf& cdf, Scratch& sc,
                 hipStream_t st, uint64_t* nedges);
-int gnp_fill(uint64_t n, uint64_t seed, const uint32_t* off, uint32_t* src, hipStream_t st);
+int gnp_fill(uint64_t n, uint64_t seed, const uint32_t* off, uint32_t* src, uint32_t* off_out, hipStream_t st);
 // one in-edge CSR of an out-edge build (vh_ensemble.hip)
 struct OutSeg {
     const uint32_t *off, *src;     // off[rows + 1], sources as 1-based numbers <= nsrc

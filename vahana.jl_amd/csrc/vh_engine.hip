@@ -1046,7 +1046,7 @@ static int build_gnp_csr(Sim& s, EdgeStore& E) {
         RC(E.off.ensure((rows + 1) * 4, st));
         int rc = gnp_degrees(rows, E.gen_mean_deg, E.gen_seed, E.off.as<uint32_t>(), cdf, s.scratch, st, &ne);
         if (!rc) rc = E.src.ensure(ne * 4 + 8, st);
-        if (!rc) rc = gnp_fill(rows, E.gen_seed, E.off.as<uint32_t>(), E.src.as<uint32_t>(), st);
+        if (!rc) rc = gnp_fill(rows, E.gen_seed, E.off.as<uint32_t>(), E.src.as<uint32_t>(), nullptr, st);
         if (!rc && E.bytes) {
             rc = E.st.ensure(ne * 4 + 8, st);
             if (!rc) fill_weights(E.st.as<float>(), ne, E.gen_wseed, st);

@@ -51,8 +51,7 @@ __host__ __device__ inline uint32_t gnp_degree(const double* cdf, uint32_t ncdf,
     return d;
 }
 // the d distinct sources of target t (1-based), in draw order
-__host__ __device__ inline void gnp_sources(uint64_t n, uint64_t seed, uint64_t t, uint32_t d,
-                                            uint32_t* out) {
+inline void gnp_sources(uint64_t n, uint64_t seed, uint64_t t, uint32_t d, uint32_t* out) {
     uint64_t draw = 0;
     for (uint32_t j = 0; j < d;) {
         uint64_t h = vh_hash(seed, t, ++draw, KEY_SRC);
@@ -70,9 +69,91 @@ __global__ void k_gnp_degree(const double* cdf, uint32_t ncdf, uint64_t seed, ui
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) deg[i] = gnp_degree(cdf, ncdf, seed, i + 1);
 }
-__global__ void k_gnp_fill(uint64_t n, uint64_t seed, const uint32_t* off, uint32_t* src) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) gnp_sources(n, seed, i + 1, off[i + 1] - off[i], src + off[i]);
+// The sources of GNP_ROWS targets per block (and off copied to off_out unless
+// null), a thread per edge: edge j of a target takes draw j + 1, which is the
+// result unless a source comes twice. Equal sources set the same bit of a
+// table in LDS (bit x + 1024 row mod 2^16): an edge that finds its bit set is
+// listed and compared with its target's list, and a target with a source twice
+// (or every target, if the list overflows) draws again, a wave at a time.
+// (A thread per target that compared each draw with its list in global memory
+// was a chain of those reads: 48 graphs of 10^3..10^6 targets, degree 4..16, 67
+// us each, so 22, or 44 if a thread redraws a target; 128 targets per block: 26.)
+constexpr uint32_t GNP_ROWS = 64;
+__device__ __forceinline__ uint32_t gnp_draw(uint64_t n, uint64_t pre, uint64_t t, uint64_t draw) {
+    const uint64_t h = vh_hash_fin(vh_mix64(pre + draw + VH_GOLDEN), KEY_SRC);
+    const uint64_t x = 1 + (((h >> 32) * (n - 1)) >> 32);
+    return (uint32_t)(x + (x >= t ? 1 : 0));
+}
+// gnp_sources by a wave, 64 draws at a time: a draw counts unless it is in the
+// list already or an earlier lane has the same source
+__device__ void gnp_redraw(uint64_t n, uint64_t pre, uint64_t t, uint32_t d, uint32_t* out) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t have = 0;
+    for (uint64_t draw = 1; have < d; draw += 64) {
+        const uint32_t x = gnp_draw(n, pre, t, draw + lane);
+        bool dup = false;
+        for (uint32_t q = 0; q < have; q++) dup |= out[q] == x;
+        for (uint32_t q = 0; q < 63; q++)
+            dup |= q < lane && (uint32_t)__builtin_amdgcn_readlane((int)x, (int)q) == x;
+        const uint64_t m = __ballot(!dup);
+        const uint32_t at = have + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+        if (!dup && at < d) out[at] = x;
+        have += (uint32_t)__popcll(m);
+        __threadfence_block();   // the list, before other lanes read it
+    }
+}
+constexpr uint32_t GNP_LIST = 1024;
+__global__ __launch_bounds__(256) void k_gnp_fill(uint64_t n, uint64_t seed, const uint32_t* __restrict__ off,
+                                                  uint32_t* src, uint32_t* __restrict__ off_out) {
+    __shared__ uint64_t s_pre[GNP_ROWS];
+    __shared__ uint32_t s_off[GNP_ROWS + 1], s_bit[2048], s_list[GNP_LIST], s_n, s_dup[GNP_ROWS / 32];
+    const uint32_t tid = threadIdx.x;
+    const uint64_t r0 = (uint64_t)blockIdx.x * GNP_ROWS;
+    const uint32_t nr = n - r0 < GNP_ROWS ? (uint32_t)(n - r0) : GNP_ROWS;
+    if (tid < nr) {
+        s_off[tid] = off[r0 + tid];
+        // the stages of vh_hash before the draw's number
+        s_pre[tid] = vh_mix64(vh_mix64(seed + VH_GOLDEN) + r0 + tid + 1 + VH_GOLDEN);
+    }
+    if (tid == 0) {
+        s_off[nr] = off[r0 + nr];
+        s_n = 0;
+    }
+    if (tid < GNP_ROWS / 32) s_dup[tid] = 0;
+    for (uint32_t q = tid; q < 2048; q += 256) s_bit[q] = 0;
+    __syncthreads();
+    if (off_out) {
+        if (tid < nr) off_out[r0 + tid] = s_off[tid];
+        if (tid == 0 && r0 + nr == n) off_out[n] = s_off[nr];
+    }
+    const uint32_t e0 = s_off[0], cnt = s_off[nr] - e0;   // (degrees end below 4096)
+    for (uint32_t k = tid; k < cnt; k += 256) {
+        uint32_t r = 0;   // the last target that starts at or before edge k
+#pragma unroll
+        for (uint32_t q = GNP_ROWS / 2; q; q >>= 1)
+            if (r + q < nr && s_off[r + q] - e0 <= k) r += q;
+        const uint32_t x = gnp_draw(n, s_pre[r], r0 + r + 1, k + e0 - s_off[r] + 1);
+        src[e0 + k] = x;
+        const uint32_t bit = (x + 1024u * r) & 0xFFFFu;
+        if ((atomicOr(&s_bit[bit >> 5], 1u << (bit & 31u)) >> (bit & 31u)) & 1u) {
+            const uint32_t l = atomicAdd(&s_n, 1u);
+            if (l < GNP_LIST) s_list[l] = k << 8 | r;
+        }
+    }
+    __syncthreads();
+    if (s_n == 0) return;   // whole block
+    if (s_n <= GNP_LIST) {
+        for (uint32_t l = tid; l < s_n; l += 256) {
+            const uint32_t k = e0 + (s_list[l] >> 8), r = s_list[l] & 0xFFu, x = src[k];
+            bool dup = false;
+            for (uint32_t q = s_off[r]; q < s_off[r + 1]; q++) dup |= src[q] == x && q != k;
+            if (dup) atomicOr(&s_dup[r >> 5], 1u << (r & 31u));
+        }
+        __syncthreads();
+    }
+    for (uint32_t r = tid >> 6; r < nr; r += 4)   // uniform per wave
+        if (s_n > GNP_LIST || ((s_dup[r >> 5] >> (r & 31u)) & 1u))
+            gnp_redraw(n, s_pre[r], r0 + r + 1, s_off[r + 1] - s_off[r], src + s_off[r]);
 }
 // initial state: I with probability n_init / n (hash keyed like the solo input)
 __global__ void k_sir_init(uint32_t* st, uint64_t n, uint64_t seed, double frac, uint32_t type) {
@@ -414,7 +495,7 @@ namespace vh {
 // in-degree of target t is Binomial(n - 1, p) by inverse CDF, its sources are
 // distinct uniform draws != t in draw order (vh_graph_gnp is the host twin).
 // gnp_degrees gives off[n + 1] (device) and, after a host synchronisation, the
-// number of edges, gnp_fill the sources; `cdf` and `sc` are working buffers.
+// number of edges, gnp_fill the sources (and a copy of off in off_out, unless null); `cdf` and `sc` are working buffers.
 int gnp_degrees(uint64_t n, double mean_deg, uint64_t seed, uint32_t* off, DevBuf& cdf_buf, Scratch& sc,
                 hipStream_t st, uint64_t* nedges) {
     if (n == 0 || n >= 0xFFFFFFFFull) return set_error(VH_ERR_ARG, "G(n, p): bad n");
@@ -433,8 +514,8 @@ int gnp_degrees(uint64_t n, double mean_deg, uint64_t seed, uint32_t* off, DevBu
     *nedges = ne;
     return VH_OK;
 }
-int gnp_fill(uint64_t n, uint64_t seed, const uint32_t* off, uint32_t* src, hipStream_t st) {
-    hipLaunchKernelGGL(k_gnp_fill, dim3(grid_for(n, 256)), dim3(256), 0, st, n, seed, off, src);
+int gnp_fill(uint64_t n, uint64_t seed, const uint32_t* off, uint32_t* src, uint32_t* off_out, hipStream_t st) {
+    hipLaunchKernelGGL(k_gnp_fill, dim3(grid_for(n, GNP_ROWS)), dim3(256), 0, st, n, seed, off, src, off_out);
     HIPCHECK(hipGetLastError());
     return VH_OK;
 }
@@ -773,10 +854,9 @@ extern "C" int vh_ensemble_add_sir(vh_ensemble_t e, const vh_sir_member* sm, uin
         m->off = (uint32_t*)(p + 2 * sb);
         m->src = (uint32_t*)(p + 2 * sb + ob);
         if (out) m->out_place(p + m->bytes);
-        rc = gnp_fill(sm->n, sm->graph_seed, off, m->src, st);
+        rc = gnp_fill(sm->n, sm->graph_seed, off, m->src, m->off, st);
     }
     if (rc) { m->release(); delete m; return rc; }
-    HIPCHECK(hipMemcpyAsync(m->off, off, (sm->n + 1) * 4, hipMemcpyDeviceToDevice, st));
     double frac = (double)sm->n_init / (double)sm->n;
     hipLaunchKernelGGL(k_sir_init, dim3(grid_for(sm->n, 256)), dim3(256), 0, st, m->st[0],
                        sm->n, sm->seed, frac, 1u);
