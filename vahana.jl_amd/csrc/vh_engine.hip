@@ -450,20 +450,27 @@ struct RowLayout {
     uint64_t nrows[VH_MAXA + 1];
 };
 
-// keys of log entries in the new row layout
+// row of a target in the layout; 0 and *bad for an id that is none of it
+__device__ __forceinline__ uint32_t log_key(uint64_t id, const RowLayout& L, bool* bad) {
+    const uint32_t t = vh_type_of(id);
+    const uint64_t nr = vh_nr_of(id);
+    *bad = t == 0 || t > VH_MAXA || nr == 0 || nr > L.nrows[t];
+    return *bad ? 0u : (uint32_t)(L.base[t] + nr - 1);
+}
+// keys of log entries in the new row layout; *unsorted is set when one is
+// below the one before it (null: not asked)
 __global__ void k_log_keys(const uint64_t* __restrict__ to, uint64_t n, RowLayout L,
-                           uint32_t* __restrict__ keys, uint32_t* err) {
+                           uint32_t* __restrict__ keys, uint32_t* err, uint32_t* unsorted) {
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    uint64_t id = to[i];
-    uint32_t t = vh_type_of(id);
-    uint64_t nr = vh_nr_of(id);
-    if (t == 0 || t > VH_MAXA || nr == 0 || nr > L.nrows[t]) {
-        atomicOr(err, VH_DERR_TARGET);
-        keys[i] = 0;
-        return;
-    }
-    keys[i] = (uint32_t)(L.base[t] + nr - 1);
+    bool bad, bad0 = false;
+    const uint32_t key = log_key(to[i], L, &bad);
+    if (bad) atomicOr(err, VH_DERR_TARGET);
+    keys[i] = key;
+    if (!unsorted) return;
+    const bool below = i && key < log_key(to[i - 1], L, &bad0);
+    const uint64_t m = __ballot(below);
+    if (m && (threadIdx.x & 63u) == (uint32_t)__builtin_ctzll(m)) *unsorted = 1u;
 }
 
 // removal entries of the log (remove_edges!): not edges (key past every
@@ -600,9 +607,50 @@ __global__ void k_remap_offsets(const uint32_t* __restrict__ off, const uint32_t
     uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r <= rows) offo[r] = pos[off[r]];
 }
-__global__ void k_u64_to_nr(const uint64_t* __restrict__ in, uint32_t* __restrict__ out, uint64_t n) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = (uint32_t)vh_nr_of(in[i]);
+// entries in sorted order (idx null: as they are): sources as ids or numbers
+// (srcw 8 or 4; 0: none), states of `words` W. Random reads of a line per
+// source and state: four entries per thread, all their reads in flight (1.6
+// 10^6 entries with 8-byte states: 67 us; a gather each, a conversion and
+// copies into the store: 125)
+template <class W>
+__global__ __launch_bounds__(256) void k_place(const uint32_t* __restrict__ idx, uint64_t n,
+                                               const uint64_t* __restrict__ from, void* __restrict__ srco,
+                                               uint32_t srcw, const W* __restrict__ st, W* __restrict__ sto,
+                                               uint32_t words) {
+    const uint64_t i0 = (uint64_t)blockIdx.x * 1024 + threadIdx.x;
+    uint64_t j[4], f[4];
+    W v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint64_t i = i0 + 256 * u;
+        j[u] = i < n ? (idx ? idx[i] : i) : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {   // (n > 0: entry 0 is there)
+        f[u] = srcw ? from[j[u]] : 0;
+        v[u] = words ? st[j[u] * words] : (W)0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint64_t i = i0 + 256 * u;
+        if (i >= n) continue;
+        if (srcw == 8) ((uint64_t*)srco)[i] = f[u];
+        else if (srcw == 4) ((uint32_t*)srco)[i] = (uint32_t)vh_nr_of(f[u]);
+        if (words) sto[i * words] = v[u];
+        for (uint32_t w = 1; w < words; w++) sto[i * words + w] = st[j[u] * words + w];
+    }
+}
+static void place_entries(const uint32_t* idx, uint64_t n, const uint64_t* from, void* srco, uint32_t srcw,
+                          const void* sts, void* sto, uint32_t bytes, hipStream_t st) {
+    if (!n || (!srcw && !bytes)) return;
+    const dim3 g(grid_for(n, 1024)), b(256);
+#define VH_PLACE(W) hipLaunchKernelGGL(k_place<W>, g, b, 0, st, idx, n, from, srco, srcw, (const W*)sts, (W*)sto, \
+                                       bytes / (uint32_t)sizeof(W))
+    if (bytes % 8 == 0) VH_PLACE(uint64_t);
+    else if (bytes % 4 == 0) VH_PLACE(uint32_t);
+    else if (bytes % 2 == 0) VH_PLACE(uint16_t);
+    else VH_PLACE(uint8_t);
+#undef VH_PLACE
 }
 __global__ void k_u8_to_u32(const uint8_t* __restrict__ in, uint32_t* __restrict__ out, uint64_t n) {
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -684,23 +732,28 @@ static int build_csr(Sim& s, EdgeStore& E, bool keep_base, const uint64_t* d_to,
     uint32_t* vals = (uint32_t*)sc.take(n * 4 + 4);
     uint32_t* kalt = (uint32_t*)sc.take(n * 4 + 4);
     uint32_t* valt = (uint32_t*)sc.take(n * 4 + 4);
-    uint64_t* from = ignorefrom ? nullptr : (uint64_t*)sc.take(n * 8 + 8);
-    uint8_t* sts = bytes ? (uint8_t*)sc.take(n * bytes + 8) : nullptr;
-    uint32_t* flag = (uint32_t*)sc.take(4);
-    if (!keys || !vals || !kalt || !valt || (!ignorefrom && !from) || (bytes && !sts) || !flag)
+    // the entries: the log itself, or the kept edges with the log behind them
+    uint64_t* from2 = !nbase || ignorefrom ? nullptr : (uint64_t*)sc.take(n * 8 + 8);
+    uint8_t* sts2 = nbase && bytes ? (uint8_t*)sc.take(n * bytes + 8) : nullptr;
+    if (!keys || !vals || !kalt || !valt || (nbase && !ignorefrom && !from2) || (nbase && bytes && !sts2))
         return set_error(VH_ERR_OOM, "scratch allocation failed");
+    const uint64_t* from = ignorefrom ? nullptr : nbase ? from2 : d_from;
+    const uint8_t* sts = nbase ? sts2 : d_st;
     uint32_t* err = s.d_err.as<uint32_t>();
     s.err_written = true;
     if (nbase)
         hipLaunchKernelGGL(k_base_expand, dim3(grid_for(E.rows, 256)), dim3(256), 0, st,
                            E.off.as<uint32_t>(), E.src.p, (uint32_t)E.src64, E.src_type,
-                           E.st.as<uint8_t>(), bytes, oldL, newL, E.rows, keys, from, sts, err);
+                           E.st.as<uint8_t>(), bytes, oldL, newL, E.rows, keys, from2, sts2, err);
     uint32_t* ekeys = nullptr;   // removal events (remove_edges!)
     uint32_t* eidx = nullptr;
     uint32_t* seq = nullptr;
+    uint32_t* unsorted = (uint32_t*)s.d_stats.p;
     if (nlog) {
+        const bool ask_all = nbase || d_kind;   // of all keys, once they are there
+        fill_u32(unsorted, 0, 1, st);
         hipLaunchKernelGGL(k_log_keys, dim3(grid_for(nlog, 256)), dim3(256), 0, st, d_to, nlog, newL,
-                           keys + nbase, err);
+                           keys + nbase, err, ask_all ? nullptr : unsorted);
         if (d_kind) {
             ekeys = (uint32_t*)sc.take(nlog * 4 + 4);
             eidx = (uint32_t*)sc.take(nlog * 4 + 4);
@@ -714,48 +767,53 @@ static int build_csr(Sim& s, EdgeStore& E, bool keep_base, const uint64_t* d_to,
                 return set_error(VH_ERR_DEVICE, "radix sort failed");
             hipLaunchKernelGGL(k_entry_seq, dim3(grid_for(n, 256)), dim3(256), 0, st, nbase, n, seq);
         }
-        if (from) HIPCHECK(hipMemcpyAsync(from + nbase, d_from, nlog * 8, hipMemcpyDeviceToDevice, st));
-        if (bytes)
-            HIPCHECK(hipMemcpyAsync(sts + nbase * bytes, d_st, nlog * bytes, hipMemcpyDeviceToDevice, st));
+        if (from2) HIPCHECK(hipMemcpyAsync(from2 + nbase, d_from, nlog * 8, hipMemcpyDeviceToDevice, st));
+        if (sts2)
+            HIPCHECK(hipMemcpyAsync(sts2 + nbase * bytes, d_st, nlog * bytes, hipMemcpyDeviceToDevice, st));
+        if (ask_all) check_sorted(keys, n, unsorted, st);
     }
     // already in row order?  (rebuilds whose appends target their callers)
     bool sorted = nlog == 0;
     if (!sorted) {
-        check_sorted(keys, n, flag, st);
-        HIPCHECK(hipMemcpyAsync(s.d_stats.p, flag, 4, hipMemcpyDeviceToDevice, st));
         RC(readback(s, 1));
-        sorted = (uint32_t)s.h_stats[0] == 1u;
+        sorted = (uint32_t)s.h_stats[0] == 0u;
     }
-    uint64_t* from_s = from;
-    uint8_t* st_s = sts;
-    uint32_t* skeys = keys;
-    uint32_t* seq_s = seq;
+    const uint32_t* skeys = keys;
+    const uint32_t* order = nullptr;   // sorted position -> entry (null: the same)
     if (!sorted) {
         uint32_t bits = 1;
         while (bits < 32 && (rows >> bits) != 0) bits++;
         if (ekeys) bits = 32;   // removal entries sort last
-        uint32_t* sv = vals;
-        if (radix_sort_pairs(&skeys, &sv, kalt, valt, n, bits, true, sc, st))
+        if (radix_sort_pairs(&keys, &vals, kalt, valt, n, bits, true, sc, st))
             return set_error(VH_ERR_DEVICE, "radix sort failed");
-        if (from) {
-            from_s = (uint64_t*)sc.take(n * 8 + 8);
-            if (!from_s) return set_error(VH_ERR_OOM, "scratch");
-            gather_records(from_s, from, sv, n, 8, st);
-        }
-        if (bytes) {
-            st_s = (uint8_t*)sc.take(n * bytes + 8);
-            if (!st_s) return set_error(VH_ERR_OOM, "scratch");
-            gather_records(st_s, sts, sv, n, bytes, st);
-        }
-        if (seq) {
-            seq_s = (uint32_t*)sc.take(n * 4 + 4);
-            if (!seq_s) return set_error(VH_ERR_OOM, "scratch");
-            gather_records(seq_s, seq, sv, n, 4, st);
-        }
+        skeys = keys;
+        order = vals;
     }
-    // offsets
-    uint32_t* off = (uint32_t*)sc.take((rows + 1) * 4);
-    if (!off) return set_error(VH_ERR_OOM, "scratch");
+    // without a filter the entries go straight to the store, else to scratch
+    const bool filtered = n && (ekeys || has(E.hints, VH_HINT_SINGLEEDGE));
+    uint32_t* off;
+    uint64_t* from_s = nullptr;
+    uint8_t* st_s = nullptr;
+    if (filtered) {
+        off = (uint32_t*)sc.take((rows + 1) * 4);
+        if (from) from_s = (uint64_t*)sc.take(n * 8 + 8);
+        if (bytes) st_s = (uint8_t*)sc.take(n * bytes + 8);
+        if (!off || (from && !from_s) || (bytes && !st_s)) return set_error(VH_ERR_OOM, "scratch");
+        place_entries(order, n, from, from_s, from ? 8u : 0u, sts, st_s, bytes, st);
+        if (seq && order) {
+            uint32_t* seq_s = (uint32_t*)sc.take(n * 4 + 4);
+            if (!seq_s) return set_error(VH_ERR_OOM, "scratch");
+            gather_u32(seq_s, seq, order, n, st);
+            seq = seq_s;
+        }
+    } else {
+        const uint32_t srcw = ignorefrom ? 0u : E.src64 ? 8u : 4u;
+        RC(E.off.ensure((rows + 1) * 4, st));
+        if (srcw) RC(E.src.ensure(n * srcw + 8, st));
+        if (bytes) RC(E.st.ensure(n * bytes + 8, st));
+        off = E.off.as<uint32_t>();
+        place_entries(order, n, from, E.src.p, srcw, sts, E.st.p, bytes, st);
+    }
     hipLaunchKernelGGL(k_offsets_from_sorted, dim3(grid_for(rows + 1, 256)), dim3(256), 0, st, skeys, n,
                        rows, off);
     uint64_t nfinal = n;
@@ -771,7 +829,7 @@ static int build_csr(Sim& s, EdgeStore& E, bool keep_base, const uint64_t* d_to,
         if (!keep || !pos || !k32 || !off2 || (from_s && !from2) || (bytes && !st2))
             return set_error(VH_ERR_OOM, "scratch");
         fill_u8(keep, 0, n, st);   // (removal entries, past the last row, are dropped)
-        hipLaunchKernelGGL(k_remove_filter, dim3(grid_for(rows, 256)), dim3(256), 0, st, off, from_s, seq_s,
+        hipLaunchKernelGGL(k_remove_filter, dim3(grid_for(rows, 256)), dim3(256), 0, st, off, from_s, seq,
                            rows, has(E.hints, VH_HINT_SINGLEEDGE) ? 1u : 0u, ekeys, eidx, nlog, d_kind, d_from,
                            keep);
         hipLaunchKernelGGL(k_u8_to_u32, dim3(grid_for(n, 256)), dim3(256), 0, st, keep, k32, n);
@@ -812,23 +870,13 @@ static int build_csr(Sim& s, EdgeStore& E, bool keep_base, const uint64_t* d_to,
         RC(readback(s, 1));
         nfinal = (uint32_t)s.h_stats[0];
     }
-    // publish into the store
-    RC(E.off.ensure((rows + 1) * 4, st));
-    HIPCHECK(hipMemcpyAsync(E.off.p, off, (rows + 1) * 4, hipMemcpyDeviceToDevice, st));
-    if (!ignorefrom) {
-        if (E.src64) {
-            RC(E.src.ensure(nfinal * 8 + 8, st));
-            HIPCHECK(hipMemcpyAsync(E.src.p, from_s, nfinal * 8, hipMemcpyDeviceToDevice, st));
-        } else {
-            RC(E.src.ensure(nfinal * 4 + 8, st));
-            if (nfinal)
-                hipLaunchKernelGGL(k_u64_to_nr, dim3(grid_for(nfinal, 256)), dim3(256), 0, st, from_s,
-                                   E.src.as<uint32_t>(), nfinal);
-        }
-    }
-    if (bytes) {
-        RC(E.st.ensure(nfinal * bytes + 8, st));
-        HIPCHECK(hipMemcpyAsync(E.st.p, st_s, nfinal * bytes, hipMemcpyDeviceToDevice, st));
+    if (filtered) {   // into the store
+        RC(E.off.ensure((rows + 1) * 4, st));
+        HIPCHECK(hipMemcpyAsync(E.off.p, off, (rows + 1) * 4, hipMemcpyDeviceToDevice, st));
+        const uint32_t srcw = ignorefrom ? 0u : E.src64 ? 8u : 4u;
+        if (srcw) RC(E.src.ensure(nfinal * srcw + 8, st));
+        if (bytes) RC(E.st.ensure(nfinal * bytes + 8, st));
+        place_entries(nullptr, nfinal, from_s, E.src.p, srcw, st_s, E.st.p, bytes, st);
     }
     for (int t = 0; t <= VH_MAXA; t++) {
         E.rowbase[t] = newL.base[t];
@@ -1618,15 +1666,13 @@ static int apply_one(Sim& s, const vh_apply_desc* d) {
                               s.a[d->call[i]].nslots, 0, d->with_edge, st));
         if (ecnt) {
             if (scan_excl_u64(ecnt, eoff, ncallers, s.scratch, st)) return set_error(VH_ERR_DEVICE, "scan");
-            HIPCHECK(hipMemcpyAsync((uint64_t*)s.d_stats.p + 0, eoff + ncallers, 8,
-                                    hipMemcpyDeviceToDevice, st));
+            RC(copy_words(s.h_stats, eoff + ncallers, 8, st));
         }
         if (bcnt) {
             if (scan_excl_u64(bcnt, boff, ncallers, s.scratch, st)) return set_error(VH_ERR_DEVICE, "scan");
-            HIPCHECK(hipMemcpyAsync((uint64_t*)s.d_stats.p + 1, boff + ncallers, 8,
-                                    hipMemcpyDeviceToDevice, st));
+            RC(copy_words(s.h_stats + 1, boff + ncallers, 8, st));
         }
-        RC(readback(s, 2));
+        RC(wait_stream(s));
         ne_tot[0] = ecnt ? s.h_stats[0] : 0;
         nb_tot = bcnt ? s.h_stats[1] : 0;
         RC(check_errors(s));

@@ -53,11 +53,10 @@ int radix_sort_pairs(uint32_t** keys, uint32_t** vals, uint32_t* keys_alt, uint3
 void fill_u8(uint8_t* p, uint8_t v, uint64_t n, hipStream_t st);
 void fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t st);
 void iota_u32(uint32_t* p, uint64_t n, hipStream_t st);
-// dst[i] = src[idx[i]] for records of `bytes` bytes (bytes % 4 == 0 or 1/2)
-void gather_records(void* dst, const void* src, const uint32_t* idx, uint64_t n, uint32_t bytes,
-                    hipStream_t st);
-// 1 if keys[0..n) is non-decreasing, written to *flag (device)
-void check_sorted(const uint32_t* keys, uint64_t n, uint32_t* flag, hipStream_t st);
+// dst[i] = src[idx[i]]
+void gather_u32(uint32_t* dst, const uint32_t* src, const uint32_t* idx, uint64_t n, hipStream_t st);
+// *unsorted (device, cleared before) is set unless keys[0..n) is non-decreasing
+void check_sorted(const uint32_t* keys, uint64_t n, uint32_t* unsorted, hipStream_t st);
 
 inline unsigned grid_for(uint64_t n, unsigned block) {
     uint64_t g = (n + block - 1) / block;

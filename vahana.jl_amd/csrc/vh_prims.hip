@@ -201,53 +201,62 @@ int scan_excl_u64(const uint32_t* in, uint64_t* out, uint64_t n, Scratch& s, hip
 }
 
 // ------------------------------------------------------------------ radix sort
-// 8-bit digits, tiles of 512 threads x RI items.  Tile element e of wave w is
-// tile_base + w * 64 RI + i * 64 + lane (i < RI), so each wave walks its
+// Digits of DB bits, tiles of 512 threads x RI items.  Tile element e of wave
+// w is tile_base + w * 64 RI + i * 64 + lane (i < RI), so each wave walks its
 // contiguous eighth in index order; ranks inside an item row come from a
-// ballot match over the 8 digit bits and the wave's count of the digit so
+// ballot match over the digit's bits and the wave's count of the digit so
 // far, which keeps the sort stable.
 //
 // The scatter puts the tile in digit order in LDS first and writes it from
 // there, so that the elements of a digit leave as one run: written straight
 // from the ranks, a wave's 64 elements went to as many lines, and the lines of
 // all tiles at work (2 x 256 each) were evicted half written (a pass over 10^8
-// pairs: 1416 us, so 558; over 10^6: 31, so 21). Tiles of 8192 make runs of 32,
-// a line; below RADIX_LARGE pairs tiles of 2048 leave no CU idle.
+// pairs: 1416 us, so 558; over 10^6: 31, so 21).
 constexpr int RB = 512;
 constexpr int RW = RB / 64;
 constexpr uint64_t RADIX_LARGE = 4u << 20;
 
-template <int RI>
+template <int DB, int RI>
 __global__ __launch_bounds__(RB) void k_radix_hist(const uint32_t* __restrict__ keys, uint64_t n,
                                                    uint32_t shift, uint32_t ntiles,
                                                    uint32_t* __restrict__ hist) {
-    __shared__ uint32_t h[256];
-    if (threadIdx.x < 256) h[threadIdx.x] = 0;
+    constexpr uint32_t NB = 1u << DB;
+    __shared__ uint32_t h[NB];
+    for (uint32_t d = threadIdx.x; d < NB; d += RB) h[d] = 0;
     __syncthreads();
     const uint64_t base = (uint64_t)blockIdx.x * (RB * RI);
-#pragma unroll 4
-    for (int i = 0; i < RI; i++) {
-        const uint64_t e = base + (uint64_t)i * RB + threadIdx.x;
-        if (e < n) atomicAdd(&h[(keys[e] >> shift) & 255u], 1u);
+    if (n - base >= RB * RI) {
+        const uint4* k4 = (const uint4*)(keys + base);   // (the buffers start at multiples of 256 bytes)
+#pragma unroll
+        for (int i = 0; i < RI / 4; i++) {
+            const uint4 k = k4[i * RB + threadIdx.x];
+            atomicAdd(&h[(k.x >> shift) & (NB - 1)], 1u);
+            atomicAdd(&h[(k.y >> shift) & (NB - 1)], 1u);
+            atomicAdd(&h[(k.z >> shift) & (NB - 1)], 1u);
+            atomicAdd(&h[(k.w >> shift) & (NB - 1)], 1u);
+        }
+    } else {
+        for (uint64_t e = base + threadIdx.x; e < n; e += RB) atomicAdd(&h[(keys[e] >> shift) & (NB - 1)], 1u);
     }
     __syncthreads();
-    if (threadIdx.x < 256) hist[(uint64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    for (uint32_t d = threadIdx.x; d < NB; d += RB) hist[(uint64_t)d * ntiles + blockIdx.x] = h[d];
 }
 
-template <int RI>
+template <int DB, int RI>
 __global__ __launch_bounds__(RB) void k_radix_scatter(const uint32_t* __restrict__ kin,
                                                       const uint32_t* __restrict__ vin,
                                                       uint32_t* __restrict__ kout,
                                                       uint32_t* __restrict__ vout, uint64_t n,
                                                       uint32_t shift, uint32_t ntiles,
                                                       const uint32_t* __restrict__ goff) {
-    constexpr uint32_t TILE = RB * RI;
-    __shared__ uint32_t whist[RW][256];   // the waves' digit counts, then their first places in the tile
-    __shared__ uint32_t gbase[256], wsum[4];
+    constexpr uint32_t TILE = RB * RI, NB = 1u << DB;
+    constexpr uint32_t PT = NB > RB ? NB / RB : 1;   // digits per thread of the tile's scan
+    __shared__ uint32_t whist[RW][NB];   // the waves' digit counts, then their first places in the tile
+    __shared__ uint32_t gbase[NB], wsum[RW];
     __shared__ uint32_t sk[TILE], sv[TILE];
     const uint32_t tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6;
-    for (uint32_t d = tid; d < RW * 256; d += RB) (&whist[0][0])[d] = 0;
+    for (uint32_t d = tid; d < RW * NB; d += RB) (&whist[0][0])[d] = 0;
     __syncthreads();
     const uint64_t tbase = (uint64_t)blockIdx.x * TILE, wbase = tbase + (uint64_t)w * (64 * RI);
     const uint32_t cnt = n - tbase < TILE ? (uint32_t)(n - tbase) : TILE;
@@ -262,10 +271,10 @@ __global__ __launch_bounds__(RB) void k_radix_scatter(const uint32_t* __restrict
 #pragma unroll
     for (int i = 0; i < RI; i++) {
         const bool valid = wbase + (uint64_t)i * 64 + lane < n;
-        const uint32_t d = (k[i] >> shift) & 255u;
+        const uint32_t d = (k[i] >> shift) & (NB - 1);
         uint64_t peers = __ballot(valid);
 #pragma unroll
-        for (int b = 0; b < 8; b++) {
+        for (int b = 0; b < DB; b++) {
             const uint64_t bal = __ballot((d >> b) & 1u);
             peers &= ((d >> b) & 1u) ? bal : ~bal;
         }
@@ -277,56 +286,66 @@ __global__ __launch_bounds__(RB) void k_radix_scatter(const uint32_t* __restrict
     }
     __syncthreads();
     // digit d: its place in the tile and the waves' places behind it
-    uint32_t c = 0, incl = 0;
-    if (tid < 256) {
+    uint32_t c[PT], sum = 0;
 #pragma unroll
-        for (int q = 0; q < RW; q++) {
-            const uint32_t t = whist[q][tid];
-            whist[q][tid] = c;
-            c += t;
+    for (uint32_t q = 0; q < PT; q++) {
+        const uint32_t d = tid * PT + q;
+        c[q] = 0;
+        if (d < NB)
+#pragma unroll
+            for (int x = 0; x < RW; x++) {
+                const uint32_t t = whist[x][d];
+                whist[x][d] = c[q];
+                c[q] += t;
+            }
+        sum += c[q];
+    }
+    uint32_t start = wave_incl_scan(sum);
+    if (lane == 63) wsum[w] = start;
+    __syncthreads();
+    start -= sum;
+    for (int q = 0; q < w; q++) start += wsum[q];
+#pragma unroll
+    for (uint32_t q = 0; q < PT; q++) {
+        const uint32_t d = tid * PT + q;
+        if (d < NB) {
+#pragma unroll
+            for (int x = 0; x < RW; x++) whist[x][d] += start;
+            gbase[d] = goff[(uint64_t)d * ntiles + blockIdx.x] - start;
         }
-        incl = wave_incl_scan(c);
-        if (lane == 63) wsum[w] = incl;
-    }
-    __syncthreads();
-    if (tid < 256) {
-        uint32_t start = incl - c;
-        for (int q = 0; q < w; q++) start += wsum[q];
-#pragma unroll
-        for (int q = 0; q < RW; q++) whist[q][tid] += start;
-        gbase[tid] = goff[(uint64_t)tid * ntiles + blockIdx.x] - start;
+        start += c[q];
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < RI; i++) {
+    for (int i = 0; i < RI; i++)
         if (wbase + (uint64_t)i * 64 + lane < n) {
-            const uint32_t p = whist[w][(k[i] >> shift) & 255u] + rank[i];
+            const uint32_t p = whist[w][(k[i] >> shift) & (NB - 1)] + rank[i];
             sk[p] = k[i];
             sv[p] = v[i];
         }
-    }
     __syncthreads();
     for (uint32_t p = tid; p < cnt; p += RB) {
-        const uint32_t key = sk[p], o = gbase[(key >> shift) & 255u] + p;
+        const uint32_t key = sk[p], o = gbase[(key >> shift) & (NB - 1)] + p;
         kout[o] = key;
         vout[o] = sv[p];
     }
 }
 
-template <int RI>
+template <int DB, int RI>
 static int radix_sort_impl(uint32_t** keys, uint32_t** vals, uint32_t* kalt, uint32_t* valt, uint64_t n,
                            uint32_t bits, bool iota_vals, Scratch& s, hipStream_t st) {
     const uint32_t ntiles = (uint32_t)((n + RB * RI - 1) / (RB * RI));
-    uint32_t* hist = (uint32_t*)s.take((uint64_t)256 * ntiles * sizeof(uint32_t));
-    uint32_t* goff = (uint32_t*)s.take(((uint64_t)256 * ntiles + 1) * sizeof(uint32_t));
+    const uint64_t nh = (uint64_t)ntiles << DB;
+    uint32_t* hist = (uint32_t*)s.take(nh * sizeof(uint32_t));
+    uint32_t* goff = (uint32_t*)s.take((nh + 1) * sizeof(uint32_t));
     if (!hist || !goff) return -3;
     uint32_t *kin = *keys, *vin = *vals, *kout = kalt, *vout = valt;
     bool first = true;
-    for (uint32_t shift = 0; shift < bits; shift += 8) {
-        hipLaunchKernelGGL(k_radix_hist<RI>, dim3(ntiles), dim3(RB), 0, st, kin, n, shift, ntiles, hist);
-        int r = scan_excl_u32(hist, goff, (uint64_t)256 * ntiles, s, st);
+    for (uint32_t shift = 0; shift < bits; shift += DB) {
+        hipLaunchKernelGGL((k_radix_hist<DB, RI>), dim3(ntiles), dim3(RB), 0, st, kin, n, shift, ntiles, hist);
+        int r = scan_excl_u32(hist, goff, nh, s, st);
         if (r) return r;
-        hipLaunchKernelGGL(k_radix_scatter<RI>, dim3(ntiles), dim3(RB), 0, st, kin,
+        hipLaunchKernelGGL((k_radix_scatter<DB, RI>), dim3(ntiles), dim3(RB), 0, st, kin,
                            (first && iota_vals) ? (const uint32_t*)nullptr : vin, kout, vout, n,
                            shift, ntiles, goff);
         first = false;
@@ -337,12 +356,22 @@ static int radix_sort_impl(uint32_t** keys, uint32_t** vals, uint32_t* kalt, uin
     *vals = vin;
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
+// Below RADIX_LARGE pairs a pass is launches and latency: digits of 9 or 10
+// bits where they save one (17..20 bits of rows: two passes for three; 1.6 10^6
+// pairs, 18 bits: 88 us, three passes of 8 bits 122), with tiles of 4096, as
+// their counts per tile are two or four times as many; else tiles of 2048.
+// From there on 8-bit digits and tiles of 8192 (10^7 pairs, 20 bits: scatters
+// of 3 x 49 us, with 10-bit digits 2 x 76).
 int radix_sort_pairs(uint32_t** keys, uint32_t** vals, uint32_t* kalt, uint32_t* valt, uint64_t n,
                      uint32_t bits, bool iota_vals, Scratch& s, hipStream_t st) {
     if (n == 0) return 0;
     if (bits == 0) bits = 1;
-    return n < RADIX_LARGE ? radix_sort_impl<4>(keys, vals, kalt, valt, n, bits, iota_vals, s, st)
-                           : radix_sort_impl<16>(keys, vals, kalt, valt, n, bits, iota_vals, s, st);
+    const uint32_t passes = (bits + 9) / 10;
+#define VH_RADIX(DB, RI) radix_sort_impl<DB, RI>(keys, vals, kalt, valt, n, bits, iota_vals, s, st)
+    if (n >= RADIX_LARGE) return VH_RADIX(8, 16);
+    if ((bits + 7) / 8 == passes) return VH_RADIX(8, 4);
+    return bits <= 9 * passes ? VH_RADIX(9, 8) : VH_RADIX(10, 8);
+#undef VH_RADIX
 }
 
 // ------------------------------------------------------------------ helpers
@@ -368,41 +397,22 @@ void iota_u32(uint32_t* p, uint64_t n, hipStream_t st) {
     if (n) hipLaunchKernelGGL(k_iota_u32, dim3(grid_for(n, 256)), dim3(256), 0, st, p, n);
 }
 
-template <class W>
-__global__ void k_gather(W* __restrict__ dst, const W* __restrict__ src,
-                         const uint32_t* __restrict__ idx, uint64_t n, uint32_t words) {
+__global__ void k_gather_u32(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
+                             const uint32_t* __restrict__ idx, uint64_t n) {
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint64_t j = idx ? idx[i] : i;
-    for (uint32_t w = 0; w < words; w++) dst[i * words + w] = src[j * words + w];
+    if (i < n) dst[i] = src[idx[i]];
 }
-void gather_records(void* dst, const void* src, const uint32_t* idx, uint64_t n, uint32_t bytes,
-                    hipStream_t st) {
-    if (!n || !bytes) return;
-    unsigned g = grid_for(n, 256);
-    if (bytes % 8 == 0)
-        hipLaunchKernelGGL(k_gather<uint64_t>, dim3(g), dim3(256), 0, st, (uint64_t*)dst,
-                           (const uint64_t*)src, idx, n, bytes / 8);
-    else if (bytes % 4 == 0)
-        hipLaunchKernelGGL(k_gather<uint32_t>, dim3(g), dim3(256), 0, st, (uint32_t*)dst,
-                           (const uint32_t*)src, idx, n, bytes / 4);
-    else if (bytes % 2 == 0)
-        hipLaunchKernelGGL(k_gather<uint16_t>, dim3(g), dim3(256), 0, st, (uint16_t*)dst,
-                           (const uint16_t*)src, idx, n, bytes / 2);
-    else
-        hipLaunchKernelGGL(k_gather<uint8_t>, dim3(g), dim3(256), 0, st, (uint8_t*)dst,
-                           (const uint8_t*)src, idx, n, bytes);
+void gather_u32(uint32_t* dst, const uint32_t* src, const uint32_t* idx, uint64_t n, hipStream_t st) {
+    if (n) hipLaunchKernelGGL(k_gather_u32, dim3(grid_for(n, 256)), dim3(256), 0, st, dst, src, idx, n);
 }
 
-__global__ void k_check_sorted(const uint32_t* __restrict__ k, uint64_t n, uint32_t* flag) {
+__global__ void k_check_sorted(const uint32_t* __restrict__ k, uint64_t n, uint32_t* unsorted) {
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x + 1;
-    if (i < n && k[i] < k[i - 1]) *flag = 0;
+    if (i < n && k[i] < k[i - 1]) *unsorted = 1;
 }
-void check_sorted(const uint32_t* keys, uint64_t n, uint32_t* flag, hipStream_t st) {
-    fill_u32(flag, 1, 1, st);
+void check_sorted(const uint32_t* keys, uint64_t n, uint32_t* unsorted, hipStream_t st) {
     if (n > 1)
-        hipLaunchKernelGGL(k_check_sorted, dim3(grid_for(n, 256)), dim3(256), 0, st, keys, n,
-                           flag);
+        hipLaunchKernelGGL(k_check_sorted, dim3(grid_for(n, 256)), dim3(256), 0, st, keys, n, unsorted);
 }
 
 }  // namespace vh
