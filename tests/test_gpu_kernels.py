@@ -1,5 +1,7 @@
 """Edges of single kernels' ranges (tile remainders, smallest and largest
 sizes of a dispatch rule) against the checker, bit for bit (GPU)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -302,3 +304,23 @@ def test_gnp_sources(vh, gpu_ready, n, deg):
     fr, to = vh.inputs.graph_gnp(n, deg, 11)
     tid = np.uint64(1) << np.uint64(56)
     assert np.array_equal(t, tid | to.astype(np.uint64)) and np.array_equal(f, tid | fr.astype(np.uint64))
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_opinion_batch_beyond_the_caches(vh, gpu_ready, f32):
+    """Five simulations whose edges are more than 256 MB together, batched,
+    against the same simulations one by one (72 MB of edges at most)."""
+    sizes = [900_000, 750_000, 800_000, 700_001, 900_017]
+
+    def build():
+        s = C.c_void_p()
+        vh._abi.lib().stream_create(C.byref(s))
+        return [vh.models.build_opinion_gnp(vh, n, mean_deg=9.0, seed=k, graph_seed=20 + k, weight_seed=40 + k, f32=f32,
+                                            stream=s) for k, n in enumerate(sizes)]
+    ms, solo = build(), build()
+    m0 = ms[0]
+    vh.Batch().apply([m.sim for m in ms], vh.transitions.opinion(m0.E, 0.3, f32), m0.T, [m0.T, m0.E], m0.T, steps=3)
+    for m, o in zip(ms, solo):
+        for _ in range(3):
+            vh.apply_(o.sim, vh.transitions.opinion(o.E, 0.3, f32), o.T, [o.T, o.E], o.T)
+        assert np.array_equal(_states(m.sim, m.T)[0].view(np.uint8), _states(o.sim, o.T)[0].view(np.uint8))

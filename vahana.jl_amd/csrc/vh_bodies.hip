@@ -499,7 +499,16 @@ __device__ __forceinline__ void op_sum_slots(const OpLDS<T>& sm, uint32_t lo, ui
     for (; p < hi; p++) op_accum(sm.x[p - t0], sm.w[p - t0], xi, eps, num, den);
 }
 
-template <class T>
+//
+// STREAM (op_stream): sources and weights are read non-temporally, which leaves
+// more of the caches to the states (the 24 simulations, 468 MB of edges: 405 ->
+// 377 us).
+template <class V, bool STREAM>
+__device__ __forceinline__ V op_edge(const V* p) {
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <class T, bool STREAM>
 __device__ __forceinline__ void opinion_block(const uint32_t* __restrict__ off,
                                               const uint32_t* __restrict__ src,
                                               const T* __restrict__ x, const float* __restrict__ w,
@@ -531,8 +540,8 @@ __device__ __forceinline__ void opinion_block(const uint32_t* __restrict__ off,
             for (int u = 0; u < OP_U; u++) {
                 const uint32_t q = t0 + (uint32_t)u * 256u + tid;
                 const uint32_t k = b0 + (q < total ? q : 0u);   // (past the end: a valid dummy)
-                sj[u] = src[k];
-                wk[u] = w[k];
+                sj[u] = op_edge<uint32_t, STREAM>(src + k);
+                wk[u] = op_edge<float, STREAM>(w + k);
             }
 #pragma unroll
             for (int u = 0; u < OP_U; u++) xj[u] = x[sj[u] - 1];
@@ -616,7 +625,7 @@ __device__ __forceinline__ void opinion_heavy(const uint32_t* __restrict__ off,
 
 // blocks [0, nh) run one wave per heavy agent (the longest work starts
 // first), the others are light blocks
-template <class T>
+template <class T, bool STREAM>
 __global__ __launch_bounds__(256) void k_opinion(const uint32_t* __restrict__ off,
                                                  const uint32_t* __restrict__ src,
                                                  const T* __restrict__ x, const float* __restrict__ w,
@@ -624,7 +633,7 @@ __global__ __launch_bounds__(256) void k_opinion(const uint32_t* __restrict__ of
                                                  uint64_t rowbase, T eps, const uint32_t* __restrict__ heavy,
                                                  uint64_t nheavy, uint32_t nh) {
     if (blockIdx.x >= nh) {
-        opinion_block<T>(off, src, x, w, xo, n, nrows, rowbase, eps, blockIdx.x - nh);
+        opinion_block<T, STREAM>(off, src, x, w, xo, n, nrows, rowbase, eps, blockIdx.x - nh);
     } else {
         const uint64_t wv = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
         if (wv < nheavy) opinion_heavy<T>(off, src, x, w, xo, heavy[wv], rowbase, eps);
@@ -638,7 +647,7 @@ __global__ __launch_bounds__(256) void k_opinion(const uint32_t* __restrict__ of
 // [q per, (q + 1) per): its L2 then holds the states of one or two members at
 // a time instead of a share of every member's (24 members of 10^4 to 10^6
 // Float64 agents: 494 -> 462 us a step, with the kernel as it was then).
-template <class T>
+template <class T, bool STREAM>
 __global__ __launch_bounds__(256) void k_opinion_multi(const OpMember* __restrict__ mem, uint32_t nm,
                                                        uint32_t nblocks) {
     const uint32_t per = gridDim.x / 8u, blk = (blockIdx.x % 8u) * per + blockIdx.x / 8u;
@@ -652,7 +661,7 @@ __global__ __launch_bounds__(256) void k_opinion_multi(const OpMember* __restric
     const OpMember& m = mem[lo];
     const uint32_t local = blk - m.blk0;
     if (local >= m.nh) {
-        opinion_block<T>(m.off, m.src, (const T*)m.x, m.w, (T*)m.xo, m.n, m.nrows, m.rowbase, (T)m.eps,
+        opinion_block<T, STREAM>(m.off, m.src, (const T*)m.x, m.w, (T*)m.xo, m.n, m.nrows, m.rowbase, (T)m.eps,
                          local - m.nh);
     } else {
         const uint64_t wv = ((uint64_t)local * blockDim.x + threadIdx.x) >> 6;
@@ -2349,6 +2358,13 @@ static int opinion_plan(Sim& s, int t, int et, bool f32, bool& plan) {
     return VH_OK;
 }
 
+// Whether a launch's edges (source and weight) are more than the 256 MB of the
+// cache behind the L2s, where they would stay from step to step: 24 simulations,
+// us for 20 steps and reading the states, without and with: Float64 187 MB 5637
+// and 5672, 280 MB 7114 and 6960, 374 MB 8172 and 7798; Float32 234 MB 4274 and
+// 4378, 280 MB 4886 and 4905, 374 MB 5862 and 5796
+static bool op_stream(uint64_t nedges) { return nedges * 8 > (256u << 20); }
+
 int launch_opinion(Sim& s, int t, int et, const vh_opinion_params& p, bool f32, uint64_t step) {
     (void)step;
     RC(check_model_layout(s, t, et, f32 ? 4 : 8, 4, "opinion"));
@@ -2374,6 +2390,7 @@ int launch_opinion(Sim& s, int t, int et, const vh_opinion_params& p, bool f32, 
         om.nrows = nrows;
         om.rowbase = E.rowbase[t];
         om.nheavy = nheavy;
+        om.nedges = E.nedges;
         om.eps = f32 ? (double)(float)p.eps : p.eps;
         om.nh = nh;
         om.blk0 = nlight + nh;   // (the block count until the launch assigns offsets)
@@ -2381,15 +2398,17 @@ int launch_opinion(Sim& s, int t, int et, const vh_opinion_params& p, bool f32, 
         return VH_OK;
     }
     if (!plan) {
-        dim3 g(nlight + nh), b(256);
-        if (f32)
-            hipLaunchKernelGGL(k_opinion<float>, g, b, 0, s.stream, E.off.as<uint32_t>(), E.src.as<uint32_t>(),
-                               (const float*)A.rstate(), E.st.as<float>(), (float*)A.wstate(), A.nslots, nrows,
-                               E.rowbase[t], (float)p.eps, E.heavy.as<uint32_t>(), nheavy, nh);
-        else
-            hipLaunchKernelGGL(k_opinion<double>, g, b, 0, s.stream, E.off.as<uint32_t>(), E.src.as<uint32_t>(),
-                               (const double*)A.rstate(), E.st.as<float>(), (double*)A.wstate(), A.nslots, nrows,
-                               E.rowbase[t], p.eps, E.heavy.as<uint32_t>(), nheavy, nh);
+        const dim3 g(nlight + nh), b(256);
+        const bool stream = op_stream(E.nedges);
+#define VH_OPINION(T, S) \
+    hipLaunchKernelGGL((k_opinion<T, S>), g, b, 0, s.stream, E.off.as<uint32_t>(), E.src.as<uint32_t>(), \
+                       (const T*)A.rstate(), E.st.as<float>(), (T*)A.wstate(), A.nslots, nrows, E.rowbase[t], \
+                       (T)p.eps, E.heavy.as<uint32_t>(), nheavy, nh)
+        if (f32 && stream) VH_OPINION(float, true);
+        else if (f32) VH_OPINION(float, false);
+        else if (stream) VH_OPINION(double, true);
+        else VH_OPINION(double, false);
+#undef VH_OPINION
         HIPCHECK(hipGetLastError());
         return VH_OK;
     }
@@ -2444,8 +2463,9 @@ int opinion_defer_launch(OpinionDefer& c, hipStream_t st, DevBuf& dev, void** ho
     for (int k = 0; k < 2; k++) {
         std::vector<OpMember>& v = c.m[k];
         if (v.empty()) continue;
-        uint64_t blocks = 0;
+        uint64_t blocks = 0, edges = 0;
         for (OpMember& om : v) {
+            edges += om.nedges;
             const uint32_t nb = om.blk0;   // the member's block count
             om.blk0 = (uint32_t)blocks;
             blocks += nb;
@@ -2459,12 +2479,14 @@ int opinion_defer_launch(OpinionDefer& c, hipStream_t st, DevBuf& dev, void** ho
         const uint32_t grid = (uint32_t)((blocks + 7) / 8 * 8);
         const OpMember* d = (const OpMember*)((uint8_t*)dev.p + *host_off);
         *host_off += (bytes + 255) & ~(size_t)255;
-        if (k == 0)
-            hipLaunchKernelGGL(k_opinion_multi<double>, dim3(grid), dim3(256), 0, st, d, (uint32_t)v.size(),
-                               (uint32_t)blocks);
-        else
-            hipLaunchKernelGGL(k_opinion_multi<float>, dim3(grid), dim3(256), 0, st, d, (uint32_t)v.size(),
-                               (uint32_t)blocks);
+        const bool stream = op_stream(edges);
+#define VH_OPINION(T, S) \
+    hipLaunchKernelGGL((k_opinion_multi<T, S>), dim3(grid), dim3(256), 0, st, d, (uint32_t)v.size(), (uint32_t)blocks)
+        if (k == 0 && stream) VH_OPINION(double, true);
+        else if (k == 0) VH_OPINION(double, false);
+        else if (stream) VH_OPINION(float, true);
+        else VH_OPINION(float, false);
+#undef VH_OPINION
         HIPCHECK(hipGetLastError());
         v.clear();
     }

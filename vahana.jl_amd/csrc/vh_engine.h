@@ -176,7 +176,7 @@ struct OpMember {
     const float* w;
     void* xo;
     const uint32_t* heavy;
-    uint64_t n, nrows, rowbase, nheavy;
+    uint64_t n, nrows, rowbase, nheavy, nedges;
     double eps;
     uint32_t blk0, nh;   // first block of the member in the launch; its heavy-wave blocks
 };
