@@ -324,3 +324,35 @@ def test_opinion_batch_beyond_the_caches(vh, gpu_ready, f32):
         for _ in range(3):
             vh.apply_(o.sim, vh.transitions.opinion(o.E, 0.3, f32), o.T, [o.T, o.E], o.T)
         assert np.array_equal(_states(m.sim, m.T)[0].view(np.uint8), _states(o.sim, o.T)[0].view(np.uint8))
+
+
+# in-degrees around a wave's 64 lanes, the limits of the plan's classes (64,
+# 65, 512, 513) and blocks of more than 2048 agents (most without in-edges)
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("degs,n", [([0, 1, 2, 3, 63, 64, 65, 130, 512, 513, 700], 3000), ([64], 1025), ([65], 900),
+                                    ([0] * 60 + [1, 7], 40_000), ([5, 5, 5, 6, 9, 70], 6000), ([1], 64)])
+def test_opinion_plan_order(vh, ora, gpu_ready, opts, degs, n, f32):
+    """The two-pass gather over blocks ordered by in-degree, three steps."""
+    opts(opinion_plan_bytes=0, opinion_part_bytes=4096)
+    rng = np.random.default_rng(n + f32)
+    d = rng.choice(degs, n)
+    d[0] = max(d[0], 1)
+    to = np.repeat(np.arange(1, n + 1), d)
+    fr = rng.integers(1, n + 1, len(to))
+    dt = np.float32 if f32 else np.float64
+    got = []
+    for V in (vh, ora):
+        A, E = V.struct("A", [("x", dt)]), V.struct("E", [("w", "<f4")])
+        r = np.random.default_rng(n)
+        sim = V.create_simulation(V.ModelTypes() | V.register_agenttype_(A, "Immortal")
+                                  | V.register_edgetype_(E, target=A) | V.create_model("order"))
+        st, ws = np.zeros(n, dtype=A.dtype), np.zeros(len(to), dtype=E.dtype)
+        st["x"], ws["w"] = r.random(n), r.random(len(to)) + 0.01
+        sim._add_agents_array(A, st)
+        tid = np.uint64(1) << np.uint64(56)
+        sim._add_edges_array(E, tid | fr.astype(np.uint64), tid | to.astype(np.uint64), ws)
+        V.finish_init_(sim)
+        for _ in range(3):
+            V.apply_(sim, V.transitions.opinion(E, 0.3, f32), A, [A, E], A)
+        got.append(_states(sim, A)[0])
+    assert np.array_equal(*got)

@@ -692,13 +692,14 @@ __global__ __launch_bounds__(256) void k_opinion_multi(const OpMember* __restric
 // sees sequential streams (the plan's local source indices, y, the windows).
 //
 // Pass 2 (k_win_sum) takes the agent blocks from a queue. A block's staged
-// entries are listed by (window, slot): entry e holds its slot (bit 15 set on
-// the first entry of a run) and its weight, and its value is
+// entries are listed by (window, CSR slot): entry e holds its slot in LDS (bit
+// 15 set on the first entry of a run) and its weight, and its value is
 // y[prun[r] + e - pfirst[r]] for its run r, counted from the run starts
 // before its 64-entry chunk (cbase) and a ballot of the start bits. Values and
-// weights are staged in LDS by slot; then each agent of in-degree <= 64 adds
-// its slots in order, and a wave each agent of in-degree 65..WIN_HMAX (lane l
-// its slots l, l + 64, ..., then the xor butterfly). Agents above WIN_HMAX go
+// weights are staged in LDS by slot; then a lane adds the slots of each agent
+// of in-degree <= 64 in order, and a wave those of each agent of in-degree
+// 65..WIN_HMAX (lane l the l-th, l + 64th, ..., then the xor butterfly), with
+// the agents ordered by in-degree (k_win_order). Agents above WIN_HMAX go
 // first, one wave each, through their chunk lists. Most of the next block's
 // values, and its list, runs and agents, load while a block is summed. The
 // values are exactly x[src[k]] and the sums keep the canonical order, so the
@@ -708,7 +709,7 @@ struct WinCfg {
     static constexpr uint32_t WSZ = 163840 / sizeof(T);             // states per window at most
     static constexpr uint32_t TB = sizeof(T) == 8 ? 12288 : 16384;  // staged slots per block at most
     static constexpr uint32_t QU = TB / 1024;                       // list entries per thread
-    static constexpr uint32_t QA = sizeof(T) == 8 ? 8 : 12;         // of them, loaded during the previous sums
+    static constexpr uint32_t QA = sizeof(T) == 8 ? 6 : 10;         // of them, loaded during the previous sums
     static constexpr uint32_t CPB = TB / 64;                        // 64-entry chunks per block
     static constexpr uint32_t CHUNK = sizeof(T) == 8 ? 256 : 384;   // heavy-row slots staged per wave
 };
@@ -876,123 +877,141 @@ template <class T>
 struct WinLDS {
     T val[WinCfg<T>::TB];          // values by slot (heavy waves: CHUNK each)
     float wgt[WinCfg<T>::TB];      // weights by slot
-    uint32_t rp[2][WIN_RUNS];      // runs of this block and the next: plan position, list index
-    uint16_t rf[2][WIN_RUNS];
-    uint32_t wsum[WinCfg<T>::TB / 1024 + 1][16];
+    uint32_t rp[2][WIN_RUNS];      // runs of this block and the next: plan position - list index (mod 2^32)
     uint32_t nextq[2];             // queue items taken ahead
-    uint32_t nmed;                 // agents of in-degree 65..WIN_HMAX of the block (< TB / 64)
+    uint32_t nmed[4];              // agents of in-degree 65..WIN_HMAX in each wave's first 64 (< TB / 64 in all)
     uint32_t mpk[WinCfg<T>::TB / 64], magent[WinCfg<T>::TB / 64];   // slot | in-degree << 16
     T mx[WinCfg<T>::TB / 64];
 };
 
-// The round-0 and round-1 agents of a block (a0 + tid, a0 + 1024 + tid):
-// in-degrees and states, loaded with the block's list
+// A block's agents are ordered by in-degree: those of 65..WIN_HMAX ("medium"),
+// then 64 down to 0 ("light"), then the ones with chunk lists. An entry of the
+// order is the agent's index in the block | in-degree << 14 (ORD_HUGE: chunk
+// lists), and 64 entries are a group, summed by a wave. The slots of a group
+// follow those of the groups before it (gbase): its medium agents' one after
+// the other, then the light ones' by position: position q of all light agents
+// that have one, in order. So the lanes of a wave add the same number of
+// slots, give or take one, and read neighbouring ones. With a lane per agent
+// in agent order and its slots in a row, a wave took as many rounds as its
+// largest in-degree (10^7 agents, BA m = 5, about 40 for a mean of 9) with
+// bank conflicts, and the slots' starts were a block scan: 434 us a launch, so
+// 403; Float32, 5 10^6 agents of mean in-degree 10: 126, so 109. (What is left
+// is loads: without the sums 397 us, with the values read in list order 371,
+// with all values from the caches 307.)
+constexpr uint32_t ORD_LOCAL = 0x3FFFu, ORD_HUGE = 1023u;
+
+// The agents of a block at tid and 1024 + tid of its order: the entries,
+// loaded with the block's list, the waves' first slots, and the states, loaded
+// once the entries are there
 template <class T>
 struct WinAgents {
-    uint32_t o0, o1, o2, o3;   // raw loads; selected where used
+    uint32_t e0, e1, g0, g1;
     T x0, x1;
 };
+__device__ __forceinline__ uint32_t win_group(uint32_t a0, uint32_t b) { return a0 / 64u + b; }   // block b's first
 
 template <class T>
-__device__ __forceinline__ WinAgents<T> win_agents(const uint32_t* __restrict__ off, const T* __restrict__ x,
-                                                   uint64_t nrows, uint32_t a0, uint32_t a1, uint32_t tid) {
-    WinAgents<T> g;
-    const uint32_t i0 = a0 + tid, i1 = i0 + 1024;
-    const uint32_t j0 = i0 < a1 ? i0 : a0, j1 = i1 < a1 ? i1 : a0;
-    const uint32_t r0 = j0 < nrows ? j0 : 0u, r1 = j1 < nrows ? j1 : 0u;
-    g.x0 = x[j0];
-    g.x1 = x[j1];
-    g.o0 = off[r0];
-    g.o1 = off[r0 + 1];
-    g.o2 = off[r1];
-    g.o3 = off[r1 + 1];
-    return g;
+__device__ __forceinline__ void win_entries(WinAgents<T>& g, const uint32_t* __restrict__ aord,
+                                            const uint32_t* __restrict__ gbase, uint32_t b, uint32_t a0,
+                                            uint32_t a1, uint32_t tid, uint32_t wv) {
+    const uint32_t i0 = a0 + tid, i1 = i0 + 1024, gi = win_group(a0, b) + wv, ng = (a1 - a0 + 63) / 64;
+    g.e0 = aord[i0 < a1 ? i0 : a0];
+    g.e1 = aord[i1 < a1 ? i1 : a0];
+    g.g0 = gbase[wv < ng ? gi : 0u];
+    g.g1 = gbase[wv + 16 < ng ? gi + 16 : 0u];
+}
+template <class T>
+__device__ __forceinline__ void win_states(WinAgents<T>& g, const T* __restrict__ x, uint32_t a0) {
+    g.x0 = x[a0 + (g.e0 & ORD_LOCAL)];
+    g.x1 = x[a0 + (g.e1 & ORD_LOCAL)];
 }
 
-// The agents of a block, in rounds of 1024 (agent a0 + 1024 r + tid): one
-// exclusive scan of the staged in-degrees over all rounds (one barrier, which
-// also publishes the staged values); each agent of in-degree <= 64 adds its
-// slots in order, the others of the block are listed and summed by a wave
-// each (lane-strided partials, xor butterfly). Rounds 0 and 1 use the agents
-// loaded early (g); later rounds load theirs when LD (without LD the block
-// has at most two rounds, and no global load is issued). after_scan() runs
-// right after the scan's barrier.
-template <class T, bool LD, class F>
-__device__ __forceinline__ void win_sum_agents(WinLDS<T>& sm, const uint32_t* __restrict__ off,
-                                               const T* __restrict__ x, T* __restrict__ xo, uint64_t nrows, T eps,
-                                               uint32_t a0, uint32_t a1, const WinAgents<T>& g, F after_scan) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t K = (a1 - a0 + 1023) / 1024;
-    uint32_t inclk[2] = {0u, 0u}, ldk[2] = {0u, 0u};
-    for (uint32_t r = 0; r < K; r++) {
-        const uint32_t i = a0 + r * 1024 + tid;
-        uint32_t d = 0;
-        if (i < a1 && i < nrows) d = r == 0 ? g.o1 - g.o0 : r == 1 ? g.o3 - g.o2 : LD ? off[i + 1] - off[i] : 0u;
-        const uint32_t ld = d <= WIN_HMAX ? d : 0u;
-        const uint32_t incl = wave_incl_scan(ld);
-        if (lane == 63) sm.wsum[r][wv] = incl;
-        if (r < 2) {
-            inclk[r] = incl;
-            ldk[r] = ld;
-        }
+// The light agents of a group: lane l has entry e, state xi (act: there is
+// one), the group's slots start at gb
+template <class T>
+__device__ __forceinline__ void win_sum_group(WinLDS<T>& sm, T* __restrict__ xo, T eps, uint32_t a0, uint32_t e,
+                                              bool act, T xi, uint32_t gb) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t c = act ? e >> 14 : ORD_HUGE;
+    const bool light = c <= 64u;
+    const uint64_t med = __ballot(act && c > 64u && c <= WIN_HMAX);
+    uint32_t base = gb, nm = 0;
+    if (med) {   // uniform; the first lanes
+        nm = (uint32_t)__popcll(med);
+        base += (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan((med >> lane) & 1ull ? c : 0u), 63);
     }
-    if (tid == 0) sm.nmed = 0;
-    __syncthreads();
-    after_scan();
-    uint32_t base = 0;
-    for (uint32_t r = 0; r < K; r++) {
-        const uint32_t i = a0 + r * 1024 + tid;
-        uint32_t pre = 0, tot = 0;
+    const uint32_t d = light ? c : 0u;
+    const uint32_t dmax = nm < 64u ? (uint32_t)__builtin_amdgcn_readlane((int)d, (int)nm) : 0u;
+    T num = (T)0, den = (T)0;
+    uint32_t p = base + lane - nm;   // (lanes without a slot q read another value, unused; past the slots: the LDS
+    for (uint32_t q = 0; q < dmax; q += 4) {   // behind them)
+        T y[4];
+        float w[4];
+        uint64_t m[4];
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const uint32_t v = sm.wsum[r][q];
-            pre += q < wv ? v : 0u;
-            tot += v;
+        for (int u = 0; u < 4; u++) {
+            m[u] = __ballot(d > q + u);
+            y[u] = sm.val[p];
+            w[u] = sm.wgt[p];
+            p += (uint32_t)__popcll(m[u]);
         }
-        uint32_t d, incl, ld;
-        T xi;
-        if (!LD || r < 2) {
-            d = (i < a1 && i < nrows) ? (r == 0 ? g.o1 - g.o0 : g.o3 - g.o2) : 0u;
-            incl = inclk[r];
-            ld = ldk[r];
-            xi = i < a1 ? (r == 0 ? g.x0 : g.x1) : (T)0;
-        } else {
-            d = (i < a1 && i < nrows) ? off[i + 1] - off[i] : 0u;
-            ld = d <= WIN_HMAX ? d : 0u;
-            incl = wave_incl_scan(ld);
-            xi = i < a1 ? x[i] : (T)0;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const bool acc = d > q + u && fabs(y[u] - xi) <= eps;   // (a rejected one adds +0.0, as in op_accum)
+            num = num + (acc ? (T)w[u] * y[u] : (T)0);
+            den = den + (acc ? (T)w[u] : (T)0);
         }
-        const uint32_t P = base + pre + incl - ld;
-        if (i < a1 && d <= 64u) {
-            T num = (T)0, den = (T)0;
-            uint32_t q = 0;
-            for (; q + 4 <= d; q += 4) {
-                const T y0 = sm.val[P + q], y1 = sm.val[P + q + 1], y2 = sm.val[P + q + 2], y3 = sm.val[P + q + 3];
-                const float w0 = sm.wgt[P + q], w1 = sm.wgt[P + q + 1], w2 = sm.wgt[P + q + 2],
-                            w3 = sm.wgt[P + q + 3];
-                op_accum(y0, w0, xi, eps, num, den);
-                op_accum(y1, w1, xi, eps, num, den);
-                op_accum(y2, w2, xi, eps, num, den);
-                op_accum(y3, w3, xi, eps, num, den);
+    }
+    if (light) xo[a0 + (e & ORD_LOCAL)] = den > (T)0 ? num / den : xi;
+}
+
+// The agents of block b, in rounds of 1024 of its order; the staged values are
+// published by the first barrier. Rounds 0 and 1 use the entries and states
+// loaded early (g); later rounds load theirs when LD (without LD the block has
+// at most two rounds, and no global load is issued). The medium agents, which
+// are among the first TB / 64, are listed before the barrier and summed by a
+// wave each (lane-strided partials, xor butterfly). after_barrier() runs right
+// after the barrier.
+template <class T, bool LD, class F>
+__device__ __forceinline__ void win_sum_agents(WinLDS<T>& sm, const uint32_t* __restrict__ aord,
+                                               const uint32_t* __restrict__ gbase, const T* __restrict__ x,
+                                               T* __restrict__ xo, T eps, uint32_t b, uint32_t a0, uint32_t a1,
+                                               const WinAgents<T>& g, F after_barrier) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    static_assert(WinCfg<T>::TB / 64 <= 256, "the medium agents are the first four waves'");
+    if (wv < 4) {
+        const uint32_t c = a0 + tid < a1 ? g.e0 >> 14 : 0u;
+        const bool med = c > 64u && c <= WIN_HMAX;
+        const uint64_t m = __ballot(med);
+        if (lane == 0) sm.nmed[wv] = (uint32_t)__popcll(m);
+        if (m) {   // uniform
+            const uint32_t md = med ? c : 0u, P = g.g0 + wave_incl_scan(md) - md;
+            if (med) {
+                sm.mpk[tid] = P | c << 16;
+                sm.magent[tid] = a0 + (g.e0 & ORD_LOCAL);
+                sm.mx[tid] = g.x0;
             }
-            for (; q < d; q++) op_accum(sm.val[P + q], sm.wgt[P + q], xi, eps, num, den);
-            xo[i] = den > (T)0 ? num / den : xi;
-        } else if (i < a1 && d <= WIN_HMAX) {
-            const uint32_t m = atomicAdd(&sm.nmed, 1u);   // < TB / 64 (each costs > 65 of < TB)
-            sm.mpk[m] = P | d << 16;
-            sm.magent[m] = i;
-            sm.mx[m] = xi;
         }
-        base += tot;
     }
     __syncthreads();
-    const uint32_t nmed = sm.nmed;
-    for (uint32_t m = (uint32_t)wv; m < nmed; m += 16) {
+    after_barrier();
+    win_sum_group<T>(sm, xo, eps, a0, g.e0, a0 + tid < a1, g.x0, g.g0);
+    if (a1 - a0 > 1024u) win_sum_group<T>(sm, xo, eps, a0, g.e1, a0 + 1024 + tid < a1, g.x1, g.g1);
+    if (LD)
+        for (uint32_t r = 2; r * 1024u < a1 - a0; r++) {
+            const uint32_t i = a0 + r * 1024 + tid, gi = r * 16 + wv;
+            const bool act = i < a1;
+            const uint32_t e = aord[act ? i : a0];
+            const uint32_t gb = gi < (a1 - a0 + 63) / 64 ? gbase[win_group(a0, b) + gi] : 0u;
+            win_sum_group<T>(sm, xo, eps, a0, e, act, x[a0 + (e & ORD_LOCAL)], gb);
+        }
+    const uint32_t nmed = sm.nmed[0] + sm.nmed[1] + sm.nmed[2] + sm.nmed[3];
+    for (uint32_t m = 15 - wv; m < nmed; m += 16) {   // (the last waves have the smallest light in-degrees)
         const uint32_t P = sm.mpk[m] & 0xFFFFu, d = sm.mpk[m] >> 16;
         const T xi = sm.mx[m];
         T num = (T)0, den = (T)0;
-        for (uint32_t q = (uint32_t)lane; q < d; q += 64) op_accum(sm.val[P + q], sm.wgt[P + q], xi, eps, num, den);
+        for (uint32_t q = lane; q < d; q += 64) op_accum(sm.val[P + q], sm.wgt[P + q], xi, eps, num, den);
         num = xor_butterfly(num);
         den = xor_butterfly(den);
         if (lane == 0) xo[sm.magent[m]] = den > (T)0 ? num / den : xi;
@@ -1005,15 +1024,18 @@ __device__ __forceinline__ void win_sum_agents(WinLDS<T>& sm, const uint32_t* __
 // the last block to finish sets both to 0 for the next launch). Each thread
 // stages QU list entries of a block; the values of its first QA entries load
 // while the previous block is summed (in registers: the block's LDS is in
-// use), the other QU - QA after the sums. Measured slower at 10^7 agents:
-// all QU loaded during the sums (past the 128 VGPRs of a 1024-thread block:
-// spills), 512 threads with 256 VGPRs and all QU during the sums, two
-// half-size blocks in LDS, each agent's first slot from the plan instead of
-// the block scan; QA = 6 or 10 of 12 (FP64) was no faster than 8.
+// use), the other QU - QA after the sums. Measured slower or no faster at 10^7
+// Float64 agents (403 us): QA = 4, 8 or 10 of 12 (405, 404, 407); two blocks
+// of 512 threads and 5120 slots per CU (442: shorter runs); the entries in
+// pairs per lane with the lists loaded two blocks ahead (414); the tables' words
+// by a vector load an iteration ahead in place of scalar loads (403); a queue
+// per XCD that hands out 8 or 32 blocks in a row, which takes the bytes read
+// from 2.06 to 1.68 and 1.62 GB (405, 411).
 template <class T>
-__global__ __launch_bounds__(1024) void k_win_sum(const uint32_t* __restrict__ off, const T* __restrict__ x,
+__global__ __launch_bounds__(1024) void k_win_sum(const uint32_t* __restrict__ aord,
+                                                  const uint32_t* __restrict__ gbase, const T* __restrict__ x,
                                                   const T* __restrict__ y, const float* __restrict__ w,
-                                                  T* __restrict__ xo, uint64_t nrows, T eps,
+                                                  T* __restrict__ xo, T eps,
                                                   const uint4* __restrict__ hinfo, uint64_t nheavy,
                                                   const uint32_t* __restrict__ hty,
                                                   const uint16_t* __restrict__ hslot,
@@ -1050,11 +1072,10 @@ __global__ __launch_bounds__(1024) void k_win_sum(const uint32_t* __restrict__ o
             pk[u] = tpk[lb + (e < L ? e : 0u)];   // (past the list: masked where used)
         }
     };
-    auto load_runs = [&](uint32_t b, uint32_t& a, uint32_t& f) __attribute__((always_inline)) {
+    auto load_runs = [&](uint32_t b) __attribute__((always_inline)) {
         const uint32_t rb = rbase[b], R = rbase[b + 1] - rb;
         const uint32_t r = rb + (ltid < R ? ltid : 0u);   // (R == 0: the slack after the runs)
-        a = prun[r];
-        f = pfirst[r];
+        return make_uint2(prun[r], pfirst[r]);
     };
     // values and weights of entries u in [U0, U0 + QH) of block b (its runs in
     // sm.rp[c]; the wave's chunk run counts by scalar loads)
@@ -1068,7 +1089,7 @@ __global__ __launch_bounds__(1024) void k_win_sum(const uint32_t* __restrict__ o
         for (uint32_t q = 0; q < QH / 2; q++) cwv[q] = cw[U0 / 2 + q];
         // the run table reads of all QH entries first (unconditional: run 0
         // for lanes past the list), then the global loads
-        uint32_t rpv[QH], rfv[QH];
+        uint32_t rpv[QH];
 #pragma unroll
         for (uint32_t k = 0; k < QH; k++) {
             const uint32_t u = U0 + k;
@@ -1078,13 +1099,12 @@ __global__ __launch_bounds__(1024) void k_win_sum(const uint32_t* __restrict__ o
             const uint32_t cb = (cwv[k >> 1] >> ((k & 1) * 16)) & 0xFFFFu;
             const uint32_t run = ok ? cb + __popcll(m & lemask) - 1u : 0u;
             rpv[k] = sm.rp[c][run];
-            rfv[k] = sm.rf[c][run];
         }
 #pragma unroll
         for (uint32_t k = 0; k < QH; k++) {
             const uint32_t e = ltid + 1024 * (U0 + k);
             const bool ok = e < L;
-            const uint32_t pos = ok ? rpv[k] + (e - rfv[k]) : 0u;
+            const uint32_t pos = ok ? rpv[k] + e : 0u;
             v[k] = y[pos];
             wt[k] = twt[lb + (ok ? e : 0u)];
         }
@@ -1114,20 +1134,19 @@ __global__ __launch_bounds__(1024) void k_win_sum(const uint32_t* __restrict__ o
         WinAgents<T> ag;
         int cur = 0, par = 0;
         {
-            uint32_t ra, rfv;
-            load_runs(b, ra, rfv);
+            const uint2 ra = load_runs(b);
             load_list(b, true, pk);
-            ag = win_agents<T>(off, x, nrows, ablk[b], ablk[b + 1], ltid);
-            sm.rp[0][tid] = ra;
-            sm.rf[0][tid] = (uint16_t)rfv;
+            win_entries<T>(ag, aord, gbase, b, ablk[b], ablk[b + 1], ltid, (uint32_t)wv);
+            win_states<T>(ag, x, ablk[b]);
+            sm.rp[0][tid] = ra.x - ra.y;
             __syncthreads();
             load_vals(std::integral_constant<uint32_t, QA>(), b, true, 0, 0, pk, vA, wA);
         }
         // per block: the rest of its values; the next block's list, runs and
         // agents; all its values staged; the next queue item; the sums, whose
-        // scan barrier publishes the staged values and the next runs, after
-        // which the first QA values of the next block are issued (in flight
-        // during the sums); a barrier
+        // first barrier publishes the staged values and the next runs, after
+        // which the next block's states and first QA values are issued (in
+        // flight during the sums); a barrier
         for (;;) {
             asm volatile("" : "+v"(ltid));
             const bool hasn = bn != NONE;
@@ -1137,16 +1156,16 @@ __global__ __launch_bounds__(1024) void k_win_sum(const uint32_t* __restrict__ o
             float wB[QB];
             load_vals(std::integral_constant<uint32_t, QB>(), b, true, cur, QA, pk, vB, wB);
             uint32_t pkn[QU];
-            uint32_t ra, rfv;
             load_list(bnc, hasn, pkn);
-            load_runs(bnc, ra, rfv);
-            const WinAgents<T> agn = win_agents<T>(off, x, nrows, ablk[bnc], ablk[bnc + 1], ltid);
+            const uint2 ra = load_runs(bnc);
+            WinAgents<T> agn;
+            win_entries<T>(agn, aord, gbase, bnc, ablk[bnc], ablk[bnc + 1], ltid, (uint32_t)wv);
             scatter(std::integral_constant<uint32_t, QA>(), L, 0, pk, vA, wA);
             scatter(std::integral_constant<uint32_t, QB>(), L, QA, pk, vB, wB);
-            sm.rp[cur ^ 1][tid] = ra;
-            sm.rf[cur ^ 1][tid] = (uint16_t)rfv;
+            sm.rp[cur ^ 1][tid] = ra.x - ra.y;
             if (tid == 0) sm.nextq[par] = atomicAdd(queue, 1u);
-            auto after_scan = [&]() __attribute__((always_inline)) {
+            auto after_barrier = [&]() __attribute__((always_inline)) {
+                win_states<T>(agn, x, ablk[bnc]);
                 load_vals(std::integral_constant<uint32_t, QA>(), bnc, hasn, cur ^ 1, 0, pkn, vA, wA);
             };
             {
@@ -1154,9 +1173,9 @@ __global__ __launch_bounds__(1024) void k_win_sum(const uint32_t* __restrict__ o
                 // so the next block's values stay in flight
                 const uint32_t a0 = ablk[b], a1 = ablk[b + 1];
                 if (a1 - a0 <= 2048u)
-                    win_sum_agents<T, false>(sm, off, x, xo, nrows, eps, a0, a1, ag, after_scan);
+                    win_sum_agents<T, false>(sm, aord, gbase, x, xo, eps, b, a0, a1, ag, after_barrier);
                 else {
-                    win_sum_agents<T, true>(sm, off, x, xo, nrows, eps, a0, a1, ag, after_scan);
+                    win_sum_agents<T, true>(sm, aord, gbase, x, xo, eps, b, a0, a1, ag, after_barrier);
                     __builtin_amdgcn_s_waitcnt(0);   // (its loads have drained the counter anyway)
                 }
             }
@@ -1178,14 +1197,15 @@ __global__ __launch_bounds__(1024) void k_win_sum(const uint32_t* __restrict__ o
     }
 }
 
-// consistency of a built plan, one thread per block: its agents, list and
-// runs in range, every run's first entry and only those marked, each run
+// consistency of a built plan, one thread per block: its agents, order, list
+// and runs in range, every run's first entry and only those marked, each run
 // inside y, each chunk's run count; any failure sets *bad (the plan is then
 // refused: pass 2 trusts these bounds)
 __global__ void k_win_check(const uint32_t* __restrict__ ablk, const uint32_t* __restrict__ lbase,
                             const uint32_t* __restrict__ rbase, const uint32_t* __restrict__ prun,
                             const uint16_t* __restrict__ pfirst, const uint16_t* __restrict__ tpk,
-                            const uint16_t* __restrict__ cbase, uint32_t nb, uint64_t n, uint64_t nl,
+                            const uint16_t* __restrict__ cbase, const uint32_t* __restrict__ aord,
+                            const uint32_t* __restrict__ gbase, uint32_t nb, uint64_t n, uint64_t nl,
                             uint64_t nruns, uint64_t ne, uint32_t TB, uint32_t cpb, uint32_t* __restrict__ bad) {
     const uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= nb) return;
@@ -1211,7 +1231,14 @@ __global__ void k_win_check(const uint32_t* __restrict__ ablk, const uint32_t* _
             ok = cbase[b * 256 + (c % 16) * 16 + c / 16] == r - rb;
         }
     }
-    if (!ok) atomicOr(bad, 1u);
+    uint32_t slots = 0;   // (agents of the order in the block, slots of its groups in the list)
+    for (uint32_t p = 0; p < a1 - a0 && ok; p++) {
+        const uint32_t e = aord[a0 + p], d = e >> 14;
+        ok = (e & ORD_LOCAL) < a1 - a0 && (d <= WIN_HMAX || d == ORD_HUGE) &&
+             (p % 64 || gbase[win_group(a0, (uint32_t)b) + p / 64] == slots);
+        slots += d != ORD_HUGE ? d : 0u;
+    }
+    if (!ok || slots != lb1 - lb) atomicOr(bad, 1u);
 }
 
 // plan build: staged in-degree + 1 of each agent (rows past nrows: 1)
@@ -1238,6 +1265,77 @@ __global__ void k_win_blocks(const uint32_t* __restrict__ C, uint64_t n, uint32_
     if (i == 0 || C[i - 1] / S != b) {
         ablk[b] = (uint32_t)i;
         lbase[b] = C[i] - (uint32_t)i;
+    }
+}
+
+// order of each block's agents (entries by position), first slot of each of
+// its groups, and the slot of each staged in-edge (sl, numbered by the staged
+// prefix C[r] - r + position): a block of the launch per block
+__global__ __launch_bounds__(1024) void k_win_order(const uint32_t* __restrict__ off, uint64_t nrows,
+                                                    const uint32_t* __restrict__ C,
+                                                    const uint32_t* __restrict__ ablk, uint32_t* __restrict__ aord,
+                                                    uint32_t* __restrict__ gbase, uint16_t* __restrict__ sl) {
+    __shared__ uint32_t s_first[67], s_gb[256];   // keys: medium, 64 .. 0, chunk lists
+    __shared__ uint16_t s_code[16384], s_loc[16384];
+    const uint32_t b = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
+    const uint32_t a0 = ablk[b], na = ablk[b + 1] - a0;   // (< TB: every agent costs one)
+    auto code = [&](uint32_t i) {
+        const uint64_t r = (uint64_t)a0 + i;
+        const uint32_t d = r < nrows ? off[r + 1] - off[r] : 0u;
+        return d <= WIN_HMAX ? d : ORD_HUGE;
+    };
+    auto key = [](uint32_t c) { return c <= 64u ? 65u - c : c == ORD_HUGE ? 66u : 0u; };
+    if (tid < 67) s_first[tid] = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < na; i += 1024) atomicAdd(&s_first[key(code(i))], 1u);
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t f = 0;
+        for (int k = 0; k < 67; k++) {
+            const uint32_t c = s_first[k];
+            s_first[k] = f;
+            f += c;
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < na; i += 1024) {
+        const uint32_t c = code(i), p = atomicAdd(&s_first[key(c)], 1u);
+        s_code[p] = (uint16_t)c;
+        s_loc[p] = (uint16_t)i;
+        aord[a0 + p] = i | c << 14;
+    }
+    __syncthreads();
+    const uint32_t ng = (na + 63) / 64;
+    for (uint32_t g = wv; g < ng; g += 16) {
+        const uint32_t p = g * 64 + lane, c = p < na ? s_code[p] : ORD_HUGE;
+        const uint32_t t = wave_incl_scan(c != ORD_HUGE ? c : 0u);
+        if (lane == 63) s_gb[g] = t;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t f = 0;
+        for (uint32_t g = 0; g < ng; g++) {
+            const uint32_t t = s_gb[g];
+            s_gb[g] = f;
+            f += t;
+        }
+    }
+    __syncthreads();
+    for (uint32_t g = tid; g < ng; g += 1024) gbase[win_group(a0, b) + g] = s_gb[g];
+    for (uint32_t g = wv; g < ng; g += 16) {
+        const uint32_t p = g * 64 + lane, c = p < na ? s_code[p] : ORD_HUGE;
+        const uint32_t r = a0 + (p < na ? s_loc[p] : 0u), l0 = C[r] - r;
+        const bool light = c <= 64u, med = !light && c != ORD_HUGE;
+        const uint32_t md = med ? c : 0u, mi = wave_incl_scan(md);
+        for (uint32_t q = 0; q < md; q++) sl[l0 + q] = (uint16_t)(s_gb[g] + mi - md + q);
+        const uint32_t nm = (uint32_t)__popcll(__ballot(med)), d = light ? c : 0u;
+        uint32_t s0 = s_gb[g] + (uint32_t)__builtin_amdgcn_readlane((int)mi, 63) + lane - nm;
+        for (uint32_t q = 0; q < 64; q++) {
+            const uint64_t m = __ballot(d > q);
+            if (!m) break;
+            if (d > q) sl[l0 + q] = (uint16_t)s0;
+            s0 += (uint32_t)__popcll(m);
+        }
     }
 }
 
@@ -1296,14 +1394,14 @@ __global__ void k_win_starts(const uint32_t* __restrict__ keys, uint64_t nl, uin
 __global__ void k_win_pack(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ order,
                            const uint32_t* __restrict__ kidx, const uint32_t* __restrict__ flag,
                            const uint32_t* __restrict__ ridx, const uint32_t* __restrict__ pinv,
-                           const uint32_t* __restrict__ lbase, uint32_t W, uint64_t nl, const float* __restrict__ w,
-                           uint16_t* __restrict__ tpk, float* __restrict__ twt, uint32_t* __restrict__ prun,
+                           const uint32_t* __restrict__ lbase, const uint16_t* __restrict__ sl, uint32_t W,
+                           uint64_t nl, const float* __restrict__ w, uint16_t* __restrict__ tpk, float* __restrict__ twt, uint32_t* __restrict__ prun,
                            uint16_t* __restrict__ pfirst) {
     const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= nl) return;
     const uint32_t idx = order[e], blk = keys[e] / W, k = kidx[idx];
     const uint32_t st = flag[e];
-    tpk[e] = (uint16_t)((idx - lbase[blk]) | (st ? WIN_START : 0u));
+    tpk[e] = (uint16_t)(sl[idx] | (st ? WIN_START : 0u));
     twt[e] = w ? w[k] : 0.0f;
     if (st) {
         prun[ridx[e]] = pinv[k];
@@ -2143,7 +2241,7 @@ int build_gather_plan(Sim& s, EdgeStore& E, uint32_t wsz, uint64_t n, uint32_t t
     // the build's pieces in one block (the sorts take many), released at the
     // next reset when large
     const uint64_t nh_e = ne - nl;
-    if (s.scratch.room(24 * ne + 28 * nl + 22 * nh_e + 32 * (uint64_t)nb + ne / 4 + ((uint64_t)256 << 20)))
+    if (s.scratch.room(24 * ne + 30 * nl + 22 * nh_e + 32 * (uint64_t)nb + ne / 4 + ((uint64_t)256 << 20)))
         return set_error(VH_ERR_OOM, "scratch for the gather plan");
     s.scratch.shrink = true;
     uint32_t kbits = 1, lbits = 1;
@@ -2153,6 +2251,12 @@ int build_gather_plan(Sim& s, EdgeStore& E, uint32_t wsz, uint64_t n, uint32_t t
     RC(E.lbase.ensure(((uint64_t)nb + 1) * 4 + 8, st));
     hipLaunchKernelGGL(k_win_blocks, dim3(grid_for(n + 1, 256)), dim3(256), 0, st, C, n, S, nb,
                        E.ablk.as<uint32_t>(), E.lbase.as<uint32_t>());
+    RC(E.aord.ensure(n * 4 + 8, st));
+    RC(E.gbase.ensure((n / 64 + nb + 1) * 4 + 8, st));
+    uint16_t* sl = (uint16_t*)s.scratch.take(nl * 2 + 8);
+    if (!sl) return set_error(VH_ERR_OOM, "scratch");
+    hipLaunchKernelGGL(k_win_order, dim3(nb), dim3(1024), 0, st, off, nrows, C, E.ablk.as<uint32_t>(),
+                       E.aord.as<uint32_t>(), E.gbase.as<uint32_t>(), sl);
     // plan order: stable sort of the CSR slots by (window, block or heavy)
     RC(E.psrc.ensure(ne * 2 + 16, st));
     RC(E.wstart.ensure((W + 1) * 4 + 8, st));
@@ -2200,7 +2304,7 @@ int build_gather_plan(Sim& s, EdgeStore& E, uint32_t wsz, uint64_t n, uint32_t t
             RC(E.prun.ensure((uint64_t)nruns * 4 + 8, st));
             RC(E.pfirst.ensure((uint64_t)nruns * 2 + 8, st));
             hipLaunchKernelGGL(k_win_pack, dim3(grid_for(nl, 256)), dim3(256), 0, st, keys, vals, kidx, flag, ridx,
-                               pinv, E.lbase.as<uint32_t>(), (uint32_t)W, nl, w4, E.tpk.as<uint16_t>(),
+                               pinv, E.lbase.as<uint32_t>(), sl, (uint32_t)W, nl, w4, E.tpk.as<uint16_t>(),
                                E.twt.as<float>(), E.prun.as<uint32_t>(), E.pfirst.as<uint16_t>());
         } else {
             fill_u32(ridx, 0, 1, st);
@@ -2219,7 +2323,8 @@ int build_gather_plan(Sim& s, EdgeStore& E, uint32_t wsz, uint64_t n, uint32_t t
         HIPCHECK(hipStreamSynchronize(st));
         hipLaunchKernelGGL(k_win_check, dim3(grid_for(nb, 64)), dim3(64), 0, st, E.ablk.as<uint32_t>(),
                            E.lbase.as<uint32_t>(), E.rbase.as<uint32_t>(), E.prun.as<uint32_t>(),
-                           E.pfirst.as<uint16_t>(), E.tpk.as<uint16_t>(), E.cbase.as<uint16_t>(), nb, n, nl,
+                           E.pfirst.as<uint16_t>(), E.tpk.as<uint16_t>(), E.cbase.as<uint16_t>(),
+                           E.aord.as<uint32_t>(), E.gbase.as<uint32_t>(), nb, n, nl,
                            (uint64_t)nruns, ne, TB, CPB, E.wq.as<uint32_t>() + 2);
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipMemcpyAsync(&bad, E.wq.as<uint32_t>() + 2, 4, hipMemcpyDeviceToHost, st));
@@ -2416,8 +2521,9 @@ int launch_opinion(Sim& s, int t, int et, const vh_opinion_params& p, bool f32, 
     if (f32) {
         hipLaunchKernelGGL(k_win_gather<float>, g, bb, 0, s.stream, E.psrc.as<uint16_t>(), (const float*)A.rstate(),
                            E.pval.as<float>(), E.wstart.as<uint32_t>(), E.plan_w, E.plan_wsz, A.nslots, E.nedges);
-        hipLaunchKernelGGL(k_win_sum<float>, g, bb, 0, s.stream, E.off.as<uint32_t>(), (const float*)A.rstate(),
-                           E.pval.as<float>(), E.st.as<float>(), (float*)A.wstate(), nrows, (float)p.eps,
+        hipLaunchKernelGGL(k_win_sum<float>, g, bb, 0, s.stream, E.aord.as<uint32_t>(), E.gbase.as<uint32_t>(),
+                           (const float*)A.rstate(),
+                           E.pval.as<float>(), E.st.as<float>(), (float*)A.wstate(), (float)p.eps,
                            E.hinfo.as<uint4>(), E.plan_nhuge, E.hty.as<uint32_t>(), E.hslot.as<uint16_t>(),
                            E.ablk.as<uint32_t>(), E.lbase.as<uint32_t>(), E.tpk.as<uint16_t>(), E.twt.as<float>(),
                            E.rbase.as<uint32_t>(), E.prun.as<uint32_t>(), E.pfirst.as<uint16_t>(),
@@ -2426,8 +2532,9 @@ int launch_opinion(Sim& s, int t, int et, const vh_opinion_params& p, bool f32, 
         hipLaunchKernelGGL(k_win_gather<double>, g, bb, 0, s.stream, E.psrc.as<uint16_t>(),
                            (const double*)A.rstate(), E.pval.as<double>(), E.wstart.as<uint32_t>(), E.plan_w,
                            E.plan_wsz, A.nslots, E.nedges);
-        hipLaunchKernelGGL(k_win_sum<double>, g, bb, 0, s.stream, E.off.as<uint32_t>(), (const double*)A.rstate(),
-                           E.pval.as<double>(), E.st.as<float>(), (double*)A.wstate(), nrows, p.eps,
+        hipLaunchKernelGGL(k_win_sum<double>, g, bb, 0, s.stream, E.aord.as<uint32_t>(), E.gbase.as<uint32_t>(),
+                           (const double*)A.rstate(),
+                           E.pval.as<double>(), E.st.as<float>(), (double*)A.wstate(), p.eps,
                            E.hinfo.as<uint4>(), E.plan_nhuge, E.hty.as<uint32_t>(), E.hslot.as<uint16_t>(),
                            E.ablk.as<uint32_t>(), E.lbase.as<uint32_t>(), E.tpk.as<uint16_t>(), E.twt.as<float>(),
                            E.rbase.as<uint32_t>(), E.prun.as<uint32_t>(), E.pfirst.as<uint16_t>(),

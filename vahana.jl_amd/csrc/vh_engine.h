@@ -80,6 +80,7 @@ struct EdgeStore {
     DevBuf psrc, pval;             // per plan entry: local source index (uint16); gathered states
     DevBuf wstart;                 // first plan entry of each window
     DevBuf ablk, lbase;            // per block: first agent; first light-list entry
+    DevBuf aord, gbase;            // per block: its agents by in-degree; first slot of 64 of them
     DevBuf tpk, twt;               // light lists: slot | run start, weight
     DevBuf rbase, prun, pfirst;    // runs: first run per block; plan position, list index in the block
     DevBuf cbase;                  // run starts before each 64-entry chunk of a block's list (by wave)
@@ -99,7 +100,7 @@ struct EdgeStore {
     // every device buffer of the store (release, accounting)
     template <class F>
     void each_buf(F f) {
-        DevBuf* all[] = {&off,  &src,   &st,    &heavy, &psrc, &pval,    &wstart,  &ablk, &lbase,    &tpk,
+        DevBuf* all[] = {&off,  &src,   &st,    &heavy, &psrc, &pval,    &wstart,  &ablk, &lbase,    &aord, &gbase, &tpk,
                          &twt,  &rbase, &prun,  &pfirst, &cbase, &wq,     &huge,    &hbase, &hty,     &hslot,
                          &hinfo,
                          &out_off, &out_dst, &expo, &expo_cnt, &ba_pairs};
