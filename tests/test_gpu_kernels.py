@@ -356,3 +356,17 @@ def test_opinion_plan_order(vh, ora, gpu_ready, opts, degs, n, f32):
             V.apply_(sim, V.transitions.opinion(E, 0.3, f32), A, [A, E], A)
         got.append(_states(sim, A)[0])
     assert np.array_equal(*got)
+
+
+@pytest.mark.parametrize("n", [1, 3, 33, 1023, 1026, 4100, 70_001])
+def test_sir_exposure_two_launches(vh, ora, gpu_ready, opts, n):
+    """Solo SIR with the exposure pass from few agents on, the pass left out in
+    one step, around a lane's four agents and a block's 1024."""
+    M = vh.models
+    g, c = (M.build_sir(V, n, seed=3, n_init=max(1, n // 60), init="frac", edges=vh.inputs.graph_gnp(n, 6.0, 4))
+            for V in (vh, ora))
+    for k in range(8):
+        opts(sir_expose=int(k != 4), sir_expose_min=0)
+        for V, m in ((vh, g), (ora, c)):
+            M.step_sir(V, m, p_inf=0.2, seed=3, recovery=5)
+        assert np.array_equal(_states(g.sim, g.T)[0], _states(c.sim, c.T)[0]), k

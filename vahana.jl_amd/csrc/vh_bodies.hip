@@ -298,45 +298,62 @@ __global__ __launch_bounds__(256) void k_generic(const DCtx* __restrict__ c, int
     vh_generic_call<Body<TR>>(c, ci, t, pass, with_edge);
 }
 
+// inclusive sum over the lanes of a wave up to each lane (DPP: shifts within
+// rows of 16 lanes, then the row totals broadcast to the rows after them)
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);   // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);   // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);   // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);   // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);   // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);   // row_bcast:31
+    return v;
+}
+
 // ----------------------------------------------------------------- SIR
 // state word: health byte 0, pad byte 1, days bytes 2-3
 // Exposure pass: every infected agent (read state) sets the bit of each of
-// its out-neighbours in `expo` (cleared before). A susceptible agent without
-// the bit has no infected in-neighbour, so "some in-edge with an infected
-// source and a draw below p" is false without drawing: k_sir skips its draws.
-// The pass runs while the infected are few: k_sir counts the infected agents
-// it writes into 64 counters per step parity (one atomic per block), and
-// k_sir_decide, at the start of the next step, sums them into the decision
-// word that the pass and k_sir both read, so both take the same decision.
+// its out-neighbours in this launch's bitmap. A susceptible agent without the
+// bit has no infected in-neighbour, so "some in-edge with an infected source
+// and a draw below p" is false without drawing: k_sir skips its draws. (A bit
+// too many only makes an agent draw.) The pass runs while the infected are few:
+// k_sir counts the infected agents it writes into 64 counters (one atomic per
+// block), whose sum decides in the next launch: every wave of the pass adds
+// them up for itself, and its first block leaves the decision for k_sir.
+// Counters and bitmaps are two of each, by launch parity: the pass clears the
+// other counters, k_sir its agents' words of the other bitmap. With a launch each
+// for the clearing and the decision, a step of 10^5 agents took 13 us of
+// kernels and as many gaps more, so 7.5.
 // Words of `ctl`: [0, 128) counters (parity * 64 + j), 128 + parity: the
 // counters of that parity are complete, 130: the decision.
 constexpr uint32_t SIR_CTL_WORDS = 131;
 
-__global__ void k_sir_decide(uint32_t* __restrict__ ctl, uint64_t step, uint64_t n) {
-    __shared__ uint32_t s_sum[64];
-    const uint32_t j = threadIdx.x, cur = (uint32_t)(step & 1), nxt = cur ^ 1u;
-    s_sum[j] = ctl[cur * 64 + j];
-    __syncthreads();
-    if (j == 0) {
-        uint64_t total = 0;
-        for (int q = 0; q < 64; q++) total += s_sum[q];
-        ctl[130] = ctl[128 + cur] && total * 32 <= n ? 1u : 0u;
-        ctl[128 + nxt] = 1u;   // this step's k_sir fills the other set
-    }
-    ctl[nxt * 64 + j] = 0u;
-}
-__device__ __forceinline__ bool sir_expose_on(const uint32_t* ctl) { return ctl && ctl[130] != 0u; }
+// four consecutive agents per lane; marks as vh_expose_wave does
 __global__ __launch_bounds__(256) void k_sir_expose(const uint32_t* __restrict__ rs,
                                                     const uint32_t* __restrict__ out_off,
                                                     const uint32_t* __restrict__ out_dst, uint64_t n,
-                                                    const uint32_t* __restrict__ ctl,
+                                                    uint32_t parity, uint32_t* __restrict__ ctl,
                                                     uint32_t* __restrict__ expo) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !sir_expose_on(ctl) || (rs[i] & 0xFFu) != VH_I) return;
-    for (uint32_t k = out_off[i]; k < out_off[i + 1]; k++) {
-        const uint32_t v = out_dst[k];
-        atomicOr(expo + (v >> 5), 1u << (v & 31u));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(ctl[parity * 64 + lane]), 63);
+    const bool on = ctl[128 + parity] && (uint64_t)total * 32 <= n;
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        ctl[(parity ^ 1u) * 64 + lane] = 0u;
+        if (lane == 0) {
+            ctl[130] = on ? 1u : 0u;
+            ctl[128 + (parity ^ 1u)] = 1u;   // this launch's k_sir fills the other set
+        }
     }
+    if (!on) return;   // uniform
+    const uint64_t i = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    const uint32_t in = i >= n ? 0u : n - i < 4 ? (uint32_t)(n - i) : 4u;
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (in == 4) v = *(const u32x4*)(rs + i);
+    else
+        for (uint32_t q = 0; q < in; q++) v[q] = rs[i + q];
+#pragma unroll
+    for (uint32_t q = 0; q < 4; q++) vh_expose_wave(q < in && (v[q] & 0xFFu) == VH_I, i + q, out_off, out_dst, expo);
 }
 
 __global__ __launch_bounds__(256) void k_sir(const uint32_t* __restrict__ off,
@@ -345,13 +362,15 @@ __global__ __launch_bounds__(256) void k_sir(const uint32_t* __restrict__ off,
                                              uint32_t* __restrict__ ws, uint64_t n, uint64_t nrows,
                                              uint64_t rowbase, uint32_t t, double p, uint64_t seed,
                                              uint32_t rec, uint64_t step, const uint32_t* __restrict__ expo,
+                                             uint32_t* __restrict__ expo_next, uint32_t parity,
                                              uint32_t* __restrict__ ctl) {
     __shared__ uint32_t s_inf[4];
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool in = i < n;
     uint32_t s = in ? rs[i] : 0u;
     uint32_t h = s & 0xFFu;
-    const bool skip = in && h == VH_S && sir_expose_on(ctl) && !((expo[i >> 5] >> (i & 31u)) & 1u);
+    const bool skip = in && h == VH_S && ctl && ctl[130] && !((expo[i >> 5] >> (i & 31u)) & 1u);
+    if (ctl && in && (i & 31u) == 0) expo_next[i >> 5] = 0u;
     if (in && h == VH_S && !skip) {
         if (i < nrows) {
             const uint64_t pre = vh_hash_pre(seed, vh_make_id(t, i + 1), step);
@@ -374,7 +393,7 @@ __global__ __launch_bounds__(256) void k_sir(const uint32_t* __restrict__ off,
         __syncthreads();
         if (threadIdx.x == 0) {
             const uint32_t c = s_inf[0] + s_inf[1] + s_inf[2] + s_inf[3];
-            if (c) atomicAdd(ctl + ((step + 1) & 1) * 64 + (blockIdx.x & 63u), c);
+            if (c) atomicAdd(ctl + (parity ^ 1u) * 64 + (blockIdx.x & 63u), c);
         }
     }
 }
@@ -393,18 +412,6 @@ __device__ __forceinline__ void op_accum(T xj, float w, T xi, T eps, T& num, T& 
     const bool acc = fabs(xj - xi) <= eps;
     num = num + (acc ? (T)w * xj : (T)0);
     den = den + (acc ? (T)w : (T)0);
-}
-
-// inclusive sum over the lanes of a wave up to each lane (DPP: shifts within
-// rows of 16 lanes, then the row totals broadcast to the rows after them)
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);   // row_shr:1
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);   // row_shr:2
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);   // row_shr:4
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);   // row_shr:8
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);   // row_bcast:15
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);   // row_bcast:31
-    return v;
 }
 
 // the value of lane l ^ O (O = 1, 2: DPP quad permutations; 4, 8, 16:
@@ -2129,21 +2136,26 @@ static int check_model_layout(Sim& s, int t, int et, uint32_t abytes, uint32_t e
 
 
 // Out-edges of E's rows (one agent type, rows from 0, 1-based sources up to
-// nsrc): the transpose of its in-edges; the exposure bitmap and the counters
+// nsrc): the transpose of its in-edges; the exposure bitmaps and the counters
 static int build_out_csr(Sim& s, EdgeStore& E, uint64_t nsrc) {
-    if (E.out_version == E.version && E.expo.p && E.expo.cap >= ((nsrc + 31) / 32) * 4 + 16) return VH_OK;
+    const uint64_t words = (nsrc + 31) / 32;
+    if (E.out_version == E.version && E.out_n == nsrc && E.expo.p) return VH_OK;
     hipStream_t st = s.stream;
     RC(E.out_off.ensure((nsrc + 1) * 4 + 8, st));
     RC(E.out_dst.ensure(E.nedges * 4 + 8, st));
     OutSeg seg = {E.off.as<uint32_t>(), E.src.as<uint32_t>(), E.out_off.as<uint32_t>(), E.out_dst.as<uint32_t>(),
-                  nullptr, 0, E.rows, nsrc, E.nedges};
+                  nullptr, 2 * words, E.rows, nsrc, E.nedges};
+    E.out_version = ~0ull;
+    RC(E.expo.ensure(2 * words * 4 + 16, st));
+    seg.bits = E.expo.as<uint32_t>();
     out_edges_plan(&seg, 1);
     RC(build_out_edges(&seg, nullptr, 1, s.scratch, st));
-    RC(E.expo.ensure(((nsrc + 31) / 32) * 4 + 16, st));
     RC(E.expo_cnt.ensure(SIR_CTL_WORDS * 4 + 8, st));
     fill_u32(E.expo_cnt.as<uint32_t>(), 0u, SIR_CTL_WORDS, st);   // no complete counts yet
     HIPCHECK(hipGetLastError());
     E.out_version = E.version;
+    E.out_n = nsrc;
+    E.expo_parity = 0;
     return VH_OK;
 }
 
@@ -2155,26 +2167,30 @@ int launch_sir(Sim& s, int t, int et, const vh_sir_params& p, uint64_t step) {
     if (!A.nslots) return VH_OK;
     // the exposure pass needs the in-edges of `t` only (rows from 0, sources
     // of `t`); it runs for at least sir_expose_min agents (default 65536:
-    // below, its three extra launches per step cost more than the draws it
-    // saves) unless the options turn it off
+    // below, its extra launch per step costs more than the draws it saves)
+    // unless the options turn it off
     uint32_t* expo = nullptr;
+    uint32_t* next = nullptr;
     uint32_t* cnt = nullptr;
+    uint32_t parity = 0;
     const uint64_t nrows = E.rows ? E.nrows[t] : 0ull;
     if (nrows && E.nedges && !E.src64 && E.src_type == (uint32_t)t && E.rowbase[t] == 0 && nrows == E.rows &&
         A.nslots < 0xFFFFFFFFull && g_opts.sir_expose != 0 && (int64_t)A.nslots >= g_opts.sir_expose_min) {
         RC(build_out_csr(s, E, A.nslots));
-        expo = E.expo.as<uint32_t>();
+        parity = E.expo_parity;
+        E.expo_parity ^= 1u;
+        const uint64_t words = (E.out_n + 31) / 32;
+        expo = E.expo.as<uint32_t>() + parity * words;
+        next = E.expo.as<uint32_t>() + (parity ^ 1u) * words;
         cnt = E.expo_cnt.as<uint32_t>();
-        fill_u32(expo, 0, (A.nslots + 31) / 32, s.stream);
-        hipLaunchKernelGGL(k_sir_decide, dim3(1), dim3(64), 0, s.stream, cnt, step, A.nslots);
-        hipLaunchKernelGGL(k_sir_expose, dim3(grid_for(A.nslots, 256)), dim3(256), 0, s.stream,
+        hipLaunchKernelGGL(k_sir_expose, dim3(grid_for(A.nslots, 1024)), dim3(256), 0, s.stream,
                            (const uint32_t*)A.rstate(), E.out_off.as<uint32_t>(), E.out_dst.as<uint32_t>(),
-                           A.nslots, (const uint32_t*)cnt, expo);
+                           A.nslots, parity, cnt, expo);
     }
     hipLaunchKernelGGL(k_sir, dim3(grid_for(A.nslots, 256)), dim3(256), 0, s.stream,
                        E.off.as<uint32_t>(), E.src.as<uint32_t>(), (const uint32_t*)A.rstate(),
                        (uint32_t*)A.wstate(), A.nslots, nrows, E.rowbase[t],
-                       (uint32_t)t, p.p_inf, p.seed, p.recovery, step, (const uint32_t*)expo, cnt);
+                       (uint32_t)t, p.p_inf, p.seed, p.recovery, step, (const uint32_t*)expo, next, parity, cnt);
     HIPCHECK(hipGetLastError());
     return VH_OK;
 }

@@ -93,9 +93,11 @@ struct EdgeStore {
     uint32_t plan_wsz = 0, plan_tb = 0, plan_nb = 0, plan_w = 0;
     uint64_t plan_nhuge = 0;
     // out-edges of the SIR exposure pass (build_out_csr), valid for
-    // `out_version`; `expo`: one bit per agent, set when it has an infected
-    // in-neighbour in this step; `expo_cnt`: infected counts by step parity
+    // `out_version`; `expo`: by launch parity, one bit per agent, set when it
+    // has an infected in-neighbour; `expo_cnt`: infected counts by parity
     DevBuf out_off, out_dst, expo, expo_cnt;
+    uint64_t out_n = 0;            // their agents
+    uint32_t expo_parity = 0;      // of the next launch
     uint64_t out_version = ~0ull;
     // every device buffer of the store (release, accounting)
     template <class F>
