@@ -682,16 +682,20 @@ static void compute_layout(Sim& s, const EdgeStore& E, RowLayout& L, uint64_t& r
 }
 
 // n words between device memory and pinned host memory, either way. A kernel
-// in place of a copy command: one wave's loads and stores, where a copy of a
+// in place of a copy command: one block's loads and stores, where a copy of a
 // few bytes or of a context (6 KB) costs its own command and, from or to
-// pageable memory, a wait of its own.
-static __global__ __launch_bounds__(256) void k_words(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
-                                                      uint32_t n) {
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+// pageable memory, a wait of its own. Four words a thread where both sides
+// allow: a read of host memory takes 2 us, and a context word by word was six
+// of them in a row (@@ us, so @@).
+static __global__ __launch_bounds__(512) void k_words(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
+                                                      uint32_t n, uint32_t n4) {
+    for (uint32_t i = threadIdx.x; i < n4; i += blockDim.x) ((uint4*)dst)[i] = ((const uint4*)src)[i];
+    for (uint32_t i = 4 * n4 + threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
 }
 static int copy_words(void* dst, const void* src, size_t bytes, hipStream_t st) {
-    hipLaunchKernelGGL(k_words, dim3(1), dim3(bytes <= 256 ? 64 : 256), 0, st, (uint32_t*)dst, (const uint32_t*)src,
-                       (uint32_t)(bytes / 4));
+    const uint32_t n = (uint32_t)(bytes / 4), n4 = (((uintptr_t)dst | (uintptr_t)src) & 15u) ? 0u : n / 4;
+    hipLaunchKernelGGL(k_words, dim3(1), dim3(bytes <= 256 ? 64 : 512), 0, st, (uint32_t*)dst, (const uint32_t*)src, n,
+                       n4);
     HIPCHECK(hipGetLastError());
     return VH_OK;
 }
