@@ -370,3 +370,32 @@ def test_sir_exposure_two_launches(vh, ora, gpu_ready, opts, n):
         for V, m in ((vh, g), (ora, c)):
             M.step_sir(V, m, p_inf=0.2, seed=3, recovery=5)
         assert np.array_equal(_states(g.sim, g.T)[0], _states(c.sim, c.T)[0]), k
+
+
+@pytest.mark.parametrize("block,apt", [(64, 1), (64, 4), (128, 1), (256, 1)])
+def test_ensemble_long_runs(vh, ora, gpu_ready, opts, block, apt):
+    """Epidemics that are over, not yet everywhere, or nearly everywhere, over
+    60 steps, in tiles from a quarter of a wave's four agents per lane on,
+    one member past its horizon."""
+    opts(sir_expose=1, sir_expose_min=0)
+    E = vh.ensemble.Ensemble()
+    E.set_config(block, False)
+    E.set_tiles([apt] * 3)
+    sizes = [(3000, 3.0, 0.3, 1), (5000, 1.2, 0.3, 3), (20_000, 2.0, 0.2, 1), (4097, 6.0, 0.2, 60), (900, 0.5, 0.9, 2)]
+    ids = [E.add_sir(n, d, p, 90 + k, 30 + k, recovery=4, n_init=i) for k, (n, d, p, i) in enumerate(sizes)]
+    sims = [vh.models.build_sir(ora, n, seed=90 + k, n_init=i, init="frac", edges=vh.inputs.graph_gnp(n, d, 30 + k))
+            for k, (n, d, p, i) in enumerate(sizes)]
+    done = [0] * len(sizes)
+
+    def check(upto):
+        for k, (n, d, p, i) in enumerate(sizes):
+            while done[k] < upto[k]:
+                vh.models.step_sir(ora, sims[k], p_inf=p, seed=90 + k, recovery=4)
+                done[k] += 1
+            got, want = E.read(ids[k])[0], sims[k].sim._read_agents(sims[k].T)[0]
+            assert np.array_equal(np.ascontiguousarray(got).view(np.uint8), np.ascontiguousarray(want).view(np.uint8)), k
+    E.set_horizon(ids[2], 9)
+    E.step(14)
+    check([14, 14, 9, 14, 14])
+    E.step(46, use_graph=False)
+    check([60, 60, 9, 60, 60])

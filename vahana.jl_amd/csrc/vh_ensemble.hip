@@ -333,10 +333,12 @@ __global__ __launch_bounds__(256) void k_ens_expose(const MemberDesc* __restrict
         const MemberDesc& m = md[mi];
         uint32_t* bits = m.bits + parity * m.nw;
         const uint64_t a0 = bstart[lb];
-        // four consecutive agents per lane (tiles are multiples of 64)
-        for (uint32_t o = 4 * threadIdx.x; o < m.tile; o += 4 * 256) {
+        // four consecutive agents per lane (tiles are multiples of 64); whole
+        // waves, as vh_expose_wave takes them: a tile of 64 is a wave's first 16 lanes
+        for (uint32_t w = 4 * (threadIdx.x & ~63u); w < m.tile; w += 4 * 256) {
+            const uint32_t o = w + 4 * (threadIdx.x & 63u);
             const uint64_t i = a0 + o;
-            const uint32_t in = i >= m.n ? 0u : m.n - i < 4 ? (uint32_t)(m.n - i) : 4u;
+            const uint32_t in = o >= m.tile || i >= m.n ? 0u : m.n - i < 4 ? (uint32_t)(m.n - i) : 4u;
             ens_u32x4 v = {0u, 0u, 0u, 0u};
             if (in == 4) v = *(const ens_u32x4*)(m.rs + i);
             else
