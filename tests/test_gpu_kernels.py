@@ -375,8 +375,9 @@ def test_sir_exposure_two_launches(vh, ora, gpu_ready, opts, n):
 @pytest.mark.parametrize("block,apt", [(64, 1), (64, 4), (128, 1), (256, 1)])
 def test_ensemble_long_runs(vh, ora, gpu_ready, opts, block, apt):
     """Epidemics that are over, not yet everywhere, or nearly everywhere, over
-    60 steps, in tiles from a quarter of a wave's four agents per lane on,
-    one member past its horizon."""
+    60 steps, in tiles from a quarter of a wave's four agents per lane on: with
+    the exposure pass switched off and on between calls, members past
+    their horizon and called on again after it."""
     opts(sir_expose=1, sir_expose_min=0)
     E = vh.ensemble.Ensemble()
     E.set_config(block, False)
@@ -397,5 +398,11 @@ def test_ensemble_long_runs(vh, ora, gpu_ready, opts, block, apt):
     E.set_horizon(ids[2], 9)
     E.step(14)
     check([14, 14, 9, 14, 14])
-    E.step(46, use_graph=False)
-    check([60, 60, 9, 60, 60])
+    opts(sir_expose=0)
+    E.step(3)
+    opts(sir_expose=1)
+    E.set_horizon(ids[2], 0)
+    E.step(20, use_graph=False)
+    check([37, 37, 29, 37, 37])
+    E.step(23)
+    check([60, 60, 52, 60, 60])

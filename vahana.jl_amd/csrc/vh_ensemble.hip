@@ -371,7 +371,10 @@ __global__ void k_sir_ensemble(const MemberDesc* __restrict__ md, const uint32_t
     const uint32_t mi = bmember[b];
     const MemberDesc& m = md[mi];
     const uint64_t a0 = bstart[b];
-    if (a0 >= m.n) return;      // whole block (a member past its horizon has n = 0)
+    if (a0 >= m.n) {            // whole block (a member past its horizon has n = 0: no state is written)
+        if (dec && threadIdx.x == 0) blkcnt[(uint64_t)(parity ^ 1u) * nblocks + b] = 0xFFFFFFFFu;
+        return;
+    }
     const uint32_t dm = dec ? dec[mi] : 0u;
     const bool ex = (dm & 1u) != 0u;
     const uint32_t apt = m.tile / blockDim.x;
@@ -932,9 +935,12 @@ extern "C" int vh_ensemble_step(vh_ensemble_t e, uint32_t steps, int use_graph) 
     const bool expose = g_opts.sir_expose != 0 && (int64_t)total >= g_opts.sir_expose_min;
     if (expose) {
         RC(build_members_out(e));
-        // the bitmaps were not kept while the pass was off: every member's
-        // next exposure launch is a full one
-        if (!e->expose_last) fill_u32(e->d_dec.as<uint32_t>(), 0u, nm, e->stream);
+        // the bitmaps and counts were not kept while the pass was off: every
+        // member's next launch counts, the one after is a full one
+        if (!e->expose_last) {
+            fill_u32(e->d_dec.as<uint32_t>(), 0u, nm, e->stream);
+            fill_u32(e->d_blkcnt.as<uint32_t>(), 0xFFFFFFFFu, (uint64_t)e->nblocks * 2, e->stream);
+        }
     }
     e->expose_last = expose;
     // one descriptor table per step (buffers alternate, step numbers grow)
