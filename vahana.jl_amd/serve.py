@@ -59,9 +59,9 @@ def footprint(req):
     fp = req.n * 16 + req.n * 4 + e * 8 + req.n * 8
     if req.n * 8 >= OPINION_PLAN_MIN_BYTES:
         # the two-pass gather: local source indices, gathered states, lists
-        # with their weights, run tables; the scratch of the one-time plan
-        # build (its sorts)
-        fp += e * 17 + req.n * 8 + e * 53
+        # with their weights, run tables, the agents' order; the scratch of the
+        # one-time plan build (its sorts)
+        fp += e * 17 + req.n * 12 + e * 55
     return int(fp)
 
 
