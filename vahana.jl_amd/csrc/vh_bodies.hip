@@ -1574,6 +1574,50 @@ __device__ __forceinline__ bool contact_partner(uint64_t pre, uint32_t n, const 
     }
     return false;
 }
+// the same for a contact whose first draw is known not to be kept
+__device__ __forceinline__ bool contact_again(uint64_t pre, uint32_t n, const vh_contact_params& p, uint64_t i,
+                                              uint32_t cc, const ContactBits& B, uint32_t& j) {
+    j = contact_draw(pre, n, p, cc, 0);
+    if (j != i && !cbit(B.dead, j)) return false;
+    for (uint32_t r = 1; r < p.max_redraw; r++) {
+        j = contact_draw(pre, n, p, cc, r);
+        if (j == i) continue;
+        if (!cbit(B.sp, j)) return true;
+        if (!cbit(B.dead, j)) return false;
+    }
+    return false;
+}
+// A wave's contacts that draw again (todo: a bit each), 64 at a time, one per
+// lane: every lane calls f(act, lane of the slot, contact). With 2% deaths a
+// slot has 0.8 of them and the worst of 64 slots four: on the slots' own lanes,
+// a wave goes four times through the draws and their lookups for 51 of them
+// (k_contact_edges at 10^7 slots: 238 us so, 220 in pairs; k_contact_main, whose
+// ALU is busy anyway and whose filter leaves no LDS for the lists without larger
+// groups elsewhere, 441 and 460: not there).
+template <class F>
+__device__ __forceinline__ void contact_pairs(uint32_t todo, uint16_t* pair, F f) {
+    const uint32_t lane = threadIdx.x & 63u;
+    while (__ballot(todo != 0u)) {
+        const uint32_t c = (uint32_t)__popc(todo), incl = wave_incl_scan(c);
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        for (uint32_t k = incl - c; todo && k < 64u; k++) {
+            pair[k] = (uint16_t)(lane | (uint32_t)__builtin_ctz(todo) << 6);
+            todo &= todo - 1u;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const uint32_t e = lane < total ? pair[lane] : lane;
+        f(lane < total, e & 63u, e >> 6);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
+__device__ __forceinline__ uint64_t contact_shfl(uint64_t v, uint32_t lane) {
+    return (uint64_t)(uint32_t)__shfl((int)(uint32_t)v, (int)lane, 64) |
+           (uint64_t)(uint32_t)__shfl((int)(uint32_t)(v >> 32), (int)lane, 64) << 32;
+}
 // Infections: a susceptible slot gets infected when some in-edge (a contact of
 // the last step) has an infected source and a draw below beta * susceptibility.
 // "Some" has no order: the draw (ALU) first, the source's flag only for the
@@ -1734,23 +1778,29 @@ __global__ __launch_bounds__(256) void k_contact_edges(uint32_t n, uint32_t t, v
     uint2 m = make_uint2(0u, 0u);
     if (i < n) m = masks[i];
     const uint32_t cnt = (uint32_t)__popc(m.x), incl = wave_incl_scan(cnt);
+    __shared__ uint16_t s_pair[256];
+    uint32_t r0 = 0;   // first of the slot's contacts in lds
+    const uint64_t pre = vh_hash_pre(p.seed, vh_make_id(t, i + 1), step);
     if (i < n) {
         const uint32_t o = cpos[B.nwords + (i >> 6)] - deaths + incl - cnt;
         off[i] = o;
         if (i == n - 1) off[n] = o + cnt;
-        uint32_t* row = lds + (o - base);
-        const uint64_t pre = vh_hash_pre(p.seed, vh_make_id(t, i + 1), step);
+        r0 = o - base;
+        uint32_t* row = lds + r0;
         const uint32_t first = m.x & ~m.y;
         for (uint32_t cc = 0; cc < C; cc++)
             if ((first >> cc) & 1u)
                 row[__popc(m.x & ((1u << cc) - 1u))] = contact_draw(pre, n, p, cc, 0) + 1u;
-        for (uint32_t re = m.y; re; re &= re - 1u) {
-            const uint32_t cc = (uint32_t)__builtin_ctz(re);
-            uint32_t j = 0;
-            (void)contact_partner(pre, n, p, i, cc, B, j);
-            row[__popc(m.x & ((1u << cc) - 1u))] = j + 1u;
-        }
     }
+    contact_pairs(m.y, s_pair + (tid & ~63u), [&](bool act, uint32_t who, uint32_t cc) {
+        const uint64_t pw = contact_shfl(pre, who);
+        const uint32_t mw = (uint32_t)__shfl((int)m.x, (int)who, 64), rw = (uint32_t)__shfl((int)r0, (int)who, 64);
+        uint32_t j = 0;
+        if (act) {
+            (void)contact_again(pw, n, p, (i & ~(uint64_t)63) + who, cc, B, j);
+            lds[rw + (uint32_t)__popc(mw & ((1u << cc) - 1u))] = j + 1u;
+        }
+    });
     __syncthreads();
     for (uint32_t q = tid; q < end - base; q += 256) __builtin_nontemporal_store(lds[q], src + base + q);
 }
