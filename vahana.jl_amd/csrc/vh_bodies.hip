@@ -37,10 +37,16 @@ struct Body<VH_TR_SUM_NEIGHBORS> {
                 return true;
             }
             const Neighbors nb(c, et);
-            const uint8_t* n[4];
+            constexpr int SUM_N = 8;
+            const uint8_t* n[SUM_N];
             uint32_t k = b;
-            for (; k + 4 <= e && nb.four(k, n); k += 4)
-                sum += ld_i64(n[0]) + ld_i64(n[1]) + ld_i64(n[2]) + ld_i64(n[3]);
+            for (; k < e && nb.some(k, e, n); k = e - k > SUM_N ? k + SUM_N : e) {
+                int64_t v[SUM_N];
+#pragma unroll
+                for (int q = 0; q < SUM_N; q++) v[q] = ld_i64(n[q]);
+#pragma unroll
+                for (int q = 0; q < SUM_N; q++) sum += k + q < e ? v[q] : 0;
+            }
             for (; k < e; k++) {
                 const uint8_t* ns = nb.state(k);
                 if (!ns) return true;
