@@ -243,9 +243,11 @@ def test_ensemble_four_agents_per_thread(vh, ora, gpu_ready, opts, block, expose
 
 
 # around a tile of 2048 pairs, several, and the switch to tiles of 8192
-# (4 194 304) with and without a partial last tile
+# (4 194 304) with and without a partial last tile; digits of 9 bits (17 and 26
+# bits of rows) and 10 (10 and 20 bits)
 @pytest.mark.parametrize("ne,n", [(1, 1), (63, 300), (2047, 5), (2048, 70_000), (2049, 256), (70_001, 66_000),
-                                  (4_194_303, 100_000), (4_194_304, 257), (4_202_500, 17_000_000)])
+                                  (4_194_303, 100_000), (4_194_304, 257), (4_202_500, 17_000_000),
+                                  (5000, 900), (300_000, 900_000), (4097, 40_000_000)])
 def test_edges_sorted_stably(vh, gpu_ready, ne, n):
     """The CSR of edges added in random order: targets ascending, each
     target's edges (source, state) in the order they were added."""
