@@ -176,6 +176,12 @@ __device__ __forceinline__ uint64_t vh_src_id(const DEdge& E, uint64_t k) {
 }
 
 // ------------------------------------------------------------------ body API
+// The step of a loop over the in-edges [k, e) of a row: k + step, or e where
+// that is past it. An edge type holds up to 2^32 - 2 edges: near the last ones
+// a plain k + step in 32 bits passes 2^32 and starts over at other rows' edges.
+__host__ __device__ __forceinline__ uint32_t vh_row_next(uint32_t k, uint32_t e, uint32_t step) {
+    return e - k > step ? k + step : e;
+}
 // in-edges [b, e) of `to` for edge type et (false: none / not readable)
 __device__ __forceinline__ bool d_row(const DCtx* c, int et, uint64_t to, uint32_t& b, uint32_t& e) {
     b = e = 0;
@@ -243,7 +249,7 @@ struct Neighbors {
     const uint8_t* died;     // nullptr: no removed agents to look out for
     uint32_t nslots, bytes;
 
-    __device__ __forceinline__ Neighbors(const DCtx* ctx, int et) : c(ctx), E(&ctx->e[et]), src(nullptr) {
+    __host__ __device__ __forceinline__ Neighbors(const DCtx* ctx, int et) : c(ctx), E(&ctx->e[et]), src(nullptr) {
         const uint32_t t = E->src_type;
         if (E->src64 || t == 0 || t > VH_MAXA || !c->a[t].readable) return;
         const DAgent& A = c->a[t];
@@ -255,13 +261,13 @@ struct Neighbors {
     }
     __device__ __forceinline__ const uint8_t* state(uint64_t k) const { return d_state(c, vh_src_id(*E, k)); }
     template <int N>
-    __device__ __forceinline__ bool some(uint32_t k, uint32_t e, const uint8_t* (&p)[N]) const {
+    __host__ __device__ __forceinline__ bool some(uint32_t k, uint32_t e, const uint8_t* (&p)[N]) const {
         if (!src) return false;
         uint32_t s[N], m = 0;
 #pragma unroll
-        for (int q = 0; q < N; q++) s[q] = src[k + q < e ? k + q : e - 1u] - 1u;
+        for (uint32_t q = 0; q < N; q++) s[q] = src[q < e - k ? k + q : e - 1u] - 1u;
 #pragma unroll
-        for (int q = 0; q < N; q++) m = max(m, s[q]);
+        for (int q = 0; q < N; q++) m = m > s[q] ? m : s[q];
         if (m >= nslots) return false;
         if (died) {
             uint32_t d = 0;
@@ -286,7 +292,7 @@ struct Sources {
     __device__ __forceinline__ void four(uint32_t k, uint32_t e, uint64_t (&id)[4]) const {
 #pragma unroll
         for (uint32_t q = 0; q < 4; q++) {
-            const uint64_t j = k + q < e ? k + q : k;
+            const uint64_t j = q < e - k ? k + q : k;
             id[q] = src64 ? ((const uint64_t*)src)[j] : vh_make_id(type, ((const uint32_t*)src)[j]);
         }
         __builtin_amdgcn_s_waitcnt(0);

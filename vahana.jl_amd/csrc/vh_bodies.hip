@@ -40,12 +40,12 @@ struct Body<VH_TR_SUM_NEIGHBORS> {
             constexpr int SUM_N = 8;
             const uint8_t* n[SUM_N];
             uint32_t k = b;
-            for (; k < e && nb.some(k, e, n); k = e - k > SUM_N ? k + SUM_N : e) {
+            for (; k < e && nb.some(k, e, n); k = vh_row_next(k, e, SUM_N)) {
                 int64_t v[SUM_N];
 #pragma unroll
                 for (int q = 0; q < SUM_N; q++) v[q] = ld_i64(n[q]);
 #pragma unroll
-                for (int q = 0; q < SUM_N; q++) sum += k + q < e ? v[q] : 0;
+                for (uint32_t q = 0; q < SUM_N; q++) sum += q < e - k ? v[q] : 0;
             }
             for (; k < e; k++) {
                 const uint8_t* ns = nb.state(k);
@@ -119,7 +119,7 @@ struct Body<VH_TR_NEIGHBOR_FOO_EDGES> {
             uint8_t es[8];
             st_i64(es, foo);
             const Sources src(E);
-            for (uint32_t k = b; k < e; k += 4) {
+            for (uint32_t k = b; k < e; k = vh_row_next(k, e, 4)) {
                 uint64_t nid[4];
                 src.four(k, e, nid);
                 uint64_t f[8], t[8];

@@ -14,9 +14,9 @@
 // lookups of some lane of the wave, one after the other: the infections of
 // the 10^7-agent contact step took 162 us so, 68 us now.
 template <class F>
-__device__ __forceinline__ bool vh_any_infecting(uint64_t pre, uint64_t pt, uint32_t b, uint32_t e,
-                                                 F infected) {
-    for (uint32_t k = b; k < e; k += 32) {
+__host__ __device__ __forceinline__ bool vh_any_infecting(uint64_t pre, uint64_t pt, uint32_t b, uint32_t e,
+                                                          F infected) {
+    for (uint32_t k = b; k < e; k = vh_row_next(k, e, 32)) {
         const uint32_t cnt = e - k < 32u ? e - k : 32u;
         uint32_t m = 0;   // bit q: the draw of in-edge k + q is below p
         for (uint32_t q = 0; q < cnt; q += 4) {
@@ -56,10 +56,10 @@ __device__ __forceinline__ void vh_expose_wave(bool inf, uint64_t i, const uint3
         uint64_t t = m;   // its lowest bit: the agent of lane group g
         for (uint32_t q = 0; q < g; q++) t &= t ? t - 1ull : 0ull;
         const int who = t ? (int)__builtin_ctzll(t) : 0;
-        const uint32_t bb = (uint32_t)__shfl((int)b, who, 64), ee = (uint32_t)__shfl((int)e, who, 64);
+        const uint32_t bb = (uint32_t)__shfl((int)b, who, 64), d = (uint32_t)__shfl((int)(e - b), who, 64);
         if (t)
-            for (uint32_t k = bb + l; k < ee; k += 16) {
-                const uint32_t v = out_dst[k];
+            for (uint32_t k = l; k < d; k = vh_row_next(k, d, 16)) {
+                const uint32_t v = out_dst[bb + k];
                 atomicOr(bits + (v >> 5), 1u << (v & 31u));
             }
         for (uint32_t q = 0; q < 4; q++) m &= m ? m - 1ull : 0ull;
