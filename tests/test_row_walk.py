@@ -47,6 +47,18 @@ static void any(uint32_t b, uint32_t e) {
                 fail("any: one infected", b, e);
     }
 }
+// lane l's in-edges of a row: every 64th from its own on, in order
+static void lanes(uint32_t b, uint32_t e) {
+    for (uint32_t l = 0; l < 64; l++) {
+        uint64_t next = (uint64_t)b + l;
+        auto one = [&](uint32_t k) {
+            if (k != next || next >= e) fail("lane", b, e);
+            next += 64;
+        };
+        vh_lane_edges(b, e, l, [&](uint32_t k) { for (uint32_t q = 0; q < 4; q++) one(k + 64 * q); }, one);
+        if (next < e) fail("lane: ends early", b, e);
+    }
+}
 int main() {
     const size_t bytes = (size_t)1 << 34;
     uint32_t* src = (uint32_t*)mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
@@ -72,6 +84,8 @@ int main() {
             walk<64>(b, e);
             walk<256>(b, e);
             any(b, e);
+            lanes(b, e);
+            lanes(b - 5 * d, e);
             const uint8_t* p[8];
             for (uint32_t k = b; k < e; k = vh_row_next(k, e, 8)) {
                 if (!nb.some(k, e, p)) fail("some", b, e);

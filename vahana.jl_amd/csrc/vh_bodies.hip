@@ -614,14 +614,12 @@ __device__ __forceinline__ void opinion_heavy(const uint32_t* __restrict__ off,
                                               const uint32_t* __restrict__ src,
                                               const T* __restrict__ x, const float* __restrict__ w,
                                               T* __restrict__ xo, uint64_t r, uint64_t rowbase, T eps) {
-    const int lane = threadIdx.x & 63;
+    const uint32_t lane = threadIdx.x & 63u;
     const uint64_t i = r - rowbase;
     const T xi = x[i];
-    const uint32_t b = off[r], e = off[r + 1];
     T num = (T)0, den = (T)0;
     // lane l adds k = l, l+64, ... in order; four strides in flight per lane
-    uint32_t k = b + lane;
-    for (; k + 192 < e; k += 256) {
+    auto four = [&](uint32_t k) {
         const uint32_t s0 = src[k], s1 = src[k + 64], s2 = src[k + 128], s3 = src[k + 192];
         const float w0 = w[k], w1 = w[k + 64], w2 = w[k + 128], w3 = w[k + 192];
         const T x0 = x[s0 - 1], x1 = x[s1 - 1], x2 = x[s2 - 1], x3 = x[s3 - 1];
@@ -629,8 +627,8 @@ __device__ __forceinline__ void opinion_heavy(const uint32_t* __restrict__ off,
         op_accum(x1, w1, xi, eps, num, den);
         op_accum(x2, w2, xi, eps, num, den);
         op_accum(x3, w3, xi, eps, num, den);
-    }
-    for (; k < e; k += 64) op_accum(x[src[k] - 1], w[k], xi, eps, num, den);
+    };
+    vh_lane_edges(off[r], off[r + 1], lane, four, [&](uint32_t k) { op_accum(x[src[k] - 1], w[k], xi, eps, num, den); });
     num = xor_butterfly(num);
     den = xor_butterfly(den);
     if (lane == 0) xo[i] = den > (T)0 ? num / den : xi;
@@ -749,7 +747,7 @@ __device__ __forceinline__ void opinion_heavy_plan(const T* __restrict__ x, cons
     const uint32_t b = hi.y, d = hi.z, hb = hi.w;
     const T xi = x[r];
     T num = (T)0, den = (T)0;
-    for (uint32_t c0 = 0; c0 < d; c0 += CH) {
+    for (uint32_t c0 = 0; c0 < d; c0 = vh_row_next(c0, d, CH)) {
         const uint32_t cnt = d - c0 < CH ? d - c0 : CH;
         float wq[HU];
         uint32_t jj[HU], sl[HU];
@@ -1473,7 +1471,7 @@ __global__ __launch_bounds__(256) void k_heavy_keys(const uint32_t* __restrict__
     if (h >= nheavy) return;
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t r = heavy[h], b = off[r], d = off[r + 1] - b, hb = hbase[h], cb = cbase[h];
-    for (uint32_t t = lane; t < d; t += 64) {
+    for (uint32_t t = lane; t < d; t = vh_row_next(t, d, 64)) {
         keys[hb + t] = ((cb + t / chunk) << pbits) | ((src[b + t] - 1u) / psize);
         kidx[hb + t] = b + t;
         tsl[hb + t] = (uint16_t)(t % chunk);

@@ -37,6 +37,15 @@ __host__ __device__ __forceinline__ bool vh_any_infecting(uint64_t pre, uint64_t
     }
     return false;
 }
+// The in-edges k = b + l, b + l + 64, ... of row [b, e) that lane l of a wave
+// takes, in order: four(k) for k, k + 64, k + 128 and k + 192, then one(k).
+template <class F4, class F1>
+__host__ __device__ __forceinline__ void vh_lane_edges(uint32_t b, uint32_t e, uint32_t lane, F4 four, F1 one) {
+    const uint32_t d = e - b;
+    uint32_t t = lane;
+    for (; t < d && d - t > 192u; t = vh_row_next(t, d, 256)) four(b + t);
+    for (; t < d; t = vh_row_next(t, d, 64)) one(b + t);
+}
 // The exposure of a wave's infected agents (every lane of the wave calls; inf:
 // the lane's agent i is to be marked from): the bit of each of their
 // out-neighbours is set in `bits`. Four agents at a time, 16 lanes each: the
