@@ -458,10 +458,11 @@ int vh_set_options(const vh_options* in);
  * with asserts off apply! stays asynchronous unless it has births or deaths */
 int vh_enable_asserts(int enable);
 /* test hooks (no reference counterpart): the next n device allocations of
- * the library fail as out of memory (an injected allocation failure); OR
- * `flags` into a simulation's device error word, as a failing body would
+ * the library fail as out of memory (an injected allocation failure), or the
+ * n that follow the next `after` of them; OR `flags` into a simulation's device error word, as a failing body would
  * (an injected device error: the next checked apply! reports it) */
 int vh_debug_fail_allocs(uint32_t n);
+int vh_debug_fail_allocs_after(uint32_t after, uint32_t n);
 int vh_debug_set_device_error(vh_sim_t sim, uint32_t flags);
 
 /* ------------------------------------------------------ ensembles

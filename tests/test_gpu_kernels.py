@@ -408,3 +408,87 @@ def test_ensemble_long_runs(vh, ora, gpu_ready, opts, block, apt):
     check([37, 37, 29, 37, 37])
     E.step(23)
     check([60, 60, 52, 60, 60])
+
+
+def _edge_list(sim, E, state):
+    t, f, s = sim._read_edges(E)
+    return [np.array(t), np.array(f), np.ascontiguousarray(s).view(np.uint8).copy() if state else np.zeros(0)]
+
+
+@pytest.mark.parametrize("hints", [(), ("SingleEdge",)], ids=["plain", "single"])
+def test_edge_rebuild_out_of_memory(vh, ora, gpu_ready, hints):
+    """Each device allocation of a rebuild with more rows and edges fails
+    once: the edges are then the old ones, or none where a buffer had grown,
+    and the same call afterwards gives the checker's edges."""
+    n = 300
+    fr, to = _ragged_edges(n, 5)
+
+    def build(V):
+        A, E, F = V.struct("A", [("foo", "<i8")]), V.struct("E"), V.struct("F", [("foo", "<i8")])
+        kw = {} if "SingleEdge" in hints else {"target": A}
+        model = (V.ModelTypes() | V.register_agenttype_(A) | V.register_edgetype_(E, "Stateless", target=A)
+                 | V.register_edgetype_(F, *hints, **kw) | V.create_model("oom"))
+        sim = V.create_simulation(model)
+        st = np.zeros(n, dtype=A.dtype)
+        st["foo"] = np.arange(n)
+        sim._add_agents_array(A, st)
+        sim._add_edges_array(E, fr, to)
+        V.finish_init_(sim)
+        V.apply_(sim, V.transitions.add_self_edge(F, state=np.array([7], "<i8")), A, A, F)
+        V.apply_(sim, V.transitions.spawn(A, 4, E), A, [A, E], [A, E], add_existing=E)
+        body = (V.transitions.add_self_edge(F, state=np.array([9], "<i8")) if hints
+                else V.transitions.neighbor_foo_edges(E, F, -1))
+        return sim, A, E, F, lambda: V.apply_(sim, body, A, [A, E], F)
+
+    csim, _, _, cF, step = build(ora)
+    step()
+    want = _edge_list(csim, cF, True)
+    lib, failed, emptied = vh._abi.lib(), 0, 0
+    for after in range(100):
+        sim, A, E, F, step = build(vh)
+        old = _edge_list(sim, F, True)
+        assert len(old[0]) == n
+        lib.debug_fail_allocs_after(after, 1)
+        try:
+            step()
+            break
+        except vh.VahanaError as err:
+            assert err.code == vh._abi.VH_ERR_OOM, after
+        finally:
+            lib.debug_fail_allocs(0)
+        failed += 1
+        now = _edge_list(sim, F, True)
+        empty = len(now[0]) == 0
+        emptied += empty
+        assert empty or all(np.array_equal(a, b) for a, b in zip(now, old)), after
+        step()
+        for a, b in zip(_edge_list(sim, F, True), want):
+            assert np.array_equal(a, b), after
+    print(f"[gpu] {failed} allocations failed, {emptied} of them with the edges gone", flush=True)
+    assert 0 < emptied < failed < 100
+
+
+@pytest.mark.parametrize("C", [9, 40], ids=["masks", "log"])
+def test_contact_rebuild_out_of_memory(vh, gpu_ready, C):
+    """Each device allocation of a contact step with more contacts and newborn
+    slots fails once: the contacts are the old ones or none."""
+    M, lib = vh.models, vh._abi.lib()
+    failed, emptied = 0, 0
+    for after in range(100):
+        m = M.build_contact(vh, 3000, seed=9, n_init=600)
+        M.step_contact(vh, m, seed=9, beta=0.3, p_death=0.0, n_contacts=2)
+        old = _edge_list(m.sim, m.E, False)
+        lib.debug_fail_allocs_after(after, 1)
+        try:
+            M.step_contact(vh, m, seed=9, beta=0.3, p_death=0.3, n_contacts=C)
+            break
+        except vh.VahanaError as err:
+            assert err.code == vh._abi.VH_ERR_OOM, after
+        finally:
+            lib.debug_fail_allocs(0)
+        failed += 1
+        now = _edge_list(m.sim, m.E, False)
+        emptied += len(now[0]) == 0
+        assert len(now[0]) == 0 or all(np.array_equal(a, b) for a, b in zip(now, old)), after
+    print(f"[gpu] {failed} allocations failed, {emptied} of them with the contacts gone", flush=True)
+    assert 0 < emptied < failed < 100

@@ -1831,14 +1831,16 @@ __global__ __launch_bounds__(256) void k_contact_main_log(const uint64_t* __rest
     kept[i] = nk;
     died_now[i] = cbit(B.sp, i) && !cbit(B.dead, i);
 }
-// the CSR from the log
+// the CSR from the log (pos: the scan of `kept`)
 __global__ __launch_bounds__(256) void k_contact_edges_log(uint64_t n, uint32_t C, const uint32_t* __restrict__ kept,
                                                            const uint32_t* __restrict__ log,
-                                                           const uint32_t* __restrict__ off,
-                                                           uint32_t* __restrict__ src) {
+                                                           const uint32_t* __restrict__ pos,
+                                                           uint32_t* __restrict__ off, uint32_t* __restrict__ src) {
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const uint32_t k = kept[i], o = off[i];
+    const uint32_t k = kept[i], o = pos[i];
+    off[i] = o;
+    if (i == n - 1) off[n] = o + k;
     for (uint32_t r = 0; r < k; r++) src[o + r] = log[i * C + r];
 }
 
@@ -2770,8 +2772,10 @@ int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t st
     uint32_t* dpos = (uint32_t*)s.scratch.take((2 * nw + 1) * 4 + 8);
     uint2* masks = masked ? (uint2*)s.scratch.take(n * 8 + 8) : nullptr;
     uint32_t* kept = masked ? nullptr : (uint32_t*)s.scratch.take(n * 4 + 8);
+    uint32_t* kpos = masked ? nullptr : (uint32_t*)s.scratch.take((n + 1) * 4 + 8);
     uint32_t* log = masked ? nullptr : (uint32_t*)s.scratch.take(n * C * 4 + 8);
-    if (!B.sp || !B.dead || !B.inf || !B.sus || !B.cnt || (fwords && !B.filt) || !dpos || (masked ? !masks : !kept || !log))
+    if (!B.sp || !B.dead || !B.inf || !B.sus || !B.cnt || (fwords && !B.filt) || !dpos ||
+        (masked ? !masks : !kept || !kpos || !log))
         return set_error(VH_ERR_OOM, "scratch");
     uint64_t nd = 0, ne = 0;
     if (n) {
@@ -2806,9 +2810,8 @@ int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t st
                                (uint64_t*)A.wstate(), A.died_now.as<uint8_t>(), (uint32_t)n, (uint32_t)t, p, step, B, kept,
                                log);
             HIPCHECK(hipGetLastError());
-            RC(E.off.ensure((n + 1) * 4 + 8, st));
-            if (scan_excl_u32(kept, E.off.as<uint32_t>(), n, s.scratch, st)) return set_error(VH_ERR_DEVICE, "scan");
-            total = E.off.as<uint32_t>() + n;
+            if (scan_excl_u32(kept, kpos, n, s.scratch, st)) return set_error(VH_ERR_DEVICE, "scan");
+            total = kpos + n;
         }
         HIPCHECK(hipMemcpyAsync((uint32_t*)s.d_stats.p, dpos + nw, 4, hipMemcpyDeviceToDevice, st));
         HIPCHECK(hipMemcpyAsync((uint32_t*)s.d_stats.p + 1, total, 4, hipMemcpyDeviceToDevice, st));
@@ -2837,14 +2840,13 @@ int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t st
     }
     // rows = caller slots; rows of dead callers and of newborns are empty
     uint64_t rows = std::max(n, A.nextid - 1);
-    RC(E.off.ensure((rows + 1) * 4 + 8, st, masked ? 0 : (n + 1) * 4));
-    RC(E.src.ensure(ne * 4 + 8, st));
+    RC(edge_room(E, (rows + 1) * 4 + 8, ne * 4 + 8, 0, st));
     if (!n) fill_u32(E.off.as<uint32_t>(), 0, 1, st);
     else if (masked)
         hipLaunchKernelGGL(k_contact_edges, dim3((unsigned)nblk), dim3(256), 256 * C * 4, st, (uint32_t)n, (uint32_t)t,
                            p, step, B, masks, dpos, E.off.as<uint32_t>(), E.src.as<uint32_t>());
-    else if (ne)
-        hipLaunchKernelGGL(k_contact_edges_log, dim3((unsigned)nblk), dim3(256), 0, st, n, C, kept, log,
+    else
+        hipLaunchKernelGGL(k_contact_edges_log, dim3((unsigned)nblk), dim3(256), 0, st, n, C, kept, log, kpos,
                            E.off.as<uint32_t>(), E.src.as<uint32_t>());
     if (rows > n)
         hipLaunchKernelGGL(k_contact_extend, dim3(grid_for(rows - n, 256)), dim3(256), 0, st,

@@ -252,6 +252,7 @@ constexpr uint32_t CTX_SLOTS = 8;
 // engine services the bodies use
 int readback(Sim& s, int n);                           // d_stats -> h_stats, synchronous
 int ensure_slots(Sim& s, int t, uint64_t slots);
+int edge_room(EdgeStore& E, size_t off, size_t src, size_t states, hipStream_t st);
 // degree bins for the opinion kernels
 int build_heavy_bins(Sim& s, EdgeStore& E, int t);
 

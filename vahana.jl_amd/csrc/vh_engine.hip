@@ -144,6 +144,10 @@ extern "C" int vh_debug_fail_allocs(uint32_t n) {
     fail_next_allocs(n);
     return VH_OK;
 }
+extern "C" int vh_debug_fail_allocs_after(uint32_t after, uint32_t n) {
+    fail_next_allocs(n, after);
+    return VH_OK;
+}
 extern "C" int vh_debug_set_device_error(vh_sim_t h, uint32_t flags) {
     if (!h) return set_error(VH_ERR_ARG, "null simulation");
     Sim& s = h->s;
@@ -711,6 +715,23 @@ int vh::readback(Sim& s, int n) {
     return wait_stream(s);
 }
 
+// Memory for a rebuilt CSR: bytes of offsets, sources and states (0: not
+// used); what a buffer holds is dropped when it grows. When that fails after
+// one of them has grown, the old offsets and sources are no longer one CSR:
+// the store is then left as never built, without rows and edges.
+int vh::edge_room(EdgeStore& E, size_t off, size_t src, size_t states, hipStream_t st) {
+    const void *off0 = E.off.p, *src0 = E.src.p;
+    int rc = E.off.ensure(off, st);
+    if (!rc && src) rc = E.src.ensure(src, st);
+    if (!rc && states) rc = E.st.ensure(states, st);
+    if (rc && (E.off.p != off0 || E.src.p != src0)) {
+        for (int t = 0; t <= VH_MAXA; t++) E.rowbase[t] = E.nrows[t] = 0;
+        E.rows = E.nedges = 0;
+        E.version++;
+    }
+    return rc;
+}
+
 // Build the CSR of E from (optionally) its current entries followed by `nlog`
 // log entries (to, from, states) in add_edge! order: a stable sort by target
 // row keeps, per target, the existing edges first and the new ones in call
@@ -812,9 +833,7 @@ static int build_csr(Sim& s, EdgeStore& E, bool keep_base, const uint64_t* d_to,
         }
     } else {
         const uint32_t srcw = ignorefrom ? 0u : E.src64 ? 8u : 4u;
-        RC(E.off.ensure((rows + 1) * 4, st));
-        if (srcw) RC(E.src.ensure(n * srcw + 8, st));
-        if (bytes) RC(E.st.ensure(n * bytes + 8, st));
+        RC(edge_room(E, (rows + 1) * 4, srcw ? n * srcw + 8 : 0, bytes ? n * bytes + 8 : 0, st));
         off = E.off.as<uint32_t>();
         place_entries(order, n, from, E.src.p, srcw, sts, E.st.p, bytes, st);
     }
@@ -875,11 +894,9 @@ static int build_csr(Sim& s, EdgeStore& E, bool keep_base, const uint64_t* d_to,
         nfinal = (uint32_t)s.h_stats[0];
     }
     if (filtered) {   // into the store
-        RC(E.off.ensure((rows + 1) * 4, st));
-        HIPCHECK(hipMemcpyAsync(E.off.p, off, (rows + 1) * 4, hipMemcpyDeviceToDevice, st));
         const uint32_t srcw = ignorefrom ? 0u : E.src64 ? 8u : 4u;
-        if (srcw) RC(E.src.ensure(nfinal * srcw + 8, st));
-        if (bytes) RC(E.st.ensure(nfinal * bytes + 8, st));
+        RC(edge_room(E, (rows + 1) * 4, srcw ? nfinal * srcw + 8 : 0, bytes ? nfinal * bytes + 8 : 0, st));
+        HIPCHECK(hipMemcpyAsync(E.off.p, off, (rows + 1) * 4, hipMemcpyDeviceToDevice, st));
         place_entries(nullptr, nfinal, from_s, E.src.p, srcw, st_s, E.st.p, bytes, st);
     }
     for (int t = 0; t <= VH_MAXA; t++) {

@@ -9,15 +9,20 @@
 namespace vh {
 
 // ------------------------------------------------------------------ arena
-// every device allocation of the library; a test hook makes the next n fail
-static std::atomic<uint32_t> g_fail_allocs{0};
+// every device allocation of the library; a test hook makes some fail: `after`
+// (high word) go through, then n (low word) fail
+static std::atomic<uint64_t> g_fail_allocs{0};
 hipError_t device_alloc(void** p, size_t bytes) {
-    uint32_t k = g_fail_allocs.load();
-    while (k > 0)
-        if (g_fail_allocs.compare_exchange_weak(k, k - 1)) return hipErrorOutOfMemory;
+    uint64_t k = g_fail_allocs.load();
+    while (k & 0xFFFFFFFFull) {
+        const bool ok = k >> 32 != 0;
+        if (!g_fail_allocs.compare_exchange_weak(k, ok ? k - (1ull << 32) : k - 1)) continue;
+        if (ok) break;
+        return hipErrorOutOfMemory;
+    }
     return hipMalloc(p, bytes);
 }
-void fail_next_allocs(uint32_t n) { g_fail_allocs.store(n); }
+void fail_next_allocs(uint32_t n, uint32_t after) { g_fail_allocs.store((uint64_t)after << 32 | n); }
 
 void* Scratch::take(size_t bytes) {
     bytes = (bytes + 255) & ~(size_t)255;
