@@ -160,3 +160,46 @@ def test_ensemble_1024_replicas_config3(vh, gpu_ready):
         assert np.array_equal(np.ascontiguousarray(got).view(np.uint8),
                               _solo(vh, n, md, p, seed, 10_000 + seed, 6, max(1, n // 1000))), f"member {k} n={n}"
     E.close()
+
+
+def test_ensemble_memory_without_the_pass(vh, gpu_ready, opts):
+    """A member of an ensemble below sir_expose_min holds no out-edges (84 of
+    176 MB here)."""
+    import torch
+    opts(sir_expose=1, sir_expose_min=10 ** 9)
+    E = vh.ensemble.Ensemble()
+    before = torch.cuda.mem_get_info()[0]
+    E.add_sir(1_000_000, 20.0, 0.05, 51, 501)
+    held = before - torch.cuda.mem_get_info()[0]
+    info = E.info()
+    print(f"[gpu] {held / 1e6:.0f} MB held, states and in-edges {info['bytes'] / 1e6:.0f}", flush=True)
+    assert 90e6 < info["bytes"] < 95e6
+    assert held < info["bytes"] + 4 * info["edges"] / 2   # (generator scratch: 8 MB)
+    E.step(2)
+    E.close()
+
+
+def test_ensemble_add_without_room_for_out_edges(vh, gpu_ready, opts):
+    """Each device allocation of an add fails once: the member is refused and
+    the others go on, or it is there (its out-edges' memory taken later)."""
+    opts(sir_expose=1, sir_expose_min=1000)
+    lib = vh._abi.lib()
+    specs = [(3000, 8.0, 0.06, 61, 601), (2000, 12.0, 0.05, 62, 602)]
+    want = [_solo(vh, n, md, p, s, g, 6, n // 50) for n, md, p, s, g in specs]
+    added = 0
+    for after in range(8):
+        E = vh.ensemble.Ensemble()
+        ids = [E.add_sir(*specs[0], recovery=7, n_init=specs[0][0] // 50)]
+        lib.debug_fail_allocs_after(after, 1)
+        try:
+            ids.append(E.add_sir(*specs[1], recovery=7, n_init=specs[1][0] // 50))
+            added += 1
+        except RuntimeError as err:
+            assert f"[{vh._abi.VH_ERR_OOM}]" in str(err), after
+        finally:
+            lib.debug_fail_allocs(0)
+        E.step(6)
+        for mid, w in zip(ids, want):
+            assert np.array_equal(np.ascontiguousarray(E.read(mid)[0]).view(np.uint8), w), after
+        E.close()
+    assert added > 0

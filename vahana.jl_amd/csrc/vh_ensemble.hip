@@ -613,7 +613,7 @@ struct Member {
     uint32_t rec;
     // one allocation for all of a member's device memory (a buffer each was
     // seven allocations and frees, 17 and 58 us each): states, in-edge CSR and,
-    // unless the exposure pass is off, out-edges and the two exposure bitmaps
+    // where the exposure pass runs with it, out-edges and the two exposure bitmaps
     DevBuf buf;
     DevBuf out_buf;                  // out-edges and bitmaps when `buf` was taken without them
     uint32_t *off = nullptr, *src = nullptr, *st[2] = {nullptr, nullptr};
@@ -674,6 +674,15 @@ struct vh_ensemble {
     Scratch scratch;
     DevBuf d_cdf;
 };
+
+// exposure pass unless the options turn it off, for ensembles of at least
+// sir_expose_min agents (default 65536: below, its two extra launches per
+// step cost more than the draws it saves)
+static bool expose_runs(const vh_ensemble* e, uint64_t more) {
+    uint64_t total = more;
+    for (auto& kv : e->members) total += kv.second->n;
+    return g_opts.sir_expose != 0 && (int64_t)total >= g_opts.sir_expose_min;
+}
 
 static int pinned(void** p, size_t* cap, size_t bytes) {
     if (bytes <= *cap) return VH_OK;
@@ -875,8 +884,9 @@ extern "C" int vh_ensemble_add_sir(vh_ensemble_t e, const vh_sir_member* sm, uin
     m->nw = (m->n + 31) / 32;
     const size_t sb = Member::pad(sm->n * 4), ob = Member::pad(sm->n * 4 + 4);
     m->bytes = 2 * sb + ob + Member::pad(ne * 4);
-    const bool out = g_opts.sir_expose != 0;
-    if (!rc) rc = m->buf.ensure(m->bytes + (out ? m->out_bytes() : 0), st);
+    bool out = expose_runs(e, sm->n);
+    if (!rc && out && m->buf.ensure(m->bytes + m->out_bytes(), st)) out = false;   // (the first step asks again)
+    if (!rc && !out) rc = m->buf.ensure(m->bytes, st);
     if (!rc) {
         uint8_t* p = m->buf.as<uint8_t>();
         m->st[0] = (uint32_t*)p;
@@ -951,13 +961,9 @@ extern "C" int vh_ensemble_step(vh_ensemble_t e, uint32_t steps, int use_graph) 
     }
     if (!table_current(e)) RC(build_table(e));
     size_t nm = e->members.size();
-    // exposure pass unless the options turn it off, for ensembles of at
-    // least sir_expose_min agents (default 65536: below, its two extra
-    // launches per step cost more than the draws it saves); the members'
-    // out-edges are built on the first such step, on the step stream
-    uint64_t total = 0;
-    for (auto& kv : e->members) total += kv.second->n;
-    const bool expose = g_opts.sir_expose != 0 && (int64_t)total >= g_opts.sir_expose_min;
+    // the members' out-edges are built on the first step with the exposure
+    // pass, on the step stream
+    const bool expose = expose_runs(e, 0);
     if (expose) {
         RC(build_members_out(e));
         // the bitmaps and counts were not kept while the pass was off: every
