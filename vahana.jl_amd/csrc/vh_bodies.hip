@@ -2031,11 +2031,11 @@ constexpr uint32_t ROW_R = 2;   // rows of a wave
 struct RowSpec {
     int32_t dims[4];
     uint32_t periodic, nst;                            // nst: a multiple of ROW_U (padded with zero offsets)
-    int32_t reach;                                     // largest |offset| along dimension 0
     uint32_t off[VH_STENCIL_MAX];                      // four signed bytes in a word
 };
 // 8 bytes at any address: three words from the word they start in and a byte
-// shift. Reads up to 3 bytes past them.
+// shift. Reads up to 4 bytes past them (at an address that is a multiple of 4;
+// the last group of the last row reads them behind the cells).
 typedef uint32_t u32x3 __attribute__((ext_vector_type(3), aligned(4)));
 __device__ __forceinline__ uint64_t ld8(const uint8_t* p) {
     const uint32_t m = (uint32_t)(uintptr_t)p & 3u;
@@ -2678,29 +2678,29 @@ int launch_diffuse_stencil(Sim& s, int t, int et, uint32_t field) {
     uint64_t ncells = 1;
     for (uint32_t d = 0; d < sp.ndims; d++) ncells *= (uint64_t)sp.dims[d];
     if (!A.nslots) return VH_OK;
-    // rows of 8-cell groups: one-byte records, every slot a cell, rows of at
-    // least 16 cells (every 8-byte load stays inside its row), offsets of at
-    // most 7 cells along dimension 0 (one wrap, one partial group) and of at
-    // most the extent along the others (one wrap), and a grid within its
-    // limits; the rest takes the kernel that works cell by cell
+    // rows of 8-cell groups: one-byte records, every slot a cell, a buffer with
+    // the 4 bytes behind the cells that ld8 may read (ensure_slots leaves 8),
+    // rows of at least 16 cells (every 8-cell window lies in its row), offsets
+    // of at most 7 cells along dimension 0 (one wrap, one partial group) and of
+    // at most the extent along the others (one wrap), and at most 128000 rows:
+    // 17 500 blocks in y, of the grid's 65 535, which more than 479 000 rows
+    // would pass (between the two, both kernels are possible and only the one
+    // that works cell by cell is used); the rest takes that kernel
     const uint64_t nx = (uint64_t)sp.dims[0], nrows = ncells / nx;
     bool rows = A.bytes == 1 && field == 0 && sp.first_nr == 1 && ncells == A.nslots && ncells <= 0x7FFFFFFFull &&
-                nx >= 16 && nrows <= 128000;
+                A.state[A.rd].cap >= ncells + 4 && nx >= 16 && nrows <= 128000;
     RowSpec rsp;
     rsp.periodic = sp.periodic;
-    rsp.reach = 0;
     for (uint32_t d = 0; d < 4; d++) rsp.dims[d] = d < sp.ndims ? (int32_t)sp.dims[d] : 1;
     memset(rsp.off, 0, sizeof rsp.off);
     for (uint32_t k = 0; k < sp.nst && rows; k++) {
-        const int dx = std::abs((int)sp.off[k][0]);
-        rows = dx <= 7;
+        rows = std::abs((int)sp.off[k][0]) <= 7;
         for (uint32_t d = 1; d < 4; d++) rows = rows && std::abs((int)sp.off[k][d]) <= rsp.dims[d];
         memcpy(&rsp.off[k], sp.off[k], 4);
-        rsp.reach = std::max(rsp.reach, dx);
     }
     rsp.nst = (sp.nst + ROW_U - 1) / ROW_U * ROW_U;
     if (rows) {
-        // the blocks of 64 groups by 4 rows, then those of the end groups
+        // the blocks of 64 groups by 8 rows, then those of the end groups
         const unsigned gx = grid_for((nx + 7) / 8, 64), gy = grid_for(nrows, 4 * ROW_R);
         const unsigned ey = grid_for(3 * nrows, 256 * gx);
         hipLaunchKernelGGL(k_diffuse_rows, dim3(gx, gy + ey), dim3(256), 0, s.stream, rsp,
