@@ -460,10 +460,14 @@ int vh_enable_asserts(int enable);
 /* test hooks (no reference counterpart): the next n device allocations of
  * the library fail as out of memory (an injected allocation failure), or the
  * n that follow the next `after` of them; OR `flags` into a simulation's device error word, as a failing body would
- * (an injected device error: the next checked apply! reports it) */
+ * (an injected device error: the next checked apply! reports it); give the
+ * contact step's filter of dead partners at most `bytes` of LDS (0: the
+ * default, all of a CU's 160 KiB), which takes small simulations through the
+ * group sizes of large ones */
 int vh_debug_fail_allocs(uint32_t n);
 int vh_debug_fail_allocs_after(uint32_t after, uint32_t n);
 int vh_debug_set_device_error(vh_sim_t sim, uint32_t flags);
+int vh_debug_contact_filter(uint32_t bytes);
 
 /* ------------------------------------------------------ ensembles
  * Many independent SIR simulations advanced by one segmented launch per

@@ -492,3 +492,26 @@ def test_contact_rebuild_out_of_memory(vh, gpu_ready, C):
         assert len(now[0]) == 0 or all(np.array_equal(a, b) for a, b in zip(now, old)), after
     print(f"[gpu] {failed} allocations failed, {emptied} of them with the contacts gone", flush=True)
     assert 0 < emptied < failed < 100
+
+
+@pytest.mark.parametrize("n", [4999, 5120])
+@pytest.mark.parametrize("shift", range(7))
+def test_contact_filter_groups(vh, ora, gpu_ready, shift, n):
+    """Filter groups of 1, 2, 4, ..., 32 slots and, past them, no filter: 20
+    blocks of 256 slots (25 with newborns at most), whose bits fit the limit
+    from that group size on. Many deaths, so that a group without its mark
+    would keep dead partners."""
+    M, lib = vh.models, vh._abi.lib()
+    g, c = (M.build_contact(V, n, seed=4, n_init=n // 5) for V in (vh, ora))
+    lib.debug_contact_filter(800 >> shift)
+    try:
+        for k in range(4):
+            for V, m in ((vh, g), (ora, c)):
+                M.step_contact(V, m, seed=4, beta=0.3, p_death=0.05, n_contacts=6)
+            (a, da), (b, db) = _states(g.sim, g.T), _states(c.sim, c.T)
+            assert np.array_equal(da, db), k
+            assert np.array_equal(a[~da], b[~db]), k
+            for x, y in zip(g.sim._read_edges(g.E)[:2], c.sim._read_edges(c.E)[:2]):
+                assert np.array_equal(x, y), k
+    finally:
+        lib.debug_contact_filter(0)

@@ -8,6 +8,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 
 #include "vh_engine.h"
 
@@ -2737,6 +2738,10 @@ int stencil_csr(Sim& s, EdgeStore& E, uint64_t rowbase, uint64_t rows) {
     return VH_OK;
 }
 
+constexpr uint32_t CONTACT_FILTER = 163840;
+static std::atomic<uint32_t> g_contact_filter{CONTACT_FILTER};   // (less in tests)
+void set_contact_filter(uint32_t bytes) { g_contact_filter = bytes && bytes < CONTACT_FILTER ? bytes : CONTACT_FILTER; }
+
 // One apply! of the contact model: flags, health update with the kept
 // partners logged, one readback (deaths, contacts), newborns and deaths on
 // the reuse stack, then the contact CSR rebuilt in place from the log (its
@@ -2761,7 +2766,7 @@ int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t st
     B.nwords = nw;
     B.fshift = 0;
     B.filt = nullptr;
-    while ((nblk * 32) >> B.fshift > 163840) B.fshift++;
+    while ((nblk * 32) >> B.fshift > g_contact_filter) B.fshift++;
     const uint32_t fwords = masked && n && B.fshift <= 5 ? (uint32_t)((((nblk * 32) >> B.fshift) + 15) / 16 * 4) : 0u;
     B.sp = (uint64_t*)s.scratch.take(nw * 8 + 8);
     B.dead = (uint64_t*)s.scratch.take(nw * 8 + 8);
@@ -2790,7 +2795,7 @@ int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t st
             // their filters fit
             const uint32_t cus = device_cus(), fb = fwords * 4;
             const bool big = n >= 1024ull * cus || !fwords;
-            const uint32_t bs = big ? 1024u : 256u, fit = std::max(1u, std::min(2048u / bs, fb ? 163840u / fb : 32u));
+            const uint32_t bs = big ? 1024u : 256u, fit = std::max(1u, std::min(2048u / bs, fb ? CONTACT_FILTER / fb : 32u));
             const dim3 g((unsigned)std::min<uint64_t>((n + bs - 1) / bs, (uint64_t)cus * fit));
             auto launch = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, g, dim3(bs), fb, st, (const uint64_t*)A.rstate(), (uint64_t*)A.wstate(),

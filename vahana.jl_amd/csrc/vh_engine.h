@@ -209,6 +209,7 @@ struct ContactBits {
 };
 // one apply! of the contact model incl. its births, deaths and contact CSR
 int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t step, uint64_t* ndeaths);
+void set_contact_filter(uint32_t bytes);   // LDS of its filter at most (0: the default)
 // device G(n, p) CSR in target order (vh_ensemble.hip): off[n + 1], sources as
 // 1-based numbers; one host synchronisation (in gnp_degrees)
 int gnp_degrees(uint64_t n, double mean_deg, uint64_t seed, uint32_t* off, DevBuf& cdf, Scratch& sc,

@@ -148,6 +148,10 @@ extern "C" int vh_debug_fail_allocs_after(uint32_t after, uint32_t n) {
     fail_next_allocs(n, after);
     return VH_OK;
 }
+extern "C" int vh_debug_contact_filter(uint32_t bytes) {
+    set_contact_filter(bytes);
+    return VH_OK;
+}
 extern "C" int vh_debug_set_device_error(vh_sim_t h, uint32_t flags) {
     if (!h) return set_error(VH_ERR_ARG, "null simulation");
     Sim& s = h->s;
