@@ -515,3 +515,18 @@ def test_contact_filter_groups(vh, ora, gpu_ready, shift, n):
                 assert np.array_equal(x, y), k
     finally:
         lib.debug_contact_filter(0)
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_opinion_one_pass_beyond_the_caches(vh, gpu_ready, opts, f32):
+    """One simulation whose edges are more than 256 MB, gathered in one pass
+    (its edges read past the caches) against the two-pass gather."""
+    got = []
+    for plan in (-1, 0):
+        opts(opinion_plan_bytes=plan)
+        m = vh.models.build_opinion_gnp(vh, 3_800_001, mean_deg=9.0, seed=3, graph_seed=23, weight_seed=43, f32=f32)
+        assert vh.num_edges(m.sim, m.E) * 8 > 256 << 20
+        for _ in range(2):
+            vh.models.step_opinion(vh, m, eps=0.3)
+        got.append(_states(m.sim, m.T)[0].copy())
+    assert np.array_equal(*got)
