@@ -56,16 +56,17 @@ __device__ __forceinline__ void vh_expose_wave(bool inf, uint64_t i, const uint3
     uint64_t m = __ballot(inf);
     if (!m) return;
     const uint32_t lane = threadIdx.x & 63u, g = lane >> 4, l = lane & 15u;
-    uint32_t b = 0, e = 0;
+    uint32_t b = 0, n = 0;
     if (inf) {
         b = out_off[i];
-        e = out_off[i + 1];
+        const uint32_t e = out_off[i + 1];
+        n = e > b ? e - b : 0u;   // (sources past the agents leave the offsets in no order: no walk then)
     }
     while (m) {
         uint64_t t = m;   // its lowest bit: the agent of lane group g
         for (uint32_t q = 0; q < g; q++) t &= t ? t - 1ull : 0ull;
         const int who = t ? (int)__builtin_ctzll(t) : 0;
-        const uint32_t bb = (uint32_t)__shfl((int)b, who, 64), d = (uint32_t)__shfl((int)(e - b), who, 64);
+        const uint32_t bb = (uint32_t)__shfl((int)b, who, 64), d = (uint32_t)__shfl((int)n, who, 64);
         if (t)
             for (uint32_t k = l; k < d; k = vh_row_next(k, d, 16)) {
                 const uint32_t v = out_dst[bb + k];
