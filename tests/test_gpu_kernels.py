@@ -530,3 +530,26 @@ def test_opinion_one_pass_beyond_the_caches(vh, gpu_ready, opts, f32):
             vh.models.step_opinion(vh, m, eps=0.3)
         got.append(_states(m.sim, m.T)[0].copy())
     assert np.array_equal(*got)
+
+
+@pytest.mark.parametrize("body", ["sum", "foo_edges", "diffuse", "move_to"])
+def test_bodies_need_sources(vh, gpu_ready, body):
+    """A body that asks an :IgnoreFrom type for its neighbours fails with the
+    reference's assertion (the type keeps no sources to look at)."""
+    n = 64
+    A, E, F = vh.struct("A", [("foo", "<i8"), ("active", "?")]), vh.struct("E"), vh.struct("F", [("foo", "<i8")])
+    model = (vh.ModelTypes() | vh.register_agenttype_(A, "Immortal") | vh.register_edgetype_(E, "Stateless", "IgnoreFrom")
+             | vh.register_edgetype_(F) | vh.create_model("sources"))
+    sim = vh.create_simulation(model)
+    st = np.zeros(n, dtype=A.dtype)
+    st["foo"] = np.arange(n)
+    vh.raster.add_raster_(sim, "r", (8, 8), st, T=A)
+    ids = (np.uint64(1) << np.uint64(56)) | np.arange(1, n + 1, dtype=np.uint64)
+    sim._add_edges_array(E, np.roll(ids, 1), ids)
+    vh.finish_init_(sim)
+    T = vh.transitions
+    tr, write = {"sum": (T.sum_neighbors(E), A), "foo_edges": (T.neighbor_foo_edges(E, F, -1), F),
+                 "diffuse": (T.diffuse(E, A), A), "move_to": (T.move_to_value(sim, "r", E), [A, E])}[body]
+    with pytest.raises(AssertionError, match="hint combination"):
+        vh.apply_(sim, tr, A, [A, E], write)
+    assert vh.num_agents(sim, A) == n

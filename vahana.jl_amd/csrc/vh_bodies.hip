@@ -24,6 +24,12 @@ template <>
 struct Body<VH_TR_NOOP> {
     __device__ static bool run(const DCtx*, const uint8_t*, uint64_t, Emitter&, uint8_t*) { return true; }
 };
+// neighborids is not defined for :IgnoreFrom types: they keep no sources
+__device__ __forceinline__ bool has_sources(const DCtx* c, const DEdge& E) {
+    if (!VH_HAS(E.hints, VH_HINT_IGNOREFROM)) return true;
+    vh_flag(c, VH_DERR_HINT);
+    return false;
+}
 // create_sum_state_neighbors test/core.jl:71-83
 template <>
 struct Body<VH_TR_SUM_NEIGHBORS> {
@@ -33,10 +39,7 @@ struct Body<VH_TR_SUM_NEIGHBORS> {
         int64_t sum = 0;
         if (d_row(c, et, id, b, e)) {
             const DEdge& E = c->e[et];
-            if (VH_HAS(E.hints, VH_HINT_IGNOREFROM)) {
-                vh_flag(c, VH_DERR_HINT);
-                return true;
-            }
+            if (!has_sources(c, E)) return true;
             const Neighbors nb(c, et);
             constexpr int SUM_N = 8;
             const uint8_t* n[SUM_N];
@@ -117,6 +120,7 @@ struct Body<VH_TR_NEIGHBOR_FOO_EDGES> {
         uint32_t b, e;
         if (d_row(c, et, id, b, e)) {
             const DEdge& E = c->e[et];
+            if (!has_sources(c, E)) return true;
             uint8_t es[8];
             st_i64(es, foo);
             const Sources src(E);
@@ -182,6 +186,7 @@ struct Body<VH_TR_DIFFUSE> {
         uint32_t b, e;
         if (!v && d_row(c, et, id, b, e)) {
             const DEdge& E = c->e[et];
+            if (!has_sources(c, E)) return true;
             for (uint32_t k = b; k < e && !v; k++) {
                 const uint8_t* ns = d_state(c, vh_src_id(E, k));
                 if (!ns) return true;
@@ -206,6 +211,7 @@ struct Body<VH_TR_MOVE_TO> {
             vh_flag(c, VH_DERR_TARGET);
             return true;
         }
+        if (!has_sources(c, c->e[et])) return true;
         const uint8_t* ns = d_state(c, vh_src_id(c->e[et], b));
         if (!ns) return true;
         const int64_t v = ld_i64(ns);
@@ -235,10 +241,7 @@ struct Body<VH_TR_REMOVE_EDGES> {
         uint32_t b, e;
         if (!d_row(c, et, id, b, e) || e - b <= n) return false;
         const DEdge& E = c->e[et];
-        if (VH_HAS(E.hints, VH_HINT_IGNOREFROM)) {
-            vh_flag(c, VH_DERR_HINT);
-            return false;
-        }
+        if (!has_sources(c, E)) return false;
         out = vh_src_id(E, b + n);
         return true;
     }
