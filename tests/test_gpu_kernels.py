@@ -553,3 +553,51 @@ def test_bodies_need_sources(vh, gpu_ready, body):
     with pytest.raises(AssertionError, match="hint combination"):
         vh.apply_(sim, tr, A, [A, E], write)
     assert vh.num_agents(sim, A) == n
+
+
+def test_errors_of_replayed_steps(vh, gpu_ready):
+    """A captured general transition that flags: each replay's error is
+    reported by the next checked apply!, also by one whose own kernels can
+    not flag, and only once."""
+    import torch
+    A, E = vh.struct("A", [("foo", "<i8")]), vh.struct("E")
+    B, F = vh.struct("B", [("opinion", "<f8")]), vh.struct("F", [("w", "<f4")])
+    model = (vh.ModelTypes() | vh.register_agenttype_(A, "Immortal", "Independent") | vh.register_agenttype_(B, "Immortal")
+             | vh.register_edgetype_(E, "Stateless", target=A) | vh.register_edgetype_(F, target=B)
+             | vh.create_model("replay"))
+    sim = vh.create_simulation(model)
+    stream = torch.cuda.Stream()
+    sim._set_streams(stream.cuda_stream)
+    sim._add_agents_array(A, np.zeros(100, dtype=A.dtype))
+    sim._add_agents_array(B, np.full(50, 0.5).view(B.dtype))
+    ids = (np.uint64(1) << np.uint64(56)) | np.arange(1, 101, dtype=np.uint64)
+    sim._add_edges_array(E, np.roll(ids, 1), ids)
+    vh.finish_init_(sim)
+
+    def flag():   # A is not in `read`
+        vh.apply_(sim, vh.transitions.sum_neighbors(E), A, [E], A)
+
+    def checked():
+        vh.apply_(sim, vh.transitions.opinion(F, 0.2, False), B, [B, F], B)
+    vh.enable_asserts(False)
+    try:
+        flag()
+    finally:
+        vh.enable_asserts(True)
+    with pytest.raises(AssertionError):
+        checked()
+    checked()   # (and B's buffers are where they were: the captured step needs the context it has)
+    g = torch.cuda.CUDAGraph()
+    vh.enable_asserts(False)
+    try:
+        with torch.cuda.graph(g, stream=stream, capture_error_mode="thread_local"):
+            flag()
+    finally:
+        vh.enable_asserts(True)
+    for _ in range(3):
+        checked()
+        with torch.cuda.stream(stream):
+            g.replay()
+        with pytest.raises(AssertionError, match="read"):
+            checked()
+    assert vh.num_agents(sim, A) == 100

@@ -150,6 +150,7 @@ struct Sim {
     uint32_t ctx_used = 0;
     DevBuf d_err;                  // uint32 error word
     bool err_written = true;       // a kernel that can set d_err was enqueued since it was last read as 0
+    bool err_captured = false;     // one was captured: its replays are not seen here
     DevBuf d_stats;                // small readback area
     uint64_t* h_stats = nullptr;   // pinned mirror of d_stats
     Scratch scratch;

@@ -1487,15 +1487,17 @@ static void fill_ctx(Sim& s, const vh_apply_desc* d, DCtx& c) {
 
 static int upload_ctx(Sim& s, const DCtx& c) {
     s.err_written = true;   // (the kernels that take a context can flag)
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIPCHECK(hipStreamIsCapturing(s.stream, &cap));
+    const bool capturing = cap != hipStreamCaptureStatusNone;
+    if (capturing) s.err_captured = true;
     if (s.ctx_valid && memcmp(&c, &s.h_ctx, sizeof c) == 0) return VH_OK;
+    // (a captured copy would read the slot as it is at each replay)
+    if (capturing)
+        return set_error(VH_ERR_DEVICE, "a transition that needs its context uploaded can not be captured");
     // through a slot of pinned memory that no copy still reads: a wait only
     // where CTX_SLOTS contexts were sent since the last one
     if (s.ctx_used == CTX_SLOTS) RC(wait_stream(s));
-    // (a captured copy would read the slot as it is at each replay)
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    HIPCHECK(hipStreamIsCapturing(s.stream, &cap));
-    if (cap != hipStreamCaptureStatusNone)
-        return set_error(VH_ERR_DEVICE, "a transition that needs its context uploaded can not be captured");
     DCtx* slot = s.h_ctx_ring + s.ctx_used;
     s.ctx_valid = false;
     *slot = s.h_ctx = c;
@@ -1507,10 +1509,10 @@ static int upload_ctx(Sim& s, const DCtx& c) {
 
 // waits for the stream and reports the device error word; the word is read
 // only when a kernel that can set it ran since it was last read (the SIR,
-// opinion and contact kernels can not)
+// opinion and contact kernels can not), or may have run in a replay
 static int check_errors(Sim& s) {
     uint32_t* const word = (uint32_t*)(s.h_stats + 63);
-    const bool read = s.err_written;
+    const bool read = s.err_written || s.err_captured;
     if (read) RC(copy_words(word, s.d_err.p, 4, s.stream));
     RC(wait_stream(s));
     const uint32_t e = read ? *word : 0u;
