@@ -601,3 +601,35 @@ def test_errors_of_replayed_steps(vh, gpu_ready):
         with pytest.raises(AssertionError, match="read"):
             checked()
     assert vh.num_agents(sim, A) == 100
+
+
+@pytest.mark.parametrize("value", [1, 255])
+@pytest.mark.parametrize("dims,dist", [((40, 9), 2), ((600, 5), 1), ((1100, 6), 5), ((24, 7, 6), 2)],
+                         ids=lambda v: str(v).replace(" ", ""))
+def test_diffuse_rows_filled(vh, ora, gpu_ready, dims, dist, value):
+    """diffuse up to the raster where all cells are active but for holes that
+    only some offsets reach, at which whole waves stop early or do not."""
+    n = int(np.prod(dims))
+    raw = np.full(n, value, dtype=np.uint8)
+    hole = np.random.default_rng(n).integers(0, n)
+    got = []
+    for V in (vh, ora):
+        Cell, Adj = V.struct("Cell", [("active", "?")]), V.struct("Adj")
+        model = (V.ModelTypes() | V.register_agenttype_(Cell, "Immortal")
+                 | V.register_edgetype_(Adj, "Stateless", target=Cell) | V.create_model("filled"))
+        sim = V.create_simulation(model)
+        cells = raw.reshape(dims, order="F").copy()
+        at = np.unravel_index(hole, dims, order="F")
+        box = tuple(slice(max(0, a - dist), a + dist + 1) for a in at)
+        cells[box] = 0   # the hole's cells see active ones at its edge only
+        V.raster.add_raster_(sim, "r", dims, cells.reshape(-1, order="F").view([("active", "?")]), T=Cell)
+        V.raster.connect_raster_neighbors_(sim, "r", Adj(), distance=dist, periodic=False,
+                                           device=None if V is vh else False)
+        V.finish_init_(sim)
+        out = []
+        for _ in range(3):
+            V.apply_(sim, V.transitions.diffuse(Adj, Cell), Cell, [Cell, Adj], Cell)
+            out.append(_states(sim, Cell)[0].copy())
+        got.append(out)
+    for k, (a, b) in enumerate(zip(*got)):
+        assert np.array_equal(a, b), k

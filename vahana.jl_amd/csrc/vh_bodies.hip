@@ -2029,7 +2029,12 @@ __global__ __launch_bounds__(256) void k_diffuse_stencil(StencilSpec sp, const u
 // k_diffuse_stencil 266 us (divisions and byte loads per cell); this with the
 // rows in scalar instructions 24 us, with the rows by lanes but the end groups
 // within the other waves 18 us, apart 16 us, two rows a wave 15 us (four: the
-// same).
+// same). A wave stops before the next ROW_U offsets once all its cells are
+// active, a lane of the end groups before the next offset: diffusion fills the
+// raster, and k_diffuse_stencil, which stops at a cell's first active
+// neighbour, takes 11 us for 10^6 active cells of any stencil. 100^3 cells,
+// 124 offsets, all active: 92 us without the stop, 11 with it; all inactive:
+// 91 and 95 (602 by cells), 3000 x 2000 and Moore 14.6 and 14.7.
 constexpr uint32_t ROW_U = 8;   // offsets at a time
 constexpr uint32_t ROW_R = 2;   // rows of a wave
 struct RowSpec {
@@ -2046,6 +2051,7 @@ __device__ __forceinline__ uint64_t ld8(const uint8_t* p) {
     const u32x3 t = *(const u32x3*)(p - m);
     return (uint64_t)__builtin_amdgcn_alignbyte(t.y, t.x, m) | (uint64_t)__builtin_amdgcn_alignbyte(t.z, t.y, m) << 32;
 }
+constexpr uint64_t ALL_ACTIVE = 0x0101010101010101ull;   // (cells with other nonzero values go on, to the same result)
 __device__ __forceinline__ uint64_t nonzero_bytes(uint64_t v) {   // each to 1
     return ((((v & 0x7F7F7F7F7F7F7F7Full) + 0x7F7F7F7F7F7F7F7Full) | v) >> 7) & 0x0101010101010101ull;
 }
@@ -2093,6 +2099,10 @@ __global__ __launch_bounds__(256) void k_diffuse_rows(RowSpec sp, const uint8_t*
             v[j] = ld8(rs + (uint64_t)rw[j] * (uint32_t)nx + x);
         }
         for (uint32_t k = 0; k < sp.nst; k += ROW_U) {
+            uint64_t on = v[0];
+#pragma unroll
+            for (uint32_t j = 1; j < ROW_R; j++) on &= v[j];
+            if (!__ballot(on != ALL_ACTIVE)) break;
             uint32_t off = sp.off[k];   // lane q: offset k + q, from scalar loads (the launch
 #pragma unroll                          // arguments are slow to reach by vector loads)
             for (uint32_t q = 1; q < ROW_U; q++) off = lane == (int32_t)q ? sp.off[k + q] : off;
@@ -2128,7 +2138,7 @@ __global__ __launch_bounds__(256) void k_diffuse_rows(RowSpec sp, const uint8_t*
     const uint8_t* r0 = rs + (uint64_t)row * (uint32_t)nx;
     const int32_t xc = x + 8 > nx ? nx - 8 : x;   // clamped; the shift drops the cells before x
     uint64_t v = ld8(r0 + xc) >> (8 * (x - xc));
-    for (uint32_t k = 0; k < sp.nst; k++) {
+    for (uint32_t k = 0; k < sp.nst && v != ALL_ACTIVE; k++) {
         int32_t first, dx;
         stencil_row(sp, c, row, sp.off[k], first, dx);
         const uint8_t* r = rs + first;
