@@ -633,3 +633,20 @@ def test_diffuse_rows_filled(vh, ora, gpu_ready, dims, dist, value):
         got.append(out)
     for k, (a, b) in enumerate(zip(*got)):
         assert np.array_equal(a, b), k
+
+
+@pytest.mark.parametrize("C,R,pd,n", [(8, 2, 0.5, 3001), (32, 16, 0.5, 5000), (20, 1, 0.5, 777), (6, 3, 0.9, 1000),
+                                      (33, 2, 0.5, 777), (5, 16, 0.3, 8)])
+def test_contact_many_deaths(vh, ora, gpu_ready, C, R, pd, n):
+    """Most first draws fail: on dying slots (not kept), on dead ones and the
+    slot itself (drawn again, up to the limit)."""
+    M = vh.models
+    g, c = (M.build_contact(V, n, seed=6, n_init=max(1, n // 3)) for V in (vh, ora))
+    for k in range(5):
+        for V, m in ((vh, g), (ora, c)):
+            M.step_contact(V, m, seed=6, beta=0.3, p_death=pd, n_contacts=C, max_redraw=R)
+        (a, da), (b, db) = _states(g.sim, g.T), _states(c.sim, c.T)
+        assert np.array_equal(da, db), k
+        assert np.array_equal(a[~da], b[~db]), k
+        for x, y in zip(g.sim._read_edges(g.E)[:2], c.sim._read_edges(c.E)[:2]):
+            assert np.array_equal(x, y), k

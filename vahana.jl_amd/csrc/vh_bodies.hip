@@ -1569,12 +1569,12 @@ __device__ __forceinline__ uint32_t contact_draw(uint64_t pre, uint32_t n, const
     const uint64_t hh = vh_hash_fin(pre, VH_KEY_PARTNER + (uint64_t)cc * p.max_redraw + r);
     return __umulhi((uint32_t)(hh >> 32), n);
 }
-// contact cc of slot i: draws until a partner that lives in the read state
-// and is not i (at most max_redraw); false when there is none or it dies in
-// this step
+// contact cc of slot i: draws, from draw r on, until a partner that lives in
+// the read state and is not i (at most max_redraw in all); false when there is
+// none or it dies in this step
 __device__ __forceinline__ bool contact_partner(uint64_t pre, uint32_t n, const vh_contact_params& p, uint64_t i,
-                                                uint32_t cc, const ContactBits& B, uint32_t& j) {
-    for (uint32_t r = 0; r < p.max_redraw; r++) {
+                                                uint32_t cc, uint32_t r, const ContactBits& B, uint32_t& j) {
+    for (; r < p.max_redraw; r++) {
         j = contact_draw(pre, n, p, cc, r);
         if (j == i) continue;
         if (!cbit(B.sp, j)) return true;
@@ -1582,26 +1582,14 @@ __device__ __forceinline__ bool contact_partner(uint64_t pre, uint32_t n, const 
     }
     return false;
 }
-// the same for a contact whose first draw is known not to be kept
-__device__ __forceinline__ bool contact_again(uint64_t pre, uint32_t n, const vh_contact_params& p, uint64_t i,
-                                              uint32_t cc, const ContactBits& B, uint32_t& j) {
-    j = contact_draw(pre, n, p, cc, 0);
-    if (j != i && !cbit(B.dead, j)) return false;
-    for (uint32_t r = 1; r < p.max_redraw; r++) {
-        j = contact_draw(pre, n, p, cc, r);
-        if (j == i) continue;
-        if (!cbit(B.sp, j)) return true;
-        if (!cbit(B.dead, j)) return false;
-    }
-    return false;
-}
 // A wave's contacts that draw again (todo: a bit each), 64 at a time, one per
 // lane: every lane calls f(act, lane of the slot, contact). With 2% deaths a
 // slot has 0.8 of them and the worst of 64 slots four: on the slots' own lanes,
 // a wave goes four times through the draws and their lookups for 51 of them
-// (k_contact_edges at 10^7 slots: 238 us so, 220 in pairs; k_contact_main, whose
-// ALU is busy anyway and whose filter leaves no LDS for the lists without larger
-// groups elsewhere, 441 and 460: not there).
+// (k_contact_edges at 10^7 slots: 238 us so, 220 in pairs, 211 with the draws
+// after the first only; k_contact_main, whose ALU is busy anyway and whose
+// filter leaves no LDS for the lists without larger groups elsewhere, 441 and
+// 460: not there).
 template <class F>
 __device__ __forceinline__ void contact_pairs(uint32_t todo, uint16_t* pair, F f) {
     const uint32_t lane = threadIdx.x & 63u;
@@ -1695,14 +1683,18 @@ __device__ __forceinline__ bool contact_health(const uint64_t* __restrict__ rs, 
 // was not its first draw, from which k_contact_edges draws the partners again
 // (8 bytes a slot in place of 4 per contact written and read back). Blocks
 // stay with the filter in LDS and take tiles of BS slots in turn. Four first
-// draws at a time: their hashes, filter bits, and the reads of `sp` that are
-// left are in flight together; what is not accepted there (4% of the draws)
-// is settled after the loop, so that a wave runs the redraws of its lanes
-// together. Bound: instruction issue, 50 vector instructions a draw with seven
-// quarter-rate products among them (0.3 ms for 2 10^8 draws). 10^7 slots, 20
-// contacts, 2% deaths: with infections in the same loop, each draw in the L2
-// and the partners to a log 1055 us, so 440 us (filter groups of 16 slots and
-// two blocks per CU 500; 2, 5, 8 or 10 draws at a time 465, 437, 476, 436).
+// draws at a time: their hashes, filter bits, the reads of `sp` that are left
+// and of `dead` for those that `sp` marks are in flight together. What has to
+// be drawn again (the slot itself, or dead in the read state) is noted and
+// drawn after the loop, a draw of some contact of its own per lane and round:
+// a wave goes round as often as its busiest lane has draws, not as the busiest
+// of each contact. Bound: instruction issue, 50 vector instructions a draw with
+// seven quarter-rate products among them (0.3 ms for 2 10^8 draws). 10^7 slots,
+// 20 contacts, 2% deaths (and, in brackets, 50%): with infections in the same
+// loop, each draw in the L2 and the partners to a log 1055 us (1908); rejected
+// first draws begun anew contact by contact after the loop 441 (2185), so 425
+// (1177). Filter groups of 16 slots and two blocks per CU 500 in place of 441;
+// 2, 5, 8 or 10 draws at a time 465, 437, 476, 436.
 template <int BS, bool FILTER>
 __global__ __launch_bounds__(BS) void k_contact_main(const uint64_t* __restrict__ rs, uint64_t* __restrict__ ws,
                                                      uint8_t* __restrict__ died_now, uint32_t n, uint32_t t,
@@ -1719,7 +1711,7 @@ __global__ __launch_bounds__(BS) void k_contact_main(const uint64_t* __restrict_
         if (i < n && !cbit(B.dead, i)) {
             const uint64_t pre = vh_hash_pre(p.seed, vh_make_id(t, i + 1), step);
             if (contact_health(rs, ws, p, B, i, pre) && p.max_redraw) {
-                uint32_t todo = 0;
+                uint32_t again = 0;   // contacts to draw again: the slot itself, or dead in the read state
                 for (uint32_t c0 = 0; c0 < C; c0 += 4) {
                     uint32_t j[4];
                     bool ask[4];
@@ -1738,20 +1730,36 @@ __global__ __launch_bounds__(BS) void k_contact_main(const uint64_t* __restrict_
                     }
 #pragma unroll
                     for (uint32_t u = 0; u < 4; u++) {
-                        const bool take = j[u] != (uint32_t)i && !((word[u] >> (j[u] & 31u)) & 1u);
-                        km |= take ? 1u << (c0 + u) : 0u;
+                        ask[u] = (word[u] >> (j[u] & 31u)) & 1u;   // dead or dying
+                        word[u] = 0;
+                        if (ask[u]) word[u] = ((const uint32_t*)B.dead)[j[u] >> 5];
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) {
+                        const bool self = j[u] == (uint32_t)i, dead = (word[u] >> (j[u] & 31u)) & 1u;
+                        km |= !self && !ask[u] ? 1u << (c0 + u) : 0u;
+                        again |= self || dead ? 1u << (c0 + u) : 0u;
                     }
                 }
                 const uint32_t all = C == 32 ? 0xFFFFFFFFu : (1u << C) - 1u;   // (the last group may pass C)
                 km &= all;
-                todo = all & ~km;
-                while (todo) {
-                    const uint32_t cc = (uint32_t)__builtin_ctz(todo);
-                    todo &= todo - 1u;
-                    uint32_t jj;
-                    if (contact_partner(pre, n, p, i, cc, B, jj)) {
-                        km |= 1u << cc;
-                        rm |= 1u << cc;
+                again &= p.max_redraw > 1 ? all : 0u;
+                for (uint32_t r = 1; again;) {   // a draw each time round, of whichever contact the lane is at
+                    const uint32_t cc = (uint32_t)__builtin_ctz(again), jj = contact_draw(pre, n, p, cc, r);
+                    bool redo = jj == (uint32_t)i;
+                    if (!redo) {
+                        redo = cbit(B.sp, jj);
+                        if (!redo) {
+                            km |= 1u << cc;
+                            rm |= 1u << cc;
+                        } else {
+                            redo = cbit(B.dead, jj);
+                        }
+                    }
+                    r++;
+                    if (!redo || r == p.max_redraw) {
+                        again &= again - 1u;
+                        r = 1;
                     }
                 }
             }
@@ -1771,7 +1779,8 @@ __global__ __launch_bounds__(BS) void k_contact_main(const uint64_t* __restrict_
 // range of the CSR: the partners are drawn into LDS at their place and
 // written out as one range per block. Dynamic LDS: 256 * n_contacts words.
 // Bound: the 800 MB of a 2 10^8 contact CSR (0.16 ms) and the hashes
-// (0.22 ms); from the log it was 337 us, so 238 us.
+// (0.22 ms); from the log it was 337 us, so 211 us (the contacts drawn again
+// on their slots' lanes 238).
 __global__ __launch_bounds__(256) void k_contact_edges(uint32_t n, uint32_t t, vh_contact_params p, uint64_t step,
                                                        ContactBits B, const uint2* __restrict__ masks,
                                                        const uint32_t* __restrict__ cpos, uint32_t* __restrict__ off,
@@ -1805,7 +1814,7 @@ __global__ __launch_bounds__(256) void k_contact_edges(uint32_t n, uint32_t t, v
         const uint32_t mw = (uint32_t)__shfl((int)m.x, (int)who, 64), rw = (uint32_t)__shfl((int)r0, (int)who, 64);
         uint32_t j = 0;
         if (act) {
-            (void)contact_again(pw, n, p, (i & ~(uint64_t)63) + who, cc, B, j);
+            (void)contact_partner(pw, n, p, (i & ~(uint64_t)63) + who, cc, 1, B, j);   // (kept, and not its first draw)
             lds[rw + (uint32_t)__popc(mw & ((1u << cc) - 1u))] = j + 1u;
         }
     });
@@ -1828,7 +1837,7 @@ __global__ __launch_bounds__(256) void k_contact_main_log(const uint64_t* __rest
             uint32_t* row = log + i * p.n_contacts;
             for (uint32_t cc = 0; cc < p.n_contacts; cc++) {
                 uint32_t j;
-                if (contact_partner(pre, n, p, i, cc, B, j)) row[nk++] = j + 1u;
+                if (contact_partner(pre, n, p, i, cc, 0, B, j)) row[nk++] = j + 1u;
             }
         }
     }
@@ -1848,20 +1857,32 @@ __global__ __launch_bounds__(256) void k_contact_edges_log(uint64_t n, uint32_t 
     for (uint32_t r = 0; r < k; r++) src[o + r] = log[i * C + r];
 }
 
-// Newborns and deaths go by words, one thread each: 2% of the slots die, so
-// a thread per slot spent its time on waves that held one or none (35 and 19
-// us at 10^7 slots, by words 12 and 5 us).
+// Newborns and deaths go by bytes of the bitmaps, a thread each. At 10^7 slots
+// with 2% and with 50% deaths, newborns take 14 and 68 us and deaths 6 and 17;
+// by words, whose 64 slots are a thread's chain of reads and writes, 12 and 147
+// and 5 and 50; by slots, whose waves mostly hold one death or none, 36 and 71
+// and 19 and 34.
+// The slots i0 .. i0 + 7 of this thread that die in this step, and the number
+// of the first of them
+__device__ __forceinline__ uint32_t dying_byte(const ContactBits& B, const uint32_t* __restrict__ dpos, uint64_t& i0,
+                                               uint64_t& g) {
+    const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, w = q >> 3;
+    const uint32_t s = 8u * (uint32_t)(q & 7u);
+    if (w >= B.nwords) return 0u;
+    const uint64_t m = B.sp[w] & ~B.dead[w];
+    i0 = 8 * q;
+    g = dpos[w] + (uint64_t)__popcll(m & ((1ull << s) - 1ull));
+    return (uint32_t)(m >> s) & 0xFFu;
+}
 // Newborns of this step's deaths, in slot order of the dying callers: the top
 // of the reuse stack first, then fresh slots (src/AgentMethods.jl:37-89).
 __global__ void k_contact_births(uint32_t t, vh_contact_params p, uint64_t step, ContactBits B,
                                  const uint32_t* __restrict__ dpos, const uint32_t* __restrict__ reuse,
                                  uint64_t nreuse, uint64_t nextid, uint64_t* __restrict__ ws,
                                  uint8_t* __restrict__ died) {
-    const uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= B.nwords) return;
-    uint64_t g = dpos[w];
-    for (uint64_t m = B.sp[w] & ~B.dead[w]; m; m &= m - 1ull, g++) {   // dying in this step
-        const uint64_t i = w * 64 + (uint32_t)__builtin_ctzll(m);
+    uint64_t g, i0;
+    for (uint32_t m = dying_byte(B, dpos, i0, g); m; m &= m - 1u, g++) {
+        const uint64_t i = i0 + (uint32_t)__builtin_ctz(m);
         const uint64_t slot = g < nreuse ? reuse[nreuse - 1 - g] : nextid + (g - nreuse);
         const float ns = 0.5f + 0.5f * vh_u01f(vh_hash(p.seed, vh_make_id(t, i + 1), step, VH_KEY_BIRTH));
         ws[slot - 1] = (uint64_t)VH_S | ((uint64_t)__float_as_uint(ns) << 32);
@@ -1872,11 +1893,9 @@ __global__ void k_contact_births(uint32_t t, vh_contact_params p, uint64_t step,
 // this step's deaths onto the reuse stack in slot order (src/AgentMethods.jl:314-345)
 __global__ void k_contact_deaths(ContactBits B, const uint32_t* __restrict__ dpos, uint32_t* __restrict__ reuse,
                                  uint64_t base, uint8_t* __restrict__ died) {
-    const uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= B.nwords) return;
-    uint64_t g = dpos[w];
-    for (uint64_t m = B.sp[w] & ~B.dead[w]; m; m &= m - 1ull, g++) {   // dying in this step
-        const uint64_t i = w * 64 + (uint32_t)__builtin_ctzll(m);
+    uint64_t g, i0;
+    for (uint32_t m = dying_byte(B, dpos, i0, g); m; m &= m - 1u, g++) {
+        const uint64_t i = i0 + (uint32_t)__builtin_ctz(m);
         reuse[base + g] = (uint32_t)(i + 1);
         died[i] = 1;
     }
@@ -2846,12 +2865,12 @@ int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t st
             if (A.nextid - 1 + fresh > n)
                 fill_u8(A.died_now.as<uint8_t>() + n, 0, A.nextid - 1 + fresh - n, st);
         }
-        hipLaunchKernelGGL(k_contact_births, dim3(grid_for(nw, 128)), dim3(128), 0, st, (uint32_t)t, p, step, B, dpos,
+        hipLaunchKernelGGL(k_contact_births, dim3(grid_for(8 * nw, 256)), dim3(256), 0, st, (uint32_t)t, p, step, B, dpos,
                            A.reuse.as<uint32_t>(), A.nreuse, A.nextid, (uint64_t*)A.wstate(), A.died.as<uint8_t>());
         A.nreuse -= consumed;
         A.nextid += fresh;
         RC(A.reuse.ensure((A.nreuse + nd) * 4 + 8, st, A.nreuse * 4));
-        hipLaunchKernelGGL(k_contact_deaths, dim3(grid_for(nw, 128)), dim3(128), 0, st, B, dpos,
+        hipLaunchKernelGGL(k_contact_deaths, dim3(grid_for(8 * nw, 256)), dim3(256), 0, st, B, dpos,
                            A.reuse.as<uint32_t>(), A.nreuse, A.died.as<uint8_t>());
         A.nreuse += nd;
         HIPCHECK(hipGetLastError());
