@@ -494,7 +494,7 @@ int vh_ensemble_add_sir(vh_ensemble_t e, const vh_sir_member* m, uint32_t* membe
 int vh_ensemble_remove(vh_ensemble_t e, uint32_t member_id);
 /* the member applies steps up to last_step and then stays (0: no limit) */
 int vh_ensemble_set_horizon(vh_ensemble_t e, uint32_t member_id, uint64_t last_step);
-/* block size (128..1024) and XCD-aware block order of the step launch */
+/* block size (64..1024, a power of two) and XCD-aware block order of the step launch */
 int vh_ensemble_set_config(vh_ensemble_t e, uint32_t block, uint32_t xcd_remap);
 /* advance every member; use_graph: capture the steps into one hipGraph.
  * Asynchronous: returns once the launches are enqueued (the call first waits
@@ -509,6 +509,8 @@ int vh_ensemble_set_streams(vh_ensemble_t e, void* step_stream, void* aux_stream
  * later steps of the others run) */
 int vh_ensemble_read(vh_ensemble_t e, uint32_t member_id, void* states, uint64_t cap, uint64_t* n,
                      uint64_t* step);
+/* bytes: the members' states and in-edges (out-edges of the exposure pass and
+ * scratch not counted) */
 int vh_ensemble_info(vh_ensemble_t e, uint64_t* members, uint64_t* agents, uint64_t* edges,
                      uint64_t* bytes);
 /* agents per thread (1, 2 or 4) of the members of each size class

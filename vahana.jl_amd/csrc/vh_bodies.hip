@@ -632,7 +632,8 @@ __device__ __forceinline__ void opinion_heavy(const uint32_t* __restrict__ off,
         op_accum(x2, w2, xi, eps, num, den);
         op_accum(x3, w3, xi, eps, num, den);
     };
-    vh_lane_edges(off[r], off[r + 1], lane, four, [&](uint32_t k) { op_accum(x[src[k] - 1], w[k], xi, eps, num, den); });
+    vh_lane_edges(off[r], off[r + 1], lane, four,
+                  [&](uint32_t k) { op_accum(x[src[k] - 1], w[k], xi, eps, num, den); });
     num = xor_butterfly(num);
     den = xor_butterfly(den);
     if (lane == 0) xo[i] = den > (T)0 ? num / den : xi;
@@ -1410,8 +1411,8 @@ __global__ void k_win_pack(const uint32_t* __restrict__ keys, const uint32_t* __
                            const uint32_t* __restrict__ kidx, const uint32_t* __restrict__ flag,
                            const uint32_t* __restrict__ ridx, const uint32_t* __restrict__ pinv,
                            const uint32_t* __restrict__ lbase, const uint16_t* __restrict__ sl, uint32_t W,
-                           uint64_t nl, const float* __restrict__ w, uint16_t* __restrict__ tpk, float* __restrict__ twt, uint32_t* __restrict__ prun,
-                           uint16_t* __restrict__ pfirst) {
+                           uint64_t nl, const float* __restrict__ w, uint16_t* __restrict__ tpk,
+                           float* __restrict__ twt, uint32_t* __restrict__ prun, uint16_t* __restrict__ pfirst) {
     const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= nl) return;
     const uint32_t idx = order[e], blk = keys[e] / W, k = kidx[idx];
@@ -2774,10 +2775,10 @@ constexpr uint32_t CONTACT_FILTER = 163840;
 static std::atomic<uint32_t> g_contact_filter{CONTACT_FILTER};   // (less in tests)
 void set_contact_filter(uint32_t bytes) { g_contact_filter = bytes && bytes < CONTACT_FILTER ? bytes : CONTACT_FILTER; }
 
-// One apply! of the contact model: flags, health update with the kept
-// partners logged, one readback (deaths, contacts), newborns and deaths on
-// the reuse stack, then the contact CSR rebuilt in place from the log (its
-// previous entries were last read by k_contact_main). Deaths of this step
+// One apply! of the contact model: flags, infections, health update with the
+// kept partners as masks (or logged), one readback (deaths, contacts), newborns
+// and deaths on the reuse stack, then the contact CSR rebuilt in place (its
+// previous entries were last read by k_contact_infect). Deaths of this step
 // are returned for the edge filtering of other edge types.
 int contact_apply(Sim& s, int t, int et, const vh_contact_params& p, uint64_t step, uint64_t* ndeaths) {
     RC(check_model_layout(s, t, et, 8, 0, "contact"));

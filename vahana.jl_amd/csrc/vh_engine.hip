@@ -617,7 +617,7 @@ __global__ void k_remap_offsets(const uint32_t* __restrict__ off, const uint32_t
 }
 // entries in sorted order (idx null: as they are): sources as ids or numbers
 // (srcw 8 or 4; 0: none), states of `words` W. Random reads of a line per
-// source and state: four entries per thread, all their reads in flight (1.6
+// source and state: four entries per thread, all their reads in flight (3.2
 // 10^6 entries with 8-byte states: 67 us; a gather each, a conversion and
 // copies into the store: 125)
 template <class W>

@@ -367,8 +367,8 @@ __global__ __launch_bounds__(256) void k_ens_expose(const MemberDesc* __restrict
 // agents per thread bstart[b] + 4 t and the three after it, the agents that
 // draw listed (48 members, 7.6 10^6 agents, 200 steps of an epidemic: one agent
 // per thread 52 us a step and 39 us with nothing to draw, blocks' chains of
-// loads; four per thread 32 and 15 us, listed 26 us) (dec null: no exposure; else per-block infected counts of the written state go to
-// blkcnt[(parity ^ 1) * nblocks + b])
+// loads; four per thread 32 and 15 us, listed 26 us). dec null: no exposure;
+// else the counts of the written state go to blkcnt[(parity ^ 1) * nblocks + b]
 __global__ void k_sir_ensemble(const MemberDesc* __restrict__ md, const uint32_t* __restrict__ bmember,
                                const uint32_t* __restrict__ bstart, uint32_t nblocks, uint32_t remap,
                                const uint32_t* __restrict__ dec, uint32_t parity, uint64_t lidx,
@@ -525,7 +525,8 @@ namespace vh {
 // in-degree of target t is Binomial(n - 1, p) by inverse CDF, its sources are
 // distinct uniform draws != t in draw order (vh_graph_gnp is the host twin).
 // gnp_degrees gives off[n + 1] (device) and, after a host synchronisation, the
-// number of edges, gnp_fill the sources (and a copy of off in off_out, unless null); `cdf` and `sc` are working buffers.
+// number of edges, gnp_fill the sources (and a copy of off in off_out, unless
+// null); `cdf` and `sc` are working buffers.
 int gnp_degrees(uint64_t n, double mean_deg, uint64_t seed, uint32_t* off, DevBuf& cdf_buf, Scratch& sc,
                 hipStream_t st, uint64_t* nedges) {
     if (n == 0 || n >= 0xFFFFFFFFull) return set_error(VH_ERR_ARG, "G(n, p): bad n");
@@ -654,7 +655,11 @@ struct vh_ensemble {
     // the members whose epidemics are over (48 members, 7.6 10^6 agents: 47 us
     // a step against 32). Four agents per thread from 10^4 agents (a block of
     // a smaller member would leave the launch with few blocks; 256 threads in
-    // place of 128 or 512: 25.9, 26.5, 28.0 us)
+    // place of 128 or 512: 25.9, 26.5, 28.0 us). us a step of other mixes at
+    // this choice, by XCD, with 512 threads, one and four agents per thread in
+    // every class: 1024 members of 10^3..10^6 agents 896, 974, 967, 1857, 876;
+    // 64 of them 60, 70, 63, 107, 59; 256 of 10^3..10^4 33, 31, 34, 33, 32; 32 of
+    // 10^4..10^5 27, 28, 30, 29, 27
     uint32_t block = 256, remap = 0;
     uint32_t apt[ENS_CLASSES] = {1, 4, 4};   // agents per thread of each size class
     DevBuf d_desc, d_bmember, d_bstart;

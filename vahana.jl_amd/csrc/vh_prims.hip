@@ -362,7 +362,7 @@ static int radix_sort_impl(uint32_t** keys, uint32_t** vals, uint32_t* kalt, uin
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 // Below RADIX_LARGE pairs a pass is launches and latency: digits of 9 or 10
-// bits where they save one (17..20 bits of rows: two passes for three; 1.6 10^6
+// bits where they save one (17..20 bits of rows: two passes for three; 3.2 10^6
 // pairs, 18 bits: 88 us, three passes of 8 bits 122), with tiles of 4096, as
 // their counts per tile are two or four times as many; else tiles of 2048.
 // From there on 8-bit digits and tiles of 8192 (10^7 pairs, 20 bits: scatters
