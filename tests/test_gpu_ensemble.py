@@ -203,3 +203,37 @@ def test_ensemble_add_without_room_for_out_edges(vh, gpu_ready, opts):
             assert np.array_equal(np.ascontiguousarray(E.read(mid)[0]).view(np.uint8), w), after
         E.close()
     assert added > 0
+
+
+def test_ensemble_step_out_of_memory(vh, gpu_ready, opts):
+    """Each device allocation of a first step (block tables, the out-edges'
+    builds, descriptors) fails once: the call is refused, no member has
+    moved, and the same call afterwards gives the solo runs."""
+    opts(sir_expose=1, sir_expose_min=1000)
+    lib = vh._abi.lib()
+    specs = [(3000, 8.0, 0.06, 71, 701), (20000, 12.0, 0.05, 72, 702), (500, 5.0, 0.1, 73, 703)]
+    want = [_solo(vh, n, md, p, s, g, 7, n // 50) for n, md, p, s, g in specs]
+    failed = 0
+    for after in range(60):
+        E = vh.ensemble.Ensemble()
+        ids = [E.add_sir(n, md, p, s, g, recovery=7, n_init=n // 50) for n, md, p, s, g in specs]
+        lib.debug_fail_allocs_after(after, 1)
+        try:
+            E.step(7)
+            done = True
+        except RuntimeError as err:
+            assert f"[{vh._abi.VH_ERR_OOM}]" in str(err), after
+            done = False
+        finally:
+            lib.debug_fail_allocs(0)
+        if not done:
+            failed += 1
+            assert all(E.read(mid)[1] == 1 for mid in ids), after
+            E.step(7)
+        for mid, w in zip(ids, want):
+            assert np.array_equal(np.ascontiguousarray(E.read(mid)[0]).view(np.uint8), w), after
+        E.close()
+        if done:
+            break
+    print(f"[gpu] {failed} allocations failed", flush=True)
+    assert done and failed > 3

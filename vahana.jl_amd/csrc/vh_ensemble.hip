@@ -970,7 +970,11 @@ extern "C" int vh_ensemble_step(vh_ensemble_t e, uint32_t steps, int use_graph) 
     // pass, on the step stream
     const bool expose = expose_runs(e, 0);
     if (expose) {
-        RC(build_members_out(e));
+        const int rc = build_members_out(e);
+        if (rc) {   // (the next call writes the staging that enqueued copies may still read)
+            (void)hipStreamSynchronize(e->stream);
+            return rc;
+        }
         // the bitmaps and counts were not kept while the pass was off: every
         // member's next launch counts, the one after is a full one
         if (!e->expose_last) {
