@@ -419,7 +419,7 @@ def _edge_list(sim, E, state):
 def test_edge_rebuild_out_of_memory(vh, ora, gpu_ready, hints):
     """Each device allocation of a rebuild with more rows and edges fails
     once: the edges are then the old ones, or none where a buffer had grown,
-    and the same call afterwards gives the checker's edges."""
+    and the same call afterwards gives the oracle's edges."""
     n = 300
     fr, to = _ragged_edges(n, 5)
 
